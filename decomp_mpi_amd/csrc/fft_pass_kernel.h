@@ -48,8 +48,9 @@ __device__ __forceinline__ void stage_any(cx<R> *buf, const Pass &P, int s, TW t
 
 // Per-line address data of one side of a tile (in LDS).
 //   uniform:     base[l] = sum over axes other than t of abs[d][g_d]
-//   non-uniform: rbase[l] = owner contribution of those axes, offs[l][k] =
-//                their local offsets (k over the axes other than t)
+//   non-uniform: (base, stride along t) of line l on each of the np rank
+//                positions along t, so a point costs one LDS read and at
+//                most one table read (its position and local offset)
 // Pointers into LDS are typed as such (address space 3) so that reads of
 // the line data are LDS instructions; through a generic pointer they would
 // be flat loads, queued in order with the global data loads.
@@ -60,11 +61,15 @@ using lds_cx = __attribute__((address_space(3))) cx<R>;
 template <typename R, bool CT>
 using lds_tw = __attribute__((address_space(3))) typename tw_local<R, CT>::type;
 
+// Line entries (line, position) a non-uniform side keeps in LDS: 16 KiB.
+constexpr int kLinePositions = 1024;
+
 template <bool UNIFORM>
 struct LineAddr;
 
 template <>
 struct LineAddr<true> {
+  static constexpr int np = 1;
   lds_i64 *base;
   __host__ __device__ static size_t bytes(int T, int) { return (size_t)T * sizeof(i64); }
   __device__ void init(char *mem, int, int) { base = (lds_i64 *)(mem); }
@@ -87,35 +92,49 @@ struct LineAddr<true> {
   }
 };
 
+// Ranks with strides of their own (uneven packed blocks).  Forming every
+// point's address from its owner's strides (two table reads and ndim stride
+// reads a point) made such passes latency-bound: the three passes of a 90 x
+// 126 x 100 complex-double transform on 6 ranks took 43, 43 and 25 us, 129
+// us for the whole call; 86 us with a base and a stride per line and
+// position, dense intermediates and two workgroups per CU.
 template <>
 struct LineAddr<false> {
-  lds_int *rbase;
-  lds_int *offs;
-  int nd;
-  __host__ __device__ static size_t bytes(int T, int ndim) { return (size_t)T * sizeof(int) * (1 + ndim); }
-  __device__ void init(char *mem, int T, int ndim) {
-    rbase = (lds_int *)(mem);
-    offs = rbase + T;
-    nd = ndim;
+  lds_i64 *base;
+  lds_i64 *str;
+  const i64 *tab;  // more positions than LDS is given: the tile's host table
+  int np;
+  __host__ __device__ static size_t bytes(int T, int np) {
+    return np > kLinePositions ? 0 : (size_t)T * np * 2 * sizeof(i64);
   }
-  __device__ void set_line(const FftLaunch &p, const FftSide &s, const int *g, int l) {
-    int r = 0;
-    for (int d = 0; d < p.ndim; d++) {
-      if (d == p.t) continue;
-      r += s.rank[d][g[d]];
-      offs[l * nd + d] = s.off[d][g[d]];
-    }
-    rbase[l] = r;
+  __device__ void init(char *mem, int T, int n) {
+    base = (lds_i64 *)(mem);
+    str = base + T * n;
+    tab = nullptr;
+    np = n;
   }
-  __device__ __forceinline__ i64 at(const FftLaunch &p, const FftSide &s, const i64 *, int l, int x) const {
-    int R = rbase[l] + s.rank[p.t][x];
-    const i64 *m = s.strides + (i64)R * p.ndim;
-    i64 a = (i64)R * s.slot + m[p.t] * s.off[p.t][x];
+  // line l on position q along t (g: the line's coordinates)
+  __device__ void set_line(const FftLaunch &p, const FftSide &s, const int *g, int l, int q) {
+    int R = s.posrank[q];
     for (int d = 0; d < p.ndim; d++)
-      if (d != p.t) a += m[d] * offs[l * nd + d];
-    return a;
+      if (d != p.t) R += s.rank[d][g[d]];
+    const i64 *m = s.strides + (i64)R * p.ndim;
+    i64 a = (i64)R * s.slot;
+    for (int d = 0; d < p.ndim; d++)
+      if (d != p.t) a += m[d] * s.off[d][g[d]];
+    base[l * np + q] = a;
+    str[l * np + q] = m[p.t];
+  }
+  __device__ __forceinline__ i64 at(const FftLaunch &, const FftSide &s, const i64 *, int l, int x) const {
+    if (s.lin) return base[l] + (i64)x * str[l];  // axis t local to every rank, in order
+    const int k = l * np + s.xt[2 * x];
+    if (np > kLinePositions) return tab[2 * k] + (i64)s.xt[2 * x + 1] * tab[2 * k + 1];
+    return base[k] + (i64)s.xt[2 * x + 1] * str[k];
   }
 };
+
+// Address data one line of a side holds (LineAddr::bytes' second argument).
+__host__ __device__ __forceinline__ int side_positions(const FftSide &s) { return s.uniform ? 1 : s.np; }
 
 // Tile t -> (tile along u, batch coordinates); fills the per-line address
 // data of both sides for that tile (threads l < T).
@@ -126,14 +145,41 @@ __device__ __forceinline__ int setup_lines(const FftLaunch &p, long long tile, L
   const int u0 = tu * T;
   const int mk = p.merge_k;
   const int nlines = mk > 1 ? T : (p.u >= 0 ? min(T, p.L[p.u] - u0) : 1);
-  if constexpr (UIN && UOUT) {
-    if (p.line_in_tab != nullptr) {  // precomputed line bases: one load each
+  if (p.line_in_tab != nullptr) {  // precomputed line bases
+    // (both sides' loads go out together: one latency)
+    if constexpr (UIN && UOUT) {
       for (int l = threadIdx.x; l < T; l += NTHR) {
         lin.base[l] = p.line_in_tab[tile * T + l];
         lout.base[l] = p.line_out_tab[tile * T + l];
       }
-      return nlines;
+    } else {
+      const int ni = UIN ? T : T * lin.np, no = UOUT ? T : T * lout.np;
+      const i64 *ti = p.line_in_tab + tile * (UIN ? ni : 2 * ni);
+      const i64 *to = p.line_out_tab + tile * (UOUT ? no : 2 * no);
+      if constexpr (!UIN) lin.tab = ti;
+      if constexpr (!UOUT) lout.tab = to;
+      for (int k = threadIdx.x; k < max(ni, no); k += NTHR) {
+        const int ki = min(k, ni - 1), ko = min(k, no - 1);
+        i64 bi, bo, si = 0, so = 0;
+        if constexpr (UIN) bi = ti[ki];
+        else bi = ti[2 * ki], si = ti[2 * ki + 1];
+        if constexpr (UOUT) bo = to[ko];
+        else bo = to[2 * ko], so = to[2 * ko + 1];
+        if constexpr (UIN) {
+          if (k < ni) lin.base[k] = bi;
+        } else if (k < ni && lin.np <= kLinePositions) {
+          lin.base[k] = bi;
+          lin.str[k] = si;
+        }
+        if constexpr (UOUT) {
+          if (k < no) lout.base[k] = bo;
+        } else if (k < no && lout.np <= kLinePositions) {
+          lout.base[k] = bo;
+          lout.str[k] = so;
+        }
+      }
     }
+    return nlines;
   }
   long long bid = tile / p.tiles_u;
   int gb[DM_MAX_DIMS];
@@ -160,9 +206,11 @@ __device__ __forceinline__ int setup_lines(const FftLaunch &p, long long tile, L
       g[p.u] = (l < nlines) ? (p.ord_u ? p.ord_u[u0 + l] : u0 + l) : 0;
     }
     if constexpr (UIN) lin.set_line(p, p.off_in, g, l);
-    else lin.set_line(p, p.sin, g, l);
+    else
+      for (int q = 0; q < lin.np; q++) lin.set_line(p, p.sin, g, l, q);
     if constexpr (UOUT) lout.set_line(p, p.off_out, g, l);
-    else lout.set_line(p, p.sout, g, l);
+    else
+      for (int q = 0; q < lout.np; q++) lout.set_line(p, p.sout, g, l, q);
   }
   return nlines;
 }
@@ -280,13 +328,16 @@ __device__ __forceinline__ void last_stage_store(const cx<R> *buf, const Pass &P
 // order: a lookup issued after a data load would make the data load's
 // latency part of every later address computation.
 // Complex float at 8 points per thread is held to 64 VGPRs (8 waves per
-// SIMD: two 1024-thread or four 512-thread workgroups per CU).
+// SIMD: two 1024-thread or four 512-thread workgroups per CU).  Complex
+// double is held to 128 (4 waves per SIMD, two 512-thread workgroups per
+// CU): the mixed-radix kernels took 129 and 130 without the bound, one
+// workgroup per CU.
 // CT: compensated twiddle products (complex float only).
 // ANY: the schedule has a prime radix above 13 (direct-sum stages); such
 // schedules get kernels of their own, so that the stage's registers do not
 // weigh on the others.
 template <typename R, bool INV, int CAP, int NTH, bool POW2, bool UIN, bool UOUT, bool CT, bool ANY>
-__global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 1) void fft_pass_kernel(Pass P) {
+__global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 4) void fft_pass_kernel(Pass P) {
   extern __shared__ char smem_raw[];
   cx<R> *buf = reinterpret_cast<cx<R> *>(smem_raw);
   const FftLaunch &p = P.p;
@@ -297,8 +348,9 @@ __global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 1) vo
   char *lmem = smem_raw + (size_t)T * P.ls * sizeof(cx<R>);
   LineAddr<UIN> lin;
   LineAddr<UOUT> lout;
-  lin.init(lmem, T, p.ndim);
-  lout.init(lmem + LineAddr<UIN>::bytes(T, p.ndim), T, p.ndim);
+  const int npi = side_positions(p.sin), npo = side_positions(p.sout);
+  lin.init(lmem, T, npi);
+  lout.init(lmem + LineAddr<UIN>::bytes(T, npi), T, npo);
   // Workgroups are dispatched round-robin over the 8 XCDs.  When a tile's
   // rows are shorter than a 128-byte line, the xcd_pair tiles that share
   // those lines are given to consecutive workgroups of one XCD, so its L2
@@ -314,8 +366,7 @@ __global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 1) vo
   tile += p.tile_base;
   const int nl = setup_lines<UIN, UOUT>(p, tile, lin, lout, T, NTH);
   // twiddle table in LDS after the line data
-  size_t tw_at = (size_t)T * P.ls * sizeof(cx<R>) + LineAddr<UIN>::bytes(T, p.ndim) +
-                 LineAddr<UOUT>::bytes(T, p.ndim);
+  size_t tw_at = (size_t)T * P.ls * sizeof(cx<R>) + LineAddr<UIN>::bytes(T, npi) + LineAddr<UOUT>::bytes(T, npo);
   typedef typename tw_local<R, CT>::type TwL;
   typedef typename tw_global<R>::type TwG;
   TwL *twl = reinterpret_cast<TwL *>(smem_raw + ((tw_at + 15) & ~(size_t)15));

@@ -180,6 +180,18 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   L.u = u;
   L.in_row = in_row ? 1 : 0;
   L.out_row = out_row ? 1 : 0;
+  // rank positions along t of a side whose ranks have strides of their own
+  auto positions = [&](const Side &s) {
+    std::vector<int> v;
+    if (!s.h.uniform) {
+      v = s.h.rank_part[t];
+      std::sort(v.begin(), v.end());
+      v.erase(std::unique(v.begin(), v.end()), v.end());
+    }
+    return v;
+  };
+  const std::vector<int> pos_in = positions(I), pos_out = positions(U);
+  const int np_most = (int)std::max(std::max(pos_in.size(), pos_out.size()), (size_t)1);
   if (u >= 0) {
     // column walk at a line stride of 64 KiB or more: wide rows pay for the
     // lower occupancy of the wide tile -- for lines of 256 points or more
@@ -191,6 +203,9 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     static const bool nowide = getenv("DM_NO_WIDE") != nullptr;
     int tcap = fft_tile_capacity(dbl, !(in_row && out_row), wide && !nowide);
     L.T = std::max(1, std::min(std::min(tcap / L.N, I.h.L[u]), 512));
+    // per-line address data of a non-uniform side: 16 KiB of LDS at most
+    // (a side with more positions than that reads its line table)
+    if (np_most > 1) L.T = std::max(1, std::min(L.T, fft_line_positions() / np_most));
     L.tiles_u = (I.h.L[u] + L.T - 1) / L.T;
   } else {
     L.T = 1;
@@ -223,7 +238,7 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     const int per = std::min(fft_tile_capacity(dbl, 0) / L.N, 512);
     const int lu = I.h.L[u];
     const int v = L.batch_axis[L.nbatch - 1];
-    if (2 * lu <= per) {
+    if (2 * lu <= per && np_most == 1) {
       for (int k = per / lu; k >= 2; k--)
         if (I.h.L[v] % k == 0) {
           L.merge_v = v;
@@ -249,7 +264,7 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     pp->out_off[d] = tb.put(U.abs[d].data(), U.abs[d].size() * sizeof(i64));
   }
   // rank-dependent strides: owner, local offset and per-rank stride tables
-  auto side = [&](const Side &s, FftSide &fs, PendingSide &ps) {
+  auto side = [&](const Side &s, FftSide &fs, PendingSide &ps, const std::vector<int> &pos) {
     fs.uniform = s.h.uniform ? 1 : 0;
     fs.proc_used = s.h.proc_used;
     fs.slot = s.slot;
@@ -285,14 +300,24 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
       }
     }
     if (s.h.uniform) return;
+    std::vector<int> xt(2 * (size_t)L.N);
+    fs.np = (int)pos.size();
+    fs.lin = fs.np == 1;
+    for (int x = 0; x < L.N; x++) {
+      xt[2 * (size_t)x] = (int)(std::lower_bound(pos.begin(), pos.end(), s.h.rank_part[t][x]) - pos.begin());
+      xt[2 * (size_t)x + 1] = s.h.off[t][x];
+      fs.lin = fs.lin && s.h.off[t][x] == x;
+    }
+    ps.xt = tb.put(xt.data(), xt.size() * sizeof(int));
+    ps.posrank = tb.put(pos.data(), pos.size() * sizeof(int));
     for (int d = 0; d < nd; d++) {
       ps.rank[d] = tb.put(s.h.rank_part[d].data(), s.h.L[d] * sizeof(int));
       ps.off[d] = tb.put(s.h.off[d].data(), s.h.L[d] * sizeof(int));
     }
     ps.strides = tb.put(s.h.strides.data(), s.h.strides.size() * sizeof(i64));
   };
-  side(I, L.sin, pp->sin);
-  side(U, L.sout, pp->sout);
+  side(I, L.sin, pp->sin, pos_in);
+  side(U, L.sout, pp->sout, pos_out);
   if (in_row && !is_identity(I.order[t])) pp->ord_in = (long)tb.put(I.order[t].data(), L.N * sizeof(int));
   if (out_row && !is_identity(U.order[t])) pp->ord_out = (long)tb.put(U.order[t].data(), L.N * sizeof(int));
   if (u >= 0) {
@@ -302,40 +327,63 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   }
   // Per-tile line bases for uniform sides: one coalesced load per tile in
   // the kernel instead of a chain of lookups (bounded to 64 MiB of tables).
+  // Non-uniform sides form theirs in the kernel (90 x 126 x 100 on 6 ranks:
+  // 86 us against 81 with tables, but 371 against 566 for a first pass),
+  // unless they have more positions than LDS holds.
   {
-    long long nlines = (long long)L.tiles_u * batch * L.T;
-    if (I.h.uniform && U.h.uniform && L.merge_k == 1 && nlines * 16 <= (64LL << 20)) {
-      std::vector<i64> bi(nlines), bo(nlines);
+    const long long nlines = (long long)L.tiles_u * batch * L.T;
+    const size_t wi = I.h.uniform ? 1 : 2 * pos_in.size(), wo = U.h.uniform ? 1 : 2 * pos_out.size();
+    if (L.merge_k == 1 && ((I.h.uniform && U.h.uniform && nlines * 16 <= (64LL << 20)) || np_most > fft_line_positions())) {
+      std::vector<i64> bi(nlines * wi), bo(nlines * wo);
       const std::vector<int> *ou = nullptr;
       if (pp->ord_u >= 0) ou = &((out_row ? I : U).order[u]);
       std::vector<int> g(nd, 0);
-      for (long long tile = 0; tile < (long long)L.tiles_u * batch; tile++) {
-        int tu = (int)(tile % L.tiles_u);
-        long long bid = tile / L.tiles_u;
-        for (int k = L.nbatch - 1; k >= 0; k--) {
-          int d = L.batch_axis[k];
-          g[d] = (int)(bid % I.h.L[d]);
-          bid /= I.h.L[d];
+      // the line through g: its base, or its base and stride per position
+      auto put = [&](const Side &s, const std::vector<int> &pos, i64 *to) {
+        int R0 = 0;
+        for (int d = 0; d < nd; d++)
+          if (d != t) R0 += s.h.rank_part[d][g[d]];
+        for (size_t q = 0; q < pos.size(); q++) {
+          const int R = R0 + pos[q];
+          const i64 *m = &s.h.strides[(size_t)R * nd];
+          i64 a = (i64)R * s.slot;
+          for (int d = 0; d < nd; d++)
+            if (d != t) a += m[d] * s.h.off[d][g[d]];
+          to[2 * q] = a;
+          to[2 * q + 1] = m[t];
         }
-        i64 base_i = 0, base_o = 0;
-        for (int k = 0; k < L.nbatch; k++) {
-          int d = L.batch_axis[k];
-          base_i += I.abs[d][g[d]];
-          base_o += U.abs[d][g[d]];
-        }
-        for (int l = 0; l < L.T; l++) {
-          i64 ai = base_i, ao = base_o;
-          if (u >= 0) {
-            int cu = tu * L.T + l;
-            if (cu >= I.h.L[u]) cu = 0;
-            else if (ou) cu = (*ou)[cu];
-            ai += I.abs[u][cu];
-            ao += U.abs[u][cu];
+      };
+      // u coordinate of every line of a row of tiles, its offsets in both
+      const int nu = L.tiles_u * L.T;
+      std::vector<int> cu(nu, 0);
+      for (int l = 0; l < nu && u >= 0; l++)
+        if (l < I.h.L[u]) cu[l] = ou ? (*ou)[l] : l;
+      auto fill = [&](const Side &s, const std::vector<int> &pos, size_t w, std::vector<i64> &to) {
+        std::vector<i64> au(nu, 0);
+        for (int l = 0; l < nu && u >= 0; l++) au[l] = s.abs[u][cu[l]];
+        std::fill(g.begin(), g.end(), 0);
+        i64 *at = to.data();
+        for (long long b = 0; b < batch; b++) {
+          if (s.h.uniform) {
+            i64 base = 0;
+            for (int k = 0; k < L.nbatch; k++) base += s.abs[L.batch_axis[k]][g[L.batch_axis[k]]];
+            for (int l = 0; l < nu; l++) at[l] = base + au[l];
+          } else {
+            for (int l = 0; l < nu; l++) {
+              if (u >= 0) g[u] = cu[l];
+              put(s, pos, at + l * w);
+            }
           }
-          bi[tile * L.T + l] = ai;
-          bo[tile * L.T + l] = ao;
+          at += nu * w;
+          for (int k = L.nbatch - 1; k >= 0; k--) {  // the next batch coordinate
+            const int d = L.batch_axis[k];
+            if (++g[d] < I.h.L[d]) break;
+            g[d] = 0;
+          }
         }
-      }
+      };
+      fill(I, pos_in, wi, bi);
+      fill(U, pos_out, wo, bo);
       pp->line_in = (long)tb.put(bi.data(), bi.size() * sizeof(i64));
       pp->line_out = (long)tb.put(bo.data(), bo.size() * sizeof(i64));
     }
@@ -413,6 +461,8 @@ void *finalize_passes(dm_comm_t comm, TableBuilder &tb, std::vector<PendingPass>
         fs.off[d] = (const int *)(b + ps.off[d]);
       }
       fs.strides = (const i64 *)(b + ps.strides);
+      fs.xt = (const int *)(b + ps.xt);
+      fs.posrank = (const int *)(b + ps.posrank);
     };
     side(L.sin, p.sin);
     side(L.sout, p.sout);

@@ -42,7 +42,7 @@ struct TableBuilder {
 struct PendingSide {
   size_t rank[DM_MAX_DIMS];
   size_t off[DM_MAX_DIMS];
-  size_t strides;
+  size_t strides, xt, posrank;
 };
 
 struct PendingPass {

@@ -46,8 +46,9 @@ struct StageInfo {
 // Lines along axis t of an ndim array.  With equal strides on every rank
 // (uniform) point g lives at element offset sum_d abs[d][g_d] from the base
 // pointer; otherwise at R*slot + sum_d strides[R][d]*off[d][g_d] with owner
-// R = sum_d rank[d][g_d].  A tile holds T consecutive lines along axis u
-// (u < 0: one line per tile) and goes through LDS.
+// R = sum_d rank[d][g_d].  The owners along t are np positions: a line has a
+// base and a stride along t on each.  A tile holds T consecutive lines along
+// axis u (u < 0: one line per tile) and goes through LDS.
 struct FftSide {
   int uniform;
   int proc_used;
@@ -55,6 +56,11 @@ struct FftSide {
   i64 aff;                     // uniform side whose offset along t is x * aff (0: see jump)
   i64 jump, rstride;           // aff 0, jump != 0: runs of rmask + 1 points, offset
   int rsh, rmask;              //   (x >> rsh) * jump + (x & rmask) * rstride; else the table
+  // non-uniform sides
+  int np;                      // rank positions along t
+  int lin;                     // one position, local offset x at point x
+  const int *xt;               // point x of t: position, local offset
+  const int *posrank;          // owner contribution of each position
   const int *rank[DM_MAX_DIMS];
   const int *off[DM_MAX_DIMS];
   const i64 *strides;          // [proc_used * ndim]
@@ -81,8 +87,9 @@ struct FftLaunch {
   const int *ord_in;          // row mode: t coordinates in input address order (or null)
   const int *ord_out;         // row mode: t coordinates in output address order (or null)
   const int *ord_u;           // tile line l holds u coordinate ord_u[u0 + l] (or u0 + l)
-  const i64 *line_in_tab;     // uniform sides: base offset of line l of tile b at [b * T + l]
-  const i64 *line_out_tab;    //   (null: computed from the per-axis tables)
+  const i64 *line_in_tab;     // base offset of line l of tile b at [b * T + l]; non-uniform sides:
+  const i64 *line_out_tab;    //   (base, stride along t) of position q at 2 * ((b * T + l) * np + q)
+                              //   (both null: computed from the per-axis tables)
   const void *twiddle;        // stage-ordered roots (N 16-byte entries, twiddle_image): stage with
                               //   Ns earlier points and radix R holds w^(jj*r*N/(Ns*R)) at
                               //   (Ns-1) + (r-1)*Ns + jj
@@ -117,6 +124,8 @@ int launch_fft_pass(const FftLaunch &p, void *stream);
 // column walks at a large line stride ("wide") a double one (16 lines of
 // 512 points, 256-byte rows).
 int fft_tile_capacity(int dbl, int column, int wide = 0);
+// (line, position) entries a non-uniform side of a tile keeps in LDS.
+int fft_line_positions();
 
 // ---- K4: twiddle multiply over every rank's local block -------------------
 // Rank r's block: count positions per axis at its memory strides; the

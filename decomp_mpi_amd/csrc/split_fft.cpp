@@ -208,8 +208,7 @@ struct dm_split_ext {
   Decomp start = nullptr;   // caller's (aliased)
   Decomp out = nullptr;     // B_flipped, or A for single-stage plans (owned by the plan)
   bool use_first = false;   // single stage: output in the A decomposition
-  bool compiled = false;
-  dm_fft_program fwd, bwd;
+  dm_fft_program fwd, bwd;  // each built for its first run
   bool phased = false;      // run in the reference's phase order
   bool fused_ok = true;     // every axis fits one pass (else phased only)
   bool custom_out = false;  // out is the caller's (dm_split_set_output)
@@ -251,53 +250,73 @@ static void twiddle_value(int y, int l, int L, double *re, double *im) {
 }
 
 // A dense intermediate layout: axes in `order` (fastest first), the slowest
-// axis split into q equal blocks, one per rank slot (q the largest divisor
-// of its length not above P).  False when a rank's block would not fit the
-// region of `region` elements per slot.
+// axis in blocks over the rank slots, and the next slowest too where the
+// slowest alone does not spread far enough.  The blocks need not be even:
+// every rank has the same strides, so the layout is uniform all the same.
+// Even blocks of the slowest axis (one per slot, the largest divisor of its
+// length not above P) are taken where they fit.  False when a rank's block
+// would not fit the region of `region` elements per slot.
 static bool dense_layout(const std::vector<int> &L, const std::vector<int> &order, int P, i64 region,
                          dm::HostLayout *out) {
   const int nd = (int)L.size();
-  const int slow = order.back();
-  int q = 1;
-  for (int c = std::min(P, L[slow]); c >= 1; c--)
-    if (L[slow] % c == 0) {
-      q = c;
-      break;
-    }
+  const int slow = order[nd - 1], second = nd > 1 ? order[nd - 2] : slow;
   i64 total = 1;
   for (int l : L) total *= l;
-  const i64 per = total / q;
+  // blocks of the slowest (blk) and the next slowest axis (blk2)
+  int blk = L[slow], blk2 = L[second];
+  for (int c = std::min(P, L[slow]); c >= 1; c--)
+    if (L[slow] % c == 0) {
+      blk = L[slow] / c;
+      break;
+    }
+  auto per_of = [&](int b, int b2) {
+    return nd > 1 ? total / L[slow] / L[second] * b * b2 : (i64)b;
+  };
+  if (per_of(blk, blk2) > region) {
+    blk = (L[slow] + P - 1) / P;
+    if (nd > 1 && per_of(blk, blk2) > region) {
+      // blocks of both axes: the smallest block of any rank grid
+      i64 best = per_of(blk, blk2);
+      const int full = L[second];
+      for (int q = 1; q <= std::min(P, L[slow]); q++) {
+        const int b = (L[slow] + q - 1) / q, b2 = (full + P / q - 1) / (P / q);
+        if (per_of(b, b2) < best) {
+          best = per_of(b, b2);
+          blk = b;
+          blk2 = b2;
+        }
+      }
+    }
+  }
+  const i64 per = per_of(blk, blk2);
   if (per > region) return false;
+  const int q1 = (L[slow] + blk - 1) / blk, q2 = nd > 1 ? (L[second] + blk2 - 1) / blk2 : 1;
   dm::HostLayout h;
   h.ndim = nd;
   h.L = L;
-  h.proc_used = q;
+  h.proc_used = q1 * q2;
   h.rank_part.assign(nd, std::vector<int>());
   h.off.assign(nd, std::vector<int>());
   h.m.assign(nd, 0);
-  const int blk = L[slow] / q;
   i64 stride = 1;
   for (int k = 0; k < nd; k++) {
     int d = order[k];
     h.m[d] = stride;
-    stride *= (d == slow) ? blk : L[d];
+    stride *= d == slow ? blk : (d == second ? blk2 : L[d]);
   }
   for (int d = 0; d < nd; d++) {
     h.rank_part[d].assign(L[d], 0);
     h.off[d].resize(L[d]);
+    const int b = d == slow ? blk : (d == second ? blk2 : L[d]);
     for (int g = 0; g < L[d]; g++) {
-      if (d == slow) {
-        h.rank_part[d][g] = g / blk;
-        h.off[d][g] = g % blk;
-      } else {
-        h.off[d][g] = g;
-      }
+      h.rank_part[d][g] = g / b * (d == slow ? q2 : 1);
+      h.off[d][g] = g % b;
     }
   }
   h.strides.clear();
-  for (int r = 0; r < q; r++) h.strides.insert(h.strides.end(), h.m.begin(), h.m.end());
+  for (int r = 0; r < h.proc_used; r++) h.strides.insert(h.strides.end(), h.m.begin(), h.m.end());
   h.uniform = true;
-  h.slot_extent.assign(q, per);
+  h.slot_extent.assign(h.proc_used, per);
   h.fastest = order[0];
   h.offsets_ok = true;
   *out = h;
@@ -314,8 +333,9 @@ static bool dense_layout(const std::vector<int> &L, const std::vector<int> &orde
 // pattern.  Without them, the intermediates stay in the output layout and
 // run in place (every tile reads all of its points before writing them,
 // tiles are disjoint, and such a pass reads and writes one layout).
+// slots: rank slots of the workspace buffer.
 static bool compile_direction(SplitPlan plan, bool inverse, const dm::Side &S, const dm::Side &O, void *dat,
-                              void *w0, void *w1, dm_fft_program *prog) {
+                              void *w0, void *w1, int slots, dm_fft_program *prog) {
   dm_split_ext *x = plan->ext;
   int nd = x->ndim;
   std::vector<int> axes;
@@ -366,7 +386,7 @@ static bool compile_direction(SplitPlan plan, bool inverse, const dm::Side &S, c
       std::sort(others.begin(), others.end(), [&](int a, int b) { return last.h.m[a] < last.h.m[b]; });
       ord.insert(ord.end(), others.begin(), others.end());
       dm::HostLayout h;
-      if (!dense_layout(x->L, ord, plan->comm->world->nranks, region, &h)) dense = false;
+      if (!dense_layout(x->L, ord, std::min(slots, plan->comm->world->nranks), region, &h)) dense = false;
       else mids.push_back(dm::make_side(h, O.slot));
     }
     if (!dense) {  // a block did not fit: the in-place scheme
@@ -449,14 +469,15 @@ static bool bind_buffers(SplitPlan plan, dm::Buffer *bd, size_t *od, dm::Buffer 
   return true;
 }
 
-static bool compile_plan(SplitPlan plan) {
+// Build the fused program of one direction, if it is not there yet.
+static bool compile_plan(SplitPlan plan, bool inverse) {
   dm_split_ext *x = plan->ext;
-  if (x->compiled) return true;
+  dm_fft_program &prog = inverse ? x->bwd : x->fwd;
+  if (prog.mem != nullptr) return true;
   if (!x->fused_ok) {
     raise_error(plan->comm, "split FFT: an axis is longer than one pass tile; this plan runs in phase order only");
     return false;
   }
-  dm_comm_t comm = plan->comm;
   size_t es = x->dbl ? 16 : 8;
   dm::Buffer bd, bw;
   size_t od, ow;
@@ -469,11 +490,9 @@ static bool compile_plan(SplitPlan plan) {
   char *dat = bd.base + od;
   char *w0 = bw.base + ow;
   char *w1 = w0 + ext * es;
-  if (!compile_direction(plan, false, S, O, dat, w0, w1, &x->fwd)) return false;
-  if (!compile_direction(plan, true, S, O, dat, w0, w1, &x->bwd)) return false;
+  if (!compile_direction(plan, inverse, S, O, dat, w0, w1, bw.nranks, &prog)) return false;
   plan->plan_a = &x->fwd;
   plan->plan_b_back = &x->bwd;
-  x->compiled = true;
   return true;
 }
 
@@ -977,7 +996,7 @@ static double model_cost(SplitPlan p) {
 // Milliseconds of a forward + backward step of plan p (the backward
 // overwrites dat: the caller saves it).
 static double time_plan(SplitPlan p, int reps) {
-  if (p->ext->phased ? !compile_phased(p) : !compile_plan(p)) return 1e30;
+  if (p->ext->phased ? !compile_phased(p) : !(compile_plan(p, false) && compile_plan(p, true))) return 1e30;
   void *s = dm::world_stream(p->comm->world);
   hipEvent_t e0, e1;
   (void)hipEventCreate(&e0);
@@ -1193,7 +1212,7 @@ static void run_split(SplitPlan plan, int direction) {
     if (compile_phased(plan)) run_phased(plan, direction);
     return;
   }
-  if (!compile_plan(plan)) return;
+  if (!compile_plan(plan, direction == FFTW_BACKWARD)) return;
   if (direction == FFTW_FORWARD) run_program(plan, plan->ext->fwd, FFT_1, FFT_2);
   else run_program(plan, plan->ext->bwd, FFT_2, FFT_1);
 }
@@ -1216,7 +1235,6 @@ extern "C" int dm_split_set_output(SplitPlan plan, Decomp out) {
   }
   program_release(x->fwd);
   program_release(x->bwd);
-  x->compiled = false;
   x->out = out;
   x->custom_out = true;
   x->phased = false;
@@ -1251,7 +1269,6 @@ extern "C" int dm_split_set_twiddles(SplitPlan plan, int mode) {
     x->ctw = ctw;
     program_release(x->fwd);
     program_release(x->bwd);
-    x->compiled = false;
     phased_release(x->ph);
   }
   return DM_SUCCESS;
