@@ -152,6 +152,9 @@ struct DevLayout {
   const int *off[DM_MAX_DIMS];
   const i64 *addr[DM_MAX_DIMS];   // uniform: m_d * off_d(g)
   const i64 *strides;             // [proc_used * ndim]
+  const int *pos[DM_MAX_DIMS];    // coordinate -> rank position (index into posrank)
+  const int *posrank[DM_MAX_DIMS];  // distinct owner contributions, ascending
+  const unsigned *part[DM_MAX_DIMS];  // uniform: (rank, addr) pairs, 32 bits each
 };
 
 // Device copy of a HostLayout's tables.
@@ -159,6 +162,7 @@ struct DeviceLayout {
   DevLayout dev{};
   void *mem = nullptr;
   size_t bytes = 0;
+  int np[DM_MAX_DIMS] = {0};      // rank positions per axis
   void upload(const HostLayout &h);
   void release();
 };

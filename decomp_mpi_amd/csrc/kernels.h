@@ -14,8 +14,19 @@ namespace dm {
 // Coordinates are walked as 2D tiles over (a, b) = (dst fastest axis, src
 // fastest axis) so that reads and writes are both coalesced; the remaining
 // axes are batch.  a == b walks 1D runs along that axis.
+// owned: every coordinate has an owner on both sides and the tile axes have
+// few rank positions (kReshapePairs pairs a side).
+struct ReshapeSide {             // index 0: axis a, 1: axis b
+  const int *pos[2];           // coordinate -> rank position along the axis
+  const int *posrank[2];       // owner contribution of each position
+  const unsigned *part[2];     // uniform: coordinate -> (owner contribution, element offset)
+  int np[2];
+};
 struct ReshapeLaunch {
   DevLayout src, dst;
+  ReshapeSide ss, sd;
+  int owned;
+  int same_order;              // owned, both sides fastest along a: b is a row axis
   int ndim;
   int L[DM_MAX_DIMS];
   int a, b;
@@ -28,9 +39,13 @@ struct ReshapeLaunch {
   char *dst_base;
   i64 src_slot;           // elements per rank slot
   i64 dst_slot;
+  i64 src_bytes;          // bytes per rank slot
+  i64 dst_bytes;
   int elem_bytes;
-  int nontemporal;            // 1: non-temporal hint on the element accesses
+  int below_4g;           // owned: both buffers below 4 GiB
+  int nontemporal;        // owned: non-temporal hint on the element accesses
 };
+constexpr int kReshapePairs = 512;  // (a position, b position) pairs of a side in LDS, at most
 // Launchers return 0 or the HIP error code of the launch (hipError_t).
 int launch_reshape(const ReshapeLaunch &p, void *stream);
 

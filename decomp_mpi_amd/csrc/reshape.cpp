@@ -22,7 +22,10 @@ struct dm_reshape_program {
   dm::DeviceLayout dsrc, ddst;
   bool uploaded = false;
   int word = 1;               // bytes per moved unit
+  int align = 1;              // alignment it needs
   int words = 1;              // units per element
+  bool owned = false;         // the kernels without ownership checks
+  bool rows = false;          // owned, both sides fastest along a: b is a row axis
   int elem = 1;               // element extent in bytes
   int a = 0, b = 0;
   std::vector<int> batch;
@@ -281,6 +284,80 @@ static void relabel_axis(dm_reshape_program *pg, int d, const dm::HostLayout &ke
   }
 }
 
+// Every coordinate has an owner.
+static bool all_owned(const dm::HostLayout &h) {
+  for (int d = 0; d < h.ndim; d++)
+    for (int r : h.rank_part[d])
+      if (r >= (1 << 27)) return false;
+  return true;
+}
+
+// Distinct owner contributions along axis d, ascending.
+static std::vector<int> rank_positions(const dm::HostLayout &h, int d) {
+  std::vector<int> v = h.rank_part[d];
+  std::sort(v.begin(), v.end());
+  v.erase(std::unique(v.begin(), v.end()), v.end());
+  return v;
+}
+
+// Pairs of rank positions along a and b that the kernel tabulates: only
+// sides whose ranks have strides of their own need them.
+static size_t pairs(const dm::HostLayout &h, int a, int b) {
+  return h.uniform ? 0 : rank_positions(h, a).size() * rank_positions(h, b).size();
+}
+
+// Tile axes, batch axes and kernel of a program whose layouts are per
+// element and whose unit (word) is chosen.
+static void plan_walk(dm_reshape_program *pg) {
+  pg->words = pg->elem / pg->word;
+  const bool split = getenv("DM_NO_SPLIT") == nullptr && split_shared_axis(pg);
+  const int nd_el = pg->src.ndim;  // element axes (a split adds one)
+  extend_by_words(pg->src, pg->words);
+  extend_by_words(pg->dst, pg->words);
+  pg->a = pg->dst.fastest;
+  pg->b = pg->src.fastest;
+  // (a split keeps its two halves as the tile axes, also over words)
+  if (!split && pg->words > 1) {  // tile over the element axes, not the word axis
+    auto pick = [&](const dm::HostLayout &h) {
+      int best = 0;
+      i64 bs = -1;
+      for (int d = nd_el - 1; d >= 0; d--)
+        if (h.L[d] > 1 && (bs < 0 || h.m[d] < bs)) bs = h.m[d], best = d;
+      return best;
+    };
+    pg->a = pick(pg->dst);
+    pg->b = pick(pg->src);
+  }
+  // writes run along a, reads along b
+  if (getenv("DM_NO_RELABEL") == nullptr) {
+    relabel_axis(pg, pg->a, pg->dst);
+    if (pg->b != pg->a) relabel_axis(pg, pg->b, pg->src);
+  }
+  std::vector<int> rest;
+  for (int d = 0; d < pg->dst.ndim; d++)
+    if (d != pg->a && d != pg->b) rest.push_back(d);
+  // slowest destination axes first so consecutive blocks stay close in memory
+  std::stable_sort(rest.begin(), rest.end(),
+                   [&](int x, int y) { return pg->dst.m[x] > pg->dst.m[y]; });
+  pg->rows = false;
+  pg->owned = all_owned(pg->src) && all_owned(pg->dst);
+  // both sides fastest along one axis: rows of it, several of the next axis
+  // per workgroup (long rows with few neighbours keep the 1D walk)
+  if (pg->owned && pg->a == pg->b) {
+    const bool rows = !rest.empty() && (pg->dst.L[pg->a] < 1024 || pg->dst.L[rest.back()] >= 8);
+    if (rows) {
+      pg->b = rest.back();
+      rest.pop_back();
+      pg->rows = true;
+    } else {
+      pg->owned = false;
+    }
+  }
+  if (pg->owned && (pairs(pg->src, pg->a, pg->b) > dm::kReshapePairs || pairs(pg->dst, pg->a, pg->b) > dm::kReshapePairs))
+    pg->owned = false;
+  pg->batch = rest;
+}
+
 extern "C" ReshapePlan makeReshapePlan(MPI_Comm comm, MPI_Datatype base, Decomp src, Decomp dest) {
   if (src == nullptr || dest == nullptr || base == nullptr) {
     dm::fail(comm, "makeReshapePlan: NULL argument");
@@ -338,8 +415,6 @@ extern "C" ReshapePlan makeReshapePlan(MPI_Comm comm, MPI_Datatype base, Decomp 
   pg->elem = (int)ext;
   int w = 16;
   while (ext % w != 0) w >>= 1;
-  pg->word = w;
-  pg->words = (int)(ext / w);
   pg->src = dm::layout_from_decomp(src);
   pg->dst = dm::layout_from_decomp(dest);
   if (!pg->src.offsets_ok || !pg->dst.offsets_ok) {
@@ -348,36 +423,17 @@ extern "C" ReshapePlan makeReshapePlan(MPI_Comm comm, MPI_Datatype base, Decomp 
     freeReshapePlan(plan);
     return nullptr;
   }
-  const bool split = getenv("DM_NO_SPLIT") == nullptr && split_shared_axis(pg);
-  const int nd_el = pg->src.ndim;  // element axes (a split adds one)
-  extend_by_words(pg->src, pg->words);
-  extend_by_words(pg->dst, pg->words);
-  pg->a = pg->dst.fastest;
-  pg->b = pg->src.fastest;
-  // (a split keeps its two halves as the tile axes, also over words)
-  if (!split && pg->words > 1) {  // tile over the element axes, not the word axis
-    auto pick = [&](const dm::HostLayout &h) {
-      int best = 0;
-      i64 bs = -1;
-      for (int d = nd_el - 1; d >= 0; d--)
-        if (h.L[d] > 1 && (bs < 0 || h.m[d] < bs)) bs = h.m[d], best = d;
-      return best;
-    };
-    pg->a = pick(pg->dst);
-    pg->b = pick(pg->src);
+  // 12- and 24-byte elements move whole where the owned kernels run, as
+  // words of the alignment they have otherwise
+  pg->align = w;
+  pg->word = ext == 3 * w && (w == 4 || w == 8) ? (int)ext : w;
+  plan_walk(pg);
+  if (!pg->owned && pg->word != w) {
+    pg->src = dm::layout_from_decomp(src);
+    pg->dst = dm::layout_from_decomp(dest);
+    pg->word = w;
+    plan_walk(pg);
   }
-  // writes run along a, reads along b
-  if (getenv("DM_NO_RELABEL") == nullptr) {
-    relabel_axis(pg, pg->a, pg->dst);
-    if (pg->b != pg->a) relabel_axis(pg, pg->b, pg->src);
-  }
-  std::vector<int> rest;
-  for (int d = 0; d < pg->dst.ndim; d++)
-    if (d != pg->a && d != pg->b) rest.push_back(d);
-  // slowest destination axes first so consecutive blocks stay close in memory
-  std::stable_sort(rest.begin(), rest.end(),
-                   [&](int x, int y) { return pg->dst.m[x] > pg->dst.m[y]; });
-  pg->batch = rest;
   plan->prog = pg;
   return plan;
 }
@@ -403,7 +459,7 @@ struct Span {
 }  // namespace
 
 // Check one side of a reshape against the buffer it runs on.
-static bool fits(dm_comm_t comm, const char *what, const void *p, const dm::HostLayout &h, int word,
+static bool fits(dm_comm_t comm, const char *what, const void *p, const dm::HostLayout &h, int word, int align,
                  Span *sp) {
   if (!dm::resolve(p, &sp->buf, &sp->off)) {
     raise_error(comm, "runReshapePlan: %s pointer is not inside a distributed buffer (dm_malloc/dm_register)",
@@ -415,8 +471,8 @@ static bool fits(dm_comm_t comm, const char *what, const void *p, const dm::Host
                 sp->buf.nranks, h.proc_used);
     return false;
   }
-  if (sp->off % word != 0 || sp->buf.slot % word != 0) {
-    raise_error(comm, "runReshapePlan: %s pointer or slot not aligned to %d bytes", what, word);
+  if (sp->off % align != 0 || sp->buf.slot % align != 0) {
+    raise_error(comm, "runReshapePlan: %s pointer or slot not aligned to %d bytes", what, align);
     return false;
   }
   for (int r = 0; r < h.proc_used; r++) {
@@ -434,8 +490,8 @@ namespace dm {
 bool enqueue_reshape(dm_comm_t comm, ReshapePlan plan, const void *src, void *dst, void *stream) {
   dm_reshape_program *pg = plan->prog;
   Span s, d;
-  if (!fits(comm, "source", src, pg->src, pg->word, &s)) return false;
-  if (!fits(comm, "destination", dst, pg->dst, pg->word, &d)) return false;
+  if (!fits(comm, "source", src, pg->src, pg->word, pg->align, &s)) return false;
+  if (!fits(comm, "destination", dst, pg->dst, pg->word, pg->align, &d)) return false;
   if (s.buf.base == d.buf.base) {
     size_t se = 0, de = 0;
     for (auto e : pg->src.slot_extent) se = std::max(se, (size_t)e * pg->word);
@@ -470,11 +526,30 @@ bool enqueue_reshape(dm_comm_t comm, ReshapePlan plan, const void *src, void *ds
   L.dst_base = d.buf.base + d.off;
   L.src_slot = (i64)(s.buf.slot / pg->word);
   L.dst_slot = (i64)(d.buf.slot / pg->word);
+  L.src_bytes = (i64)s.buf.slot;
+  L.dst_bytes = (i64)d.buf.slot;
+  L.owned = pg->owned ? 1 : 0;
+  L.same_order = pg->rows ? 1 : 0;
+  auto side = [&](const dm::DeviceLayout &dl, ReshapeSide &to) {
+    const int ax[2] = {pg->a, pg->b};
+    for (int i = 0; i < 2; i++) {
+      to.pos[i] = dl.dev.pos[ax[i]];
+      to.posrank[i] = dl.dev.posrank[ax[i]];
+      to.part[i] = dl.dev.part[ax[i]];
+      to.np[i] = dl.np[ax[i]];
+    }
+  };
+  side(pg->dsrc, L.ss);
+  side(pg->ddst, L.sd);
   L.elem_bytes = pg->word;
-  // non-temporal hint: 11-20% off the 512^3 int64 hops (each element is
-  // read once and written once)
+  L.below_4g = s.buf.slot * (size_t)s.buf.nranks < ((size_t)1 << 32) && d.buf.slot * (size_t)d.buf.nranks < ((size_t)1 << 32);
+  // Data that the memory-side cache holds (256 MB, both sides) is left
+  // there: 28 MB in and out 27 us a pass without the hint, 32 with it;
+  // the 512^3 int64 chain (1 GiB in and out a hop) 897 us without, 860 with.
+  size_t moved = 0;
+  for (auto e : pg->src.slot_extent) moved += (size_t)e * pg->word;
   static const bool nont = getenv("DM_NO_NONTEMPORAL") != nullptr;
-  L.nontemporal = nont ? 0 : 1;
+  L.nontemporal = nont || 2 * moved <= ((size_t)128 << 20) ? 0 : 1;
   return launch_ok(comm, launch_reshape(L, stream), "reshape kernel launch");
 }
 }  // namespace dm
@@ -566,8 +641,14 @@ void DeviceLayout::upload(const HostLayout &h) {
     bytes += (n + 255) & ~(size_t)255;
     return at;
   };
-  std::vector<size_t> at_rank(h.ndim), at_off(h.ndim), at_addr(h.ndim);
+  std::vector<size_t> at_rank(h.ndim), at_off(h.ndim), at_addr(h.ndim), at_pos(h.ndim), at_pr(h.ndim), at_part(h.ndim);
+  std::vector<std::vector<int>> pr(h.ndim);
   for (int d = 0; d < h.ndim; d++) {
+    pr[d] = rank_positions(h, d);
+    np[d] = (int)pr[d].size();
+    at_pos[d] = take(h.L[d] * sizeof(int));
+    at_pr[d] = take(pr[d].size() * sizeof(int));
+    at_part[d] = take(2 * h.L[d] * sizeof(unsigned));
     at_rank[d] = take(h.L[d] * sizeof(int));
     at_off[d] = take(h.L[d] * sizeof(int));
     at_addr[d] = take(h.L[d] * sizeof(i64));
@@ -577,8 +658,17 @@ void DeviceLayout::upload(const HostLayout &h) {
   for (int d = 0; d < h.ndim; d++) {
     memcpy(&host[at_rank[d]], h.rank_part[d].data(), h.L[d] * sizeof(int));
     memcpy(&host[at_off[d]], h.off[d].data(), h.L[d] * sizeof(int));
+    int *po = (int *)&host[at_pos[d]];
+    for (int g = 0; g < h.L[d]; g++)
+      po[g] = (int)(std::lower_bound(pr[d].begin(), pr[d].end(), h.rank_part[d][g]) - pr[d].begin());
+    memcpy(&host[at_pr[d]], pr[d].data(), pr[d].size() * sizeof(int));
     i64 *ad = (i64 *)&host[at_addr[d]];
-    for (int g = 0; g < h.L[d]; g++) ad[g] = h.m[d] * h.off[d][g];
+    unsigned *pt = (unsigned *)&host[at_part[d]];
+    for (int g = 0; g < h.L[d]; g++) {
+      ad[g] = h.m[d] * h.off[d][g];
+      pt[2 * g] = (unsigned)h.rank_part[d][g];
+      pt[2 * g + 1] = (unsigned)ad[g];
+    }
   }
   memcpy(&host[at_str], h.strides.data(), h.strides.size() * sizeof(i64));
   mem = device_alloc(bytes);
@@ -596,6 +686,9 @@ void DeviceLayout::upload(const HostLayout &h) {
     dev.rank[d] = (const int *)(b + at_rank[d]);
     dev.off[d] = (const int *)(b + at_off[d]);
     dev.addr[d] = (const i64 *)(b + at_addr[d]);
+    dev.pos[d] = (const int *)(b + at_pos[d]);
+    dev.posrank[d] = (const int *)(b + at_pr[d]);
+    dev.part[d] = (const unsigned *)(b + at_part[d]);
   }
   dev.strides = (const i64 *)(b + at_str);
 }
