@@ -438,8 +438,230 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   return true;
 }
 
+// Radices of a block pass stage by stage: powers of two in 16s, 8s and 4s
+// (a 16-point axis is one butterfly of a thread's 16 points).
+static bool block_radices(int n, std::vector<int> *out) {
+  out->clear();
+  for (int p : {7, 5, 3})
+    while (n % p == 0) {
+      out->push_back(p);
+      n /= p;
+    }
+  int k = 0;
+  while (n % 2 == 0) {
+    n /= 2;
+    k++;
+  }
+  if (n != 1) return false;
+  // 2^k with as few stages as 16 allows, even ones: 2^5 = 8 4, 2^6 = 8 8
+  const int stages = (k + 3) / 4;
+  for (int i = 0; i < stages; i++) {
+    const int b = (k + (stages - i) - 1) / (stages - i);
+    out->push_back(1 << b);
+    k -= b;
+  }
+  return true;
+}
+
+// Fastest axis of a layout outside `axes` (smallest stride among the axes
+// longer than one), or -1.
+static int fastest_outside(const Side &s, const std::vector<int> &axes) {
+  int best = -1;
+  for (int d = 0; d < s.h.ndim; d++) {
+    if (s.h.L[d] <= 1 || std::find(axes.begin(), axes.end(), d) != axes.end()) continue;
+    if (best < 0 || s.h.m[d] < s.h.m[best]) best = d;
+  }
+  return best;
+}
+
+// The line axis of a block pass (the fastest axis outside its axes) and
+// lines per tile: as many as fit, but where the contiguous axis is among the
+// transformed ones (whole rows anyway) no more than leave a tile for each of
+// the 256 CUs (75 x 45 x 45 complex floats: 19 full tiles 84 us a step, 75
+// of one plane 67).
+static int block_lines(const Side &I, const std::vector<int> &axes, int dbl, int *T) {
+  long long points = 1, total = 1;
+  for (int d : axes) points *= I.h.L[d];
+  for (int l : I.h.L) total *= l;
+  const int u = fastest_outside(I, axes);
+  *T = 1;
+  if (u < 0) return u;
+  const int lu = I.h.L[u];
+  int t = (int)std::max(1LL, std::min<long long>(fft_block_capacity(dbl) / points, lu));
+  if (std::find(axes.begin(), axes.end(), I.h.fastest) != axes.end()) {
+    const long long batch = total / points / lu;
+    while (t > 1 && batch * ((lu + t - 1) / t) < 256) t = (t + 1) / 2;
+  }
+  *T = t;
+  return u;
+}
+
+bool block_fits(const Side &I, const Side &U, const std::vector<int> &axes, int dbl) {
+  if (!I.h.uniform || !U.h.uniform || axes.size() < 2 || axes.size() > DM_BLOCK_DIMS - 1) return false;
+  long long points = 1, total = 1;
+  size_t stages = 0;
+  std::vector<int> rad;
+  for (int d : axes) {
+    points *= I.h.L[d];
+    if (points > fft_block_capacity(dbl) || !block_radices(I.h.L[d], &rad)) return false;
+    stages += rad.size();
+  }
+  for (int l : I.h.L) total *= l;
+  if (stages > 24) return false;
+  int T;
+  const int u = block_lines(I, axes, dbl, &T);
+  // both sides in runs of 128 bytes along the same axis, or the whole array
+  // in a tile
+  const int es = dbl ? 16 : 8;
+  if (U.h.fastest != I.h.fastest && points * T < total) return false;
+  for (const Side *s : {&I, &U}) {
+    const int f = s->h.fastest;
+    const int run = std::find(axes.begin(), axes.end(), f) != axes.end() ? I.h.L[f] : (f == u ? T : 1);
+    if (run * es < 128 && points * T < total) return false;
+  }
+  return total / points * 16 <= (64LL << 20);  // the line bases
+}
+
+bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int dbl, bool inverse, const void *in,
+                void *out, TableBuilder &tb, PendingBlock *pb, int ctw) {
+  FftBlock &B = pb->B;
+  memset(&B, 0, sizeof B);
+  const int nd = I.h.ndim;
+  int T;
+  const int u = block_lines(I, axes, dbl, &T);
+  auto magic = [](int d) { return (0x100000000ULL / (unsigned long long)d) + 1ULL; };
+  // the tile's dimensions, innermost first: by the input's strides
+  std::vector<int> dims = axes;
+  if (u >= 0) dims.push_back(u);
+  std::stable_sort(dims.begin(), dims.end(), [&](int x, int y) { return I.h.m[x] < I.h.m[y]; });
+  B.ndim = (int)dims.size();
+  B.line_dim = -1;
+  B.points = 1;
+  std::vector<int> stride(nd, 0);
+  std::vector<i64> oi, oo;
+  for (int k = 0; k < B.ndim; k++) {
+    const int d = dims[k], n = d == u ? T : I.h.L[d];
+    if (d == u) B.line_dim = k;
+    B.dim[k].n = n;
+    B.dim[k].m_n = magic(n);
+    B.dim[k].at = (int)oi.size();
+    stride[d] = B.points;
+    B.points *= n;
+    for (int x = 0; x < n; x++) {
+      oi.push_back(d == u ? 0 : I.abs[d][x]);
+      oo.push_back(d == u ? 0 : U.abs[d][x]);
+    }
+  }
+  if (u < 0) {  // one line: its base in an entry (and a dimension) of its own
+    B.line_dim = B.ndim;
+    B.dim[B.ndim].n = 1;
+    B.dim[B.ndim].m_n = magic(1);
+    B.dim[B.ndim].at = (int)oi.size();
+    B.ndim++;
+    oi.push_back(0);
+    oo.push_back(0);
+  }
+  B.ntab = (int)oi.size();
+  pb->off_in = tb.put(oi.data(), oi.size() * sizeof(i64));
+  pb->off_out = tb.put(oo.data(), oo.size() * sizeof(i64));
+  // stages: the outermost transformed axis first and last (fused with the
+  // load and the store when its radices are powers of two), the others
+  // between, innermost last
+  std::vector<int> by_stride = axes;
+  std::stable_sort(by_stride.begin(), by_stride.end(), [&](int x, int y) { return stride[x] > stride[y]; });
+  std::vector<double> tw;
+  std::vector<std::vector<BlockStage>> of(by_stride.size());
+  for (size_t a = 0; a < by_stride.size(); a++) {
+    const int d = by_stride[a], n = I.h.L[d];
+    std::vector<int> rad;
+    block_radices(n, &rad);
+    if (a == 0 && rad.size() > 1 && (rad[0] & (rad[0] - 1)) != 0) std::reverse(rad.begin(), rad.end());
+    const std::vector<double> root = roots(n);
+    int ns = 1;
+    for (int r : rad) {
+      BlockStage st{};
+      st.dim = (int)(std::find(dims.begin(), dims.end(), d) - dims.begin());
+      st.radix = r;
+      st.s = stride[d];
+      st.span = stride[d] * n;
+      st.nr = n / r;
+      st.ns = ns;
+      st.m_s = magic(st.s);
+      st.m_nr = magic(st.nr);
+      st.m_ns = magic(st.ns);
+      st.tw = (int)(tw.size() / 2);
+      for (int q = 1; q < r && ns > 1; q++)
+        for (int jj = 0; jj < ns; jj++) {
+          const size_t k = (size_t)jj * q * (n / (ns * r));
+          tw.push_back(root[2 * k]);
+          tw.push_back(root[2 * k + 1]);
+        }
+      of[a].push_back(st);
+      ns *= r;
+    }
+  }
+  std::vector<BlockStage> seq;
+  const bool split = of[0].size() > 1;
+  for (size_t i = 0; i < of[0].size(); i++)
+    if (!split || i + 1 < of[0].size()) seq.push_back(of[0][i]);
+  for (size_t a = by_stride.size(); a-- > 1;)  // innermost first: the next outer axis may end the pass
+    for (auto &st : of[a]) seq.push_back(st);
+  if (split) seq.push_back(of[0].back());
+  B.nstage = (int)seq.size();
+  for (int i = 0; i < B.nstage; i++) B.st[i] = seq[i];
+  auto pow2 = [](int r) { return (r & (r - 1)) == 0; };
+  // (along the contiguous dimension a butterfly's points are nr apart: with
+  // fewer than 8 butterflies a line, lanes would be whole rows apart)
+  B.fuse_in = pow2(seq[0].radix) && (seq[0].s > 1 || seq[0].nr >= 8);
+  B.fuse_out = B.nstage >= 2 && pow2(seq.back().radix) && (seq.back().s > 1 || seq.back().nr >= 8);
+  if (tw.empty()) tw.assign(2, 0.0);
+  B.ntw = (int)(tw.size() / 2);
+  std::vector<char> img(tw.size() / 2 * 16);
+  twiddle_image(tw.data(), tw.size() / 2, dbl, img.data());
+  pb->tw = tb.put(img.data(), img.size());
+  // line bases
+  std::vector<int> batch;
+  long long nbatch = 1;
+  for (int d = 0; d < nd; d++)
+    if (d != u && std::find(axes.begin(), axes.end(), d) == axes.end()) {
+      batch.push_back(d);
+      nbatch *= I.h.L[d];
+    }
+  // slowest first, so that neighbouring tiles are close in memory
+  std::stable_sort(batch.begin(), batch.end(), [&](int x, int y) { return I.h.m[x] > I.h.m[y]; });
+  B.lines = u < 0 ? 1 : I.h.L[u];
+  B.tiles_u = (B.lines + T - 1) / T;
+  B.tiles = nbatch * B.tiles_u;
+  const int nu = B.tiles_u * T;
+  auto fill = [&](const Side &s) {
+    std::vector<i64> to((size_t)nbatch * nu);
+    std::vector<int> g(nd, 0);
+    for (long long b = 0; b < nbatch; b++) {
+      i64 base = 0;
+      for (int d : batch) base += s.abs[d][g[d]];
+      for (int l = 0; l < nu; l++) to[b * nu + l] = base + (u < 0 ? 0 : s.abs[u][l < B.lines ? l : 0]);
+      for (size_t k = batch.size(); k-- > 0;) {
+        if (++g[batch[k]] < s.h.L[batch[k]]) break;
+        g[batch[k]] = 0;
+      }
+    }
+    return tb.put(to.data(), to.size() * sizeof(i64));
+  };
+  pb->base_in = fill(I);
+  pb->base_out = fill(U);
+  static const bool nont = getenv("DM_NO_NONTEMPORAL") != nullptr;
+  B.stream_in = B.stream_out = nont ? 0 : 1;
+  B.inverse = inverse ? 1 : 0;
+  B.dbl = dbl;
+  B.ctw = !dbl && ctw ? 1 : 0;
+  B.in = in;
+  B.out = out;
+  fft_block_lds(&B);
+  return B.lds <= 160 * 1024 && B.tiles < (1LL << 31);
+}
+
 void *finalize_passes(dm_comm_t comm, TableBuilder &tb, std::vector<PendingPass> &pp,
-                      std::vector<FftLaunch> *out) {
+                      std::vector<FftLaunch> *out, std::vector<PendingBlock> *pb, std::vector<FftBlock> *blocks) {
   void *mem = device_alloc(std::max<size_t>(tb.host.size(), 256));
   if (mem == nullptr) {
     raise_error(comm, "FFT: device allocation of %zu bytes of tables failed", tb.host.size());
@@ -448,8 +670,24 @@ void *finalize_passes(dm_comm_t comm, TableBuilder &tb, std::vector<PendingPass>
   if (!tb.host.empty()) h2d(mem, tb.host.data(), tb.host.size());
   char *b = (char *)mem;
   out->clear();
+  if (pb != nullptr) {
+    blocks->clear();
+    for (auto &p : *pb) {
+      FftBlock B = p.B;
+      B.off_in = (const i64 *)(b + p.off_in);
+      B.off_out = (const i64 *)(b + p.off_out);
+      B.base_in = (const i64 *)(b + p.base_in);
+      B.base_out = (const i64 *)(b + p.base_out);
+      B.twiddle = b + p.tw;
+      blocks->push_back(B);
+    }
+  }
   for (auto &p : pp) {
     FftLaunch L = p.L;
+    if (L.block) {
+      out->push_back(L);
+      continue;
+    }
     for (int d = 0; d < L.ndim; d++) {
       L.off_in[d] = (const i64 *)(b + p.in_off[d]);
       L.off_out[d] = (const i64 *)(b + p.out_off[d]);

@@ -59,9 +59,21 @@ struct PendingPass {
 // false after raise_error when the axis cannot be done.
 bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, bool inverse, const void *in,
                void *out, TableBuilder &tb, PendingPass *pp, int ctw = 1);
+// The block pass (K5) over several whole axes, with offsets of its tables.
+struct PendingBlock {
+  FftBlock B;
+  size_t off_in = 0, off_out = 0, base_in = 0, base_out = 0, tw = 0;
+};
+// Whether block passes can take these axes of uniform layouts I -> U in one
+// pass: their points fit a tile, every length is a product of 2, 3, 5 and 7,
+// and both sides are read and written in runs of at least 128 bytes.
+bool block_fits(const Side &I, const Side &U, const std::vector<int> &axes, int dbl);
+bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int dbl, bool inverse, const void *in,
+                void *out, TableBuilder &tb, PendingBlock *pb, int ctw);
 // Upload the tables and resolve table pointers; returns the device block.
 void *finalize_passes(dm_comm_t comm, TableBuilder &tb, std::vector<PendingPass> &pp,
-                      std::vector<FftLaunch> *out);
+                      std::vector<FftLaunch> *out, std::vector<PendingBlock> *pb = nullptr,
+                      std::vector<FftBlock> *blocks = nullptr);
 
 // Axis d of h split into sub-axes 2d (y, A[d] points) and 2d+1 (z, L_d /
 // A[d] points) over g = y + A[d] * z, when owner and offset separate into

@@ -114,6 +114,7 @@ struct FftLaunch {
   void *out;
   long long tile_base;        // this launch runs tiles [tile_base, tile_base + nblocks)
   int pass_index;             // host bookkeeping: the pass this launch belongs to
+  int block;                  // 0: this line pass; else block pass block - 1 of the program instead
   int stream_in, stream_out;  // 1: non-temporal hint on the data loads / stores
   int ctw;                    // complex float: 1 compensated twiddle products, 0 the float part only
 };
@@ -141,6 +142,49 @@ int launch_fft_pass(const FftLaunch &p, void *stream);
 int fft_tile_capacity(int dbl, int column, int wide = 0);
 // (line, position) entries a non-uniform side of a tile keeps in LDS.
 int fft_line_positions();
+
+// ---- K5: several whole axes in one pass ------------------------------------
+// A tile holds every point of the transformed dimensions times n lines of
+// dimension line_dim (-1: none); dimensions innermost (contiguous in memory)
+// first.  Element offsets of a point: the sum of its dimensions' table
+// entries, the line dimension's being the tile's line bases.
+#define DM_BLOCK_DIMS 4
+struct BlockDim {
+  unsigned long long m_n;      // magic for n
+  int n;                       // points (lines per tile)
+  int at;                      // first entry in the offset tables
+};
+struct BlockStage {
+  unsigned long long m_s, m_nr, m_ns;
+  int dim, radix;
+  int s;                       // the dimension's stride in the tile
+  int span;                    // s times its points
+  int nr, ns;                  // butterflies per line, earlier points (Stockham)
+  int tw;                      // twiddles w^(jj r) at tw + (r - 1) ns + jj
+};
+struct FftBlock {
+  int ndim, line_dim;
+  BlockDim dim[DM_BLOCK_DIMS];
+  int nstage;
+  BlockStage st[24];
+  int points;                  // of a tile
+  int lines, tiles_u;          // length of the line axis, tiles along it
+  long long tiles;
+  int fuse_in, fuse_out;       // first stage on the loaded values, last one stored from registers
+  int inverse, dbl, ctw, stream_in, stream_out;
+  int ntab, ntw;               // entries of the offset tables and of the twiddles
+  const i64 *off_in, *off_out;
+  const i64 *base_in, *base_out;  // [tile * n + line]
+  const void *twiddle;
+  const void *in;
+  void *out;
+  int lds_tab, lds_tw;         // LDS offsets of the tables
+  size_t lds;
+};
+int fft_block_capacity(int dbl);
+// Fills lds_tab, lds_tw and lds.
+void fft_block_lds(FftBlock *p);
+int launch_fft_block(const FftBlock &p, void *stream);
 
 // ---- K4: twiddle multiply over every rank's local block -------------------
 // Rank r's block: count positions per axis at its memory strides; the
