@@ -112,9 +112,11 @@ __device__ __forceinline__ void block_stage(cx<R> *buf, const BlockStage &st, in
   __syncthreads();
 }
 
-// First stage on the loaded values (no twiddle).
-template <typename R, bool INV, int RADIX, int NTH>
-__device__ __forceinline__ void block_load(cx<R> *buf, const FftBlock &p, const lds_i64 *off, int nl) {
+// First stage on the loaded values (no stage twiddle; wl: the factors of a
+// split axis's second half, or null).
+template <typename R, bool INV, int RADIX, int NTH, bool CT>
+__device__ __forceinline__ void block_load(cx<R> *buf, const FftBlock &p, const lds_i64 *off,
+                                           const lds_tw<R, CT> *wl, int nl) {
   constexpr int K = kPer / RADIX;
   const BlockStage &st = p.st[0];
   const int nb = p.points / RADIX;
@@ -141,6 +143,9 @@ __device__ __forceinline__ void block_load(cx<R> *buf, const FftBlock &p, const 
       if (!ok[k])
 #pragma unroll
         for (int r = 0; r < RADIX; r++) v[k][r] = {0, 0};
+      if (p.wtab != nullptr)
+#pragma unroll
+        for (int r = 0; r < RADIX; r++) v[k][r] = twmul<INV, CT>(v[k][r], wl, j[k] + r * st.nr);
       dft<R, INV, RADIX>(v[k]);
 #pragma unroll
       for (int r = 0; r < RADIX; r++) buf[lds_pad(base[k] + (j[k] * RADIX + r) * st.s)] = v[k][r];
@@ -207,16 +212,24 @@ __global__ __launch_bounds__(sizeof(R) == 8 ? kThreadsD : kThreadsF, sizeof(R) =
     if constexpr (sizeof(TwL) == sizeof(TwG)) twl[i] = twg[i];
     else twl[i] = TwL{twg[i].x, twg[i].y};
   }
+  if (p.wtab != nullptr) {
+    const TwG *w = reinterpret_cast<const TwG *>(p.wtab);
+    const int q = (int)(tile / p.tiles_u / p.wdiv % p.wlen);
+    for (int x = threadIdx.x; x < p.wn; x += NTH) {
+      if constexpr (sizeof(TwL) == sizeof(TwG)) twl[p.ntw + x] = w[x * q];
+      else twl[p.ntw + x] = TwL{w[x * q].x, w[x * q].y};
+    }
+  }
   __syncthreads();
   const lds_tw<R, CT> *tw = (const lds_tw<R, CT> *)twl;
   int s0 = 0;
   const int s1 = p.fuse_out ? p.nstage - 1 : p.nstage;
   if (p.fuse_in) {
     switch (p.st[0].radix) {
-      case 2: block_load<R, INV, 2, NTH>(buf, p, in_off, nl); break;
-      case 4: block_load<R, INV, 4, NTH>(buf, p, in_off, nl); break;
-      case 8: block_load<R, INV, 8, NTH>(buf, p, in_off, nl); break;
-      case 16: block_load<R, INV, 16, NTH>(buf, p, in_off, nl); break;
+      case 2: block_load<R, INV, 2, NTH, CT>(buf, p, in_off, tw + p.ntw, nl); break;
+      case 4: block_load<R, INV, 4, NTH, CT>(buf, p, in_off, tw + p.ntw, nl); break;
+      case 8: block_load<R, INV, 8, NTH, CT>(buf, p, in_off, tw + p.ntw, nl); break;
+      case 16: block_load<R, INV, 16, NTH, CT>(buf, p, in_off, tw + p.ntw, nl); break;
       default: break;
     }
     s0 = 1;
@@ -304,7 +317,7 @@ void fft_block_lds(FftBlock *p) {
   p->lds_tab = (int)b;
   b += up((size_t)p->ntab * 2 * sizeof(i64));
   p->lds_tw = (int)b;
-  b += (size_t)p->ntw * (p->dbl || p->ctw ? 16 : 8);
+  b += (size_t)(p->ntw + p->wn) * (p->dbl || p->ctw ? 16 : 8);
   p->lds = b;
 }
 

@@ -497,7 +497,7 @@ static int block_lines(const Side &I, const std::vector<int> &axes, int dbl, int
 }
 
 bool block_fits(const Side &I, const Side &U, const std::vector<int> &axes, int dbl) {
-  if (!I.h.uniform || !U.h.uniform || axes.size() < 2 || axes.size() > DM_BLOCK_DIMS - 1) return false;
+  if (!I.h.uniform || !U.h.uniform || axes.empty() || axes.size() > DM_BLOCK_DIMS - 1) return false;
   long long points = 1, total = 1;
   size_t stages = 0;
   std::vector<int> rad;
@@ -523,7 +523,7 @@ bool block_fits(const Side &I, const Side &U, const std::vector<int> &axes, int 
 }
 
 bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int dbl, bool inverse, const void *in,
-                void *out, TableBuilder &tb, PendingBlock *pb, int ctw) {
+                void *out, TableBuilder &tb, PendingBlock *pb, int ctw, int wq) {
   FftBlock &B = pb->B;
   memset(&B, 0, sizeof B);
   const int nd = I.h.ndim;
@@ -639,7 +639,7 @@ bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int 
     for (long long b = 0; b < nbatch; b++) {
       i64 base = 0;
       for (int d : batch) base += s.abs[d][g[d]];
-      for (int l = 0; l < nu; l++) to[b * nu + l] = base + (u < 0 ? 0 : s.abs[u][l < B.lines ? l : 0]);
+      for (int l = 0; l < nu; l++) to[b * nu + l] = base + (u < 0 ? 0 : s.abs[u][l < B.lines ? I.order[u][l] : 0]);
       for (size_t k = batch.size(); k-- > 0;) {
         if (++g[batch[k]] < s.h.L[batch[k]]) break;
         g[batch[k]] = 0;
@@ -649,6 +649,19 @@ bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int 
   };
   pb->base_in = fill(I);
   pb->base_out = fill(U);
+  if (wq >= 0) {
+    const auto at = std::find(batch.begin(), batch.end(), wq);
+    if (at == batch.end() || !B.fuse_in || axes.size() != 1) return false;
+    B.wn = I.h.L[axes[0]];
+    B.wlen = I.h.L[wq];
+    B.wdiv = 1;
+    for (auto k = at + 1; k != batch.end(); ++k) B.wdiv *= I.h.L[*k];
+    const int N = B.wn * B.wlen;
+    const std::vector<double> w = roots(N);
+    std::vector<char> wi((size_t)N * 16);
+    twiddle_image(w.data(), N, dbl, wi.data());
+    pb->wtab = (long)tb.put(wi.data(), wi.size());
+  }
   static const bool nont = getenv("DM_NO_NONTEMPORAL") != nullptr;
   B.stream_in = B.stream_out = nont ? 0 : 1;
   B.inverse = inverse ? 1 : 0;
@@ -679,6 +692,7 @@ void *finalize_passes(dm_comm_t comm, TableBuilder &tb, std::vector<PendingPass>
       B.base_in = (const i64 *)(b + p.base_in);
       B.base_out = (const i64 *)(b + p.base_out);
       B.twiddle = b + p.tw;
+      B.wtab = p.wtab >= 0 ? b + p.wtab : nullptr;
       blocks->push_back(B);
     }
   }

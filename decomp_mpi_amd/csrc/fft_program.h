@@ -63,13 +63,17 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
 struct PendingBlock {
   FftBlock B;
   size_t off_in = 0, off_out = 0, base_in = 0, base_out = 0, tw = 0;
+  long wtab = -1;
 };
 // Whether block passes can take these axes of uniform layouts I -> U in one
 // pass: their points fit a tile, every length is a product of 2, 3, 5 and 7,
 // and both sides are read and written in runs of at least 128 bytes.
 bool block_fits(const Side &I, const Side &U, const std::vector<int> &axes, int dbl);
+// wq >= 0: axes is the second half of an axis of N points whose first half's
+// frequencies are the coordinates of axis wq; the points are multiplied by
+// w_N^(x q) first.  False when the pass cannot be done.
 bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int dbl, bool inverse, const void *in,
-                void *out, TableBuilder &tb, PendingBlock *pb, int ctw);
+                void *out, TableBuilder &tb, PendingBlock *pb, int ctw, int wq = -1);
 // Upload the tables and resolve table pointers; returns the device block.
 void *finalize_passes(dm_comm_t comm, TableBuilder &tb, std::vector<PendingPass> &pp,
                       std::vector<FftLaunch> *out, std::vector<PendingBlock> *pb = nullptr,

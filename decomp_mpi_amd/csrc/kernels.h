@@ -176,6 +176,12 @@ struct FftBlock {
   const i64 *off_in, *off_out;
   const i64 *base_in, *base_out;  // [tile * n + line]
   const void *twiddle;
+  // the second half of an axis of N = n * len points done as two: point x of
+  // the one transformed dimension is first multiplied by w_N^(x q), q
+  // the tile's batch coordinate (tile / tiles_u / wdiv) % wlen (null: none)
+  const void *wtab;            // w_N^m, m < N
+  int wn, wlen;
+  long long wdiv;
   const void *in;
   void *out;
   int lds_tab, lds_tw;         // LDS offsets of the tables

@@ -331,6 +331,119 @@ static bool dense_layout(const std::vector<int> &L, const std::vector<int> &orde
   return true;
 }
 
+// An axis whose one-pass tile holds so few lines that a column walk touches
+// 32 bytes or less per row (2048 points and more; complex doubles at a stride
+// of 64 KiB have the wide tile's rows up to 2048): two passes of about
+// sqrt(N) points instead, each over whole rows of the fastest axis.  The
+// first does the b-point transforms of g = y + a z over z, the second
+// multiplies by w_N^(y q) and does the a-point ones over y; frequency q + b p
+// comes out.  A 4096 x 2048 complex-double inverse took 100 us for its
+// 64-byte rows and 400 for its 16-byte ones: 208 us with this, in three
+// passes.  Arrays of 16 MiB and less stay in the caches and gain nothing from
+// wider rows (4096 x 64: 49 us a step in two passes, 61 in three); in three
+// dimensions the fourth pass costs what 32-byte rows do (64 x 2048 x 64
+// complex floats 319 us a step with them, 384 split; 64 x 4096 x 64 complex
+// doubles, 16-byte rows, 2059 against 932).
+static int long_factor(int n, int dbl, i64 stride, int row_bytes) {
+  const int es = dbl ? 16 : 8;
+  const bool wide = dbl && stride * es >= (64 << 10);
+  if (dm::fft_tile_capacity(dbl, 1, wide) / n * es > row_bytes) return 0;
+  for (int a = (int)std::sqrt((double)n); a >= 8; a--)
+    if (n % a == 0) return a;  // y points; z has n / a
+  return 0;
+}
+
+// The fused program with every long axis split (false: leave it to the
+// others).  Both sides must share their fastest axis f; everything between
+// is one natural layout (f fastest, in the last side's order) in w1, run in
+// place.
+static bool compile_split_axes(SplitPlan plan, bool inverse, const dm::Side &first, const dm::Side &last,
+                               const std::vector<int> &axes, void *src, void *dst, void *w1, int slots,
+                               i64 wslot, dm_fft_program *prog) {
+  dm_split_ext *x = plan->ext;
+  const int nd = x->ndim, f = first.h.fastest;
+  if (!first.h.uniform || !last.h.uniform || last.h.fastest != f || axes.size() < 2 || x->L[f] < 16) return false;
+  i64 total = 1;
+  for (int l : x->L) total *= l;
+  if (total * (x->dbl ? 16 : 8) <= (16 << 20)) return false;
+  const int row_bytes = axes.size() == 2 ? 32 : 16;
+  std::vector<int> fa(nd, 1), fb(nd, 1);
+  bool any = false;
+  for (int d : axes) {
+    const int a = d == f ? 0 : long_factor(x->L[d], x->dbl, last.h.m[d], row_bytes);
+    if (a == 0) continue;
+    fa[d] = a;
+    fb[d] = x->L[d] / a;
+    any = true;
+  }
+  if (!any) return false;
+  // sub-axis 2d: y in, p out; 2d + 1: z in, q out
+  dm::HostLayout hi, ho;
+  std::string why;
+  if (!dm::split_layout(first.h, fa, &hi, &why) || !dm::split_layout(last.h, fb, &ho, &why)) return false;
+  for (int d = 0; d < nd; d++) {
+    if (fa[d] == 1) continue;
+    std::swap(ho.L[2 * d], ho.L[2 * d + 1]);
+    std::swap(ho.rank_part[2 * d], ho.rank_part[2 * d + 1]);
+    std::swap(ho.off[2 * d], ho.off[2 * d + 1]);
+    std::swap(ho.m[2 * d], ho.m[2 * d + 1]);
+    for (int r = 0; r < ho.proc_used; r++)
+      std::swap(ho.strides[(size_t)r * 2 * nd + 2 * d], ho.strides[(size_t)r * 2 * nd + 2 * d + 1]);
+  }
+  const dm::Side I = dm::make_side(hi, first.slot), U = dm::make_side(ho, last.slot);
+  std::vector<int> ord(2 * nd);
+  for (int i = 0; i < 2 * nd; i++) ord[i] = i;
+  const int fs = 2 * f + 1;
+  std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) {
+    if (a == fs || b == fs) return a == fs && b != fs;
+    const bool la = hi.L[a] > 1, lb = hi.L[b] > 1;
+    if (la != lb) return lb;  // (the slowest axes are the ones split over the slots)
+    return hi.m[a] < hi.m[b];
+  });
+  dm::HostLayout h;
+  if (!dense_layout(hi.L, ord, std::min(slots, plan->comm->world->nranks), (i64)plan->extent, &h)) return false;
+  const std::vector<int> natural = h.off[fs], owner = h.rank_part[fs];
+  for (int i = 0; i < hi.L[fs]; i++) {
+    h.off[fs][U.order[fs][i]] = natural[i];
+    h.rank_part[fs][U.order[fs][i]] = owner[i];
+  }
+  const dm::Side M = dm::make_side(h, wslot);
+  dm::TableBuilder tb;
+  std::vector<dm::PendingPass> pp;
+  std::vector<dm::PendingBlock> pb;
+  // the passes: f, then the others by stride (a split axis: z, then y)
+  struct Step {
+    int sub, q;
+  };
+  std::vector<Step> steps = {{fs, -1}};
+  for (int i = 0; i < 2 * nd; i++) {
+    const int d = ord[i] / 2;
+    if (ord[i] == fs || ord[i] % 2 == 0 || hi.L[2 * d] * hi.L[2 * d + 1] <= 1) continue;
+    steps.push_back({2 * d + 1, -1});
+    if (fa[d] > 1) steps.push_back({2 * d, 2 * d + 1});
+  }
+  for (size_t i = 0; i < steps.size(); i++) {
+    const int sub = steps[i].sub, d = sub / 2;
+    const dm::Side &si = i == 0 ? I : M, &so = i + 1 == steps.size() ? U : M;
+    void *bi = i == 0 ? src : w1, *bo = i + 1 == steps.size() ? dst : w1;
+    pp.emplace_back();
+    if (fa[d] > 1) {
+      pb.emplace_back();
+      if (!dm::block_fits(si, so, {sub}, x->dbl) ||
+          !dm::plan_block(si, so, {sub}, x->dbl, inverse, bi, bo, tb, &pb.back(), x->ctw, steps[i].q))
+        return false;
+      memset(&pp.back().L, 0, sizeof pp.back().L);
+      pp.back().L.block = (int)pb.size();
+    } else if (!dm::plan_pass(plan->comm, si, so, sub, x->dbl, inverse, bi, bo, tb, &pp.back(), x->ctw)) {
+      return false;
+    }
+  }
+  prog->mem = dm::finalize_passes(plan->comm, tb, pp, &prog->passes, &pb, &prog->blocks);
+  prog->inverse = inverse ? 1 : 0;
+  for (size_t i = 0; i < prog->passes.size(); i++) prog->passes[i].pass_index = (int)i;
+  return prog->mem != nullptr;
+}
+
 // Build one direction's passes.  Forward: dat (start) -> ... -> W0
 // (output); backward: W0 (output) -> ... -> dat (start).  Each direction
 // orders its own passes the same way: the axis fastest in memory on the
@@ -409,6 +522,7 @@ static bool compile_direction(SplitPlan plan, bool inverse, const dm::Side &S, c
   // backward 180 -> 131 us, 64^3 58 -> 50).
   {
     const dm::Side &first = inverse ? O : S;
+    const i64 wslot = O.slot;
     void *src = inverse ? w0 : dat, *dst = inverse ? dat : w0;
     std::vector<dm::PendingPass> pp(1);
     std::vector<dm::PendingBlock> pb(1);
@@ -420,6 +534,7 @@ static bool compile_direction(SplitPlan plan, bool inverse, const dm::Side &S, c
       return prog->mem != nullptr;
     };
     memset(&pp[0].L, 0, sizeof pp[0].L);
+    if (compile_split_axes(plan, inverse, first, last, axes, src, dst, w1, slots, wslot, prog)) return true;
     if (n >= 2 && dm::block_fits(first, last, axes, x->dbl) &&
         dm::plan_block(first, last, axes, x->dbl, inverse, src, dst, tb, &pb[0], x->ctw))
       return finish();
@@ -431,9 +546,10 @@ static bool compile_direction(SplitPlan plan, bool inverse, const dm::Side &S, c
       std::sort(rest.begin(), rest.end(), [&](int a, int b) { return first.h.m[a] < first.h.m[b]; });
       // lines of the remaining axis in rows of 128 bytes
       const int cells = 128 / (x->dbl ? 16 : 8);
-      std::vector<int> ord = {f, rest[0], rest[1]};
+      std::vector<int> ord = {f};
       for (int d = 0; d < nd; d++)
         if (x->L[d] <= 1) ord.push_back(d);
+      ord.insert(ord.end(), rest.begin(), rest.end());
       dm::HostLayout h;
       if (x->L[rest[1]] * cells <= dm::fft_tile_capacity(x->dbl, 1) &&
           dense_layout(x->L, ord, std::min(slots, plan->comm->world->nranks), (i64)plan->extent, &h)) {
