@@ -19,6 +19,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <tuple>
 #include <vector>
 
 #include "dm_batch.h"
@@ -57,7 +58,9 @@ struct dm_batch {
   // tile's points, [1] larger
   PassTables planes[2];
   size_t plane_lds[2] = {0, 0};
+  int plane_tw[2] = {0, 0};
   int plane_primes[2] = {0, 0};
+  void *d_planes = nullptr;  // plane schedules
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   void *graph_stream = nullptr;
@@ -82,7 +85,8 @@ static void release_bound(DmBatch b) {
   dm::device_free(b->d_ptrs);
   dm::device_free(b->d_sched);
   dm::device_free(b->d_tw);
-  b->d_ptrs = b->d_sched = b->d_tw = nullptr;
+  dm::device_free(b->d_planes);
+  b->d_ptrs = b->d_sched = b->d_tw = b->d_planes = nullptr;
 }
 
 extern "C" DmBatch dm_batch_plan(int count, int ndim, const int *shapes, int precision, int direction) {
@@ -181,6 +185,96 @@ bool batch_sched_any(const BatchSched &S) {
   return false;
 }
 
+// Whether planes of n1 rows of n2 points run as plane tiles: within the
+// kernel's points, each side at most the LDS-twiddle limit, radices with a
+// butterfly kernel.
+static bool plane_fits(int n1, int n2, int dbl) {
+  if ((long long)n1 * n2 > batch_plane_capacity(dbl) || !batch_tw_in_lds(n1) || !batch_tw_in_lds(n2)) return false;
+  std::vector<int> r;
+  for (int n : {n1, n2}) {
+    choose_radices(n, &r, true);
+    for (int q : r)
+      if (!has_radix_kernel(q)) return false;
+  }
+  return true;
+}
+
+// Schedule of plane tiles: the columns' first stage, the rows' stages, the
+// columns' other ones, a power of two last where there are two.
+static void make_plane_sched(int n1, int n2, int T, int radix_order, BatchPlane *out, std::vector<double> *tw) {
+  BatchPlane P{};
+  P.plane = n1 * n2;
+  P.points = T * n1 * n2;
+  auto odd_pow2 = [](int n, std::vector<int> *odd) {
+    odd->clear();
+    for (int p : {13, 11, 7, 5, 3})
+      while (n % p == 0) {
+        odd->push_back(p);
+        n /= p;
+      }
+    int k = 0;
+    while (n > 1) {
+      n /= 2;
+      k++;
+    }
+    return k;
+  };
+  std::vector<int> odd, cols, rows;
+  int k = odd_pow2(n1, &odd);
+  const int first = (k + 1) / 2, last = k / 2;  // at most 16 each: n1 <= 256
+  if (k > 0) cols.push_back(1 << (radix_order == DM_BATCH_RADIX_SMALL_FIRST && last > 0 ? last : first));
+  cols.insert(cols.end(), odd.begin(), odd.end());
+  if (last > 0) cols.push_back(1 << (radix_order == DM_BATCH_RADIX_SMALL_FIRST ? first : last));
+  k = odd_pow2(n2, &rows);
+  for (int left = (k + 3) / 4; left > 0; left--) {
+    const int b = (k + left - 1) / left;
+    rows.push_back(1 << b);
+    k -= b;
+  }
+  if (radix_order == DM_BATCH_RADIX_LARGE_FIRST) std::reverse(rows.begin(), rows.end());
+  auto stages = [&](int n, int s, const std::vector<int> &rad) {
+    const std::vector<double> root = roots(n);
+    std::vector<BlockStage> v;
+    int ns = 1;
+    for (int r : rad) {
+      BlockStage st{};
+      st.radix = r;
+      st.s = s;
+      st.span = s * n;
+      st.nr = n / r;
+      st.ns = ns;
+      st.m_s = magic(s);
+      st.m_nr = magic(n / r);
+      st.m_ns = magic(ns);
+      st.tw = (int)(tw->size() / 2);
+      for (int q = 1; q < r && ns > 1; q++)
+        for (int jj = 0; jj < ns; jj++) {
+          const size_t at = (size_t)jj * q * (n / (ns * r));
+          tw->push_back(root[2 * at]);
+          tw->push_back(root[2 * at + 1]);
+        }
+      v.push_back(st);
+      ns *= r;
+    }
+    return v;
+  };
+  tw->clear();
+  const std::vector<BlockStage> c = stages(n1, n2, cols), w = stages(n2, 1, rows);
+  std::vector<BlockStage> seq;
+  if (!c.empty()) seq.push_back(c[0]);
+  seq.insert(seq.end(), w.begin(), w.end());
+  if (!c.empty()) seq.insert(seq.end(), c.begin() + 1, c.end());
+  auto pow2 = [](int r) { return (r & (r - 1)) == 0; };
+  P.nstage = (int)seq.size();
+  for (int i = 0; i < P.nstage; i++) P.st[i] = seq[i];
+  // (fused stages of the columns only: along the rows their lanes would be
+  // whole butterflies apart)
+  P.fuse_in = !c.empty() && n2 > 1 && pow2(c[0].radix);
+  P.fuse_out = c.size() > 1 && n2 > 1 && pow2(c.back().radix);
+  P.ntw = (int)(tw->size() / 2);
+  *out = P;
+}
+
 // Host image of a batch: tiles per axis pass (last axis first), schedules
 // and their stage-ordered twiddles (complex double), LDS need, and whether a
 // radix 5, 7, 11 or 13 occurs.  DM_BATCH_TILE_PLANES: a transform whose
@@ -221,37 +315,44 @@ bool build_batch_host(int count, int ndim, const int *shapes, int dbl, int tile_
     return id;
   };
   h.tiles.assign(ndim, std::vector<BatchTile>());
+  std::map<std::tuple<int, int, int>, int> plane_of;  // (n1, n2, T) -> plane schedule
+  int plane_ntw[2] = {0, 0};
   for (int i = 0; i < count; i++) {
     const int *n = &shapes[(size_t)i * ndim];
     int dlast = ndim;  // axes [0, dlast) get line tiles
-    if (tile_choice == DM_BATCH_TILE_PLANES && ndim >= 2) {
-      const int n1 = n[ndim - 2], n2 = n[ndim - 1];
-      size_t plds = batch_plane_lds_bytes(dbl, n1, n2);
-      std::vector<int> r1, r2;  // planes take butterfly-kernel radices only
-      choose_radices(n1, &r1, true);
-      choose_radices(n2, &r2, true);
-      for (int r : r1) plds = has_radix_kernel(r) ? plds : 0;
-      for (int r : r2) plds = has_radix_kernel(r) ? plds : 0;
-      if (plds > 0 && n1 <= cap && n2 <= cap) {
-        long long outer = 1;
-        for (int e = 0; e < ndim - 2; e++) outer *= n[e];
-        const int rows = schedule(n2, n1), cols = schedule(n1, n2);
-        const int k = (long long)n1 * n2 <= cap ? 0 : 1;
-        if (has_primes(h.sched[rows]) || has_primes(h.sched[cols])) h.plane_primes[k] = 1;
-        h.plane_lds[k] = std::max(h.plane_lds[k], plds);
-        for (long long o = 0; o < outer; o++) {
-          BatchTile t{};
-          t.base = o * n1 * n2;
-          t.ps = 1;
-          t.xform = i;
-          t.sched = rows;
-          t.sched2 = cols;
-          t.nl = n1;
-          t.row = 2;
-          h.planes[k].push_back(t);
-        }
-        dlast = ndim - 2;
+    if (tile_choice == DM_BATCH_TILE_PLANES && ndim >= 2 && plane_fits(n[ndim - 2], n[ndim - 1], dbl)) {
+      const int n1 = n[ndim - 2], n2 = n[ndim - 1], plane = n1 * n2;
+      long long outer = 1;
+      for (int e = 0; e < ndim - 2; e++) outer *= n[e];
+      const int k = plane <= batch_plane_small() ? 0 : 1;
+      const int T = (int)std::min<long long>(outer, (k == 0 ? batch_plane_small() : plane) / plane);
+      const auto key = std::make_tuple(n1, n2, T);
+      auto it = plane_of.find(key);
+      if (it == plane_of.end()) {
+        BatchPlane P{};
+        std::vector<double> block;
+        make_plane_sched(n1, n2, T, radix_order, &P, &block);
+        P.tw_off = (int)(h.tw.size() / 2);
+        h.tw.insert(h.tw.end(), block.begin(), block.end());
+        it = plane_of.emplace(key, (int)h.plane_sched.size()).first;
+        h.plane_sched.push_back(P);
       }
+      const BatchPlane &P = h.plane_sched[it->second];
+      for (int q = 0; q < P.nstage; q++)
+        if (P.st[q].radix % 2) h.plane_primes[k] = 1;
+      h.plane_tw[k] = std::max(h.plane_tw[k], (int)batch_plane_tw_at(dbl, P.points));
+      plane_ntw[k] = std::max(plane_ntw[k], P.ntw);
+      for (long long o = 0; o < outer; o += T) {
+        BatchTile t{};
+        t.base = o * plane;
+        t.ps = 1;
+        t.xform = i;
+        t.sched = it->second;
+        t.nl = (int)std::min<long long>(T, outer - o);
+        t.row = 2;
+        h.planes[k].push_back(t);
+      }
+      dlast = ndim - 2;
     }
     for (int d = 0; d < dlast; d++) {
       long long inner = 1, outer = 1;
@@ -291,6 +392,7 @@ bool build_batch_host(int count, int ndim, const int *shapes, int dbl, int tile_
       }
     }
   }
+  for (int k = 0; k < 2; k++) h.plane_lds[k] = h.plane_tw[k] + (size_t)plane_ntw[k] * 16;
   // Every other launch walks its tiles in reverse transform order, so that it
   // starts on the transforms the launch before it wrote last, which are
   // still in the memory-side cache (tiles are independent: the order changes
@@ -323,6 +425,7 @@ static bool bind_tables(DmBatch b) {
     b->planes[k].tiles = std::move(h.planes[k]);
     b->plane_lds[k] = h.plane_lds[k];
     b->plane_primes[k] = h.plane_primes[k];
+    b->plane_tw[k] = h.plane_tw[k];
   }
   std::vector<dm::BatchSched> &sched = h.sched;
   std::vector<double> &tw = h.tw;
@@ -341,7 +444,8 @@ static bool bind_tables(DmBatch b) {
   std::vector<char> twimg(tw.size() / 2 * 16);
   dm::twiddle_image(tw.data(), tw.size() / 2, b->dbl, twimg.data());
   b->d_tw = up(twimg.data(), twimg.size());
-  if (!b->d_ptrs || !b->d_sched || !b->d_tw) {
+  b->d_planes = up(h.plane_sched.data(), h.plane_sched.size() * sizeof(dm::BatchPlane));
+  if (!b->d_ptrs || !b->d_sched || !b->d_tw || !b->d_planes) {
     raise_error(nullptr, "dm_batch_bind: device allocation or copy failed");
     return false;
   }
@@ -363,8 +467,7 @@ static bool bind_tables(DmBatch b) {
       raise_error(nullptr, "dm_batch_bind: device allocation or copy failed");
       return false;
     }
-    const long long res = k == 0 ? dm::batch_resident_groups(b->dbl, b->plane_primes[0], b->plane_lds[0])
-                                 : dm::batch_plane_resident_groups(b->plane_lds[1]);
+    const long long res = dm::batch_plane_resident_groups(b->dbl, k, b->plane_lds[k]);
     pl.grid = b->grid_mode == DM_BATCH_GRID_PERSISTENT ? std::min<long long>((long long)pl.tiles.size(), res)
                                                        : (long long)pl.tiles.size();
   }
@@ -430,6 +533,8 @@ extern "C" int dm_batch_run(DmBatch b, void *stream) {
     L.inverse = b->inverse;
     L.primes = b->plane_primes[k];
     L.plane = k == 0 ? 2 : 1;
+    L.planes = (const dm::BatchPlane *)b->d_planes;
+    L.plane_tw = b->plane_tw[k];
     L.grid = pl.grid;
     L.lds = b->plane_lds[k];
     if (!dm::launch_ok(nullptr, dm::launch_batch_pass(L, stream), "dm_batch_run: plane pass launch")) return 1;
@@ -563,14 +668,7 @@ extern "C" double dm_batch_bytes_moved(DmBatch b) {
     int passes = b->ndim;
     // the plane rule of build_batch_host
     if (b->tile_choice == DM_BATCH_TILE_PLANES && b->ndim >= 2) {
-      const int n1 = n[b->ndim - 2], n2 = n[b->ndim - 1], cap = dm::batch_tile_capacity(b->dbl);
-      std::vector<int> r1, r2;
-      dm::choose_radices(n1, &r1, true);
-      dm::choose_radices(n2, &r2, true);
-      bool kern = true;
-      for (int r : r1) kern = kern && dm::has_radix_kernel(r);
-      for (int r : r2) kern = kern && dm::has_radix_kernel(r);
-      if (kern && dm::batch_plane_lds_bytes(b->dbl, n1, n2) > 0 && n1 <= cap && n2 <= cap) passes -= 1;
+      if (dm::plane_fits(n[b->ndim - 2], n[b->ndim - 1], b->dbl)) passes -= 1;
     }
     total += 2.0 * passes * pts * (b->dbl ? 16 : 8);
   }

@@ -21,7 +21,7 @@
 
 #include <algorithm>
 
-#include "fft_device.h"
+#include "fft_block_device.h"
 #include "kernels.h"
 
 namespace dm {
@@ -29,13 +29,10 @@ namespace {
 
 using namespace fftdev;
 
-constexpr int kPer = 16;        // points per thread
 constexpr int kThreadsD = 256;  // 4096 complex doubles
 constexpr int kThreadsF = 512;  // 8192 complex floats
 
 typedef __attribute__((address_space(3))) i64 lds_i64;
-template <typename R, bool CT>
-using lds_tw = __attribute__((address_space(3))) typename tw_local<R, CT>::type;
 
 // Coordinates of tile element e, innermost dimension first.
 __device__ __forceinline__ void decode(const FftBlock &p, int e, int *x) {
@@ -67,49 +64,6 @@ __device__ __forceinline__ i64 offset_of(const FftBlock &p, const lds_i64 *off, 
       if (d == p.line_dim) *line = x[d];
     }
   return a;
-}
-
-// Butterfly b of a stage: its first point's element index without the
-// butterfly's place along the axis, and that place.
-__device__ __forceinline__ void butterfly(const BlockStage &st, int b, int *base, int *j) {
-  const int q = fdiv(b, st.m_s), inner = b - q * st.s;
-  const int outer = fdiv(q, st.m_nr);
-  *j = q - outer * st.nr;
-  *base = outer * st.span + inner;
-}
-
-template <typename R, bool INV, int RADIX, int NTH, bool CT>
-__device__ __forceinline__ void block_stage(cx<R> *buf, const BlockStage &st, int points, const lds_tw<R, CT> *tw) {
-  constexpr int K = (kPer + RADIX - 1) / RADIX;
-  const int nb = points / RADIX;
-  cx<R> v[K][RADIX];
-  int dst[K];
-#pragma unroll
-  for (int k = 0; k < K; k++) {
-    const int b = threadIdx.x + k * NTH;
-    dst[k] = -1;
-    if (b < nb) {
-      int base, j;
-      butterfly(st, b, &base, &j);
-      const int jn = fdiv(j, st.m_ns), jj = j - jn * st.ns;
-#pragma unroll
-      for (int r = 0; r < RADIX; r++) v[k][r] = buf[lds_pad(base + (j + r * st.nr) * st.s)];
-      if (st.ns > 1) {
-        const lds_tw<R, CT> *t = tw + st.tw + jj;
-#pragma unroll
-        for (int r = 1; r < RADIX; r++) v[k][r] = twmul<INV, CT>(v[k][r], t, (r - 1) * st.ns);
-      }
-      dft<R, INV, RADIX>(v[k]);
-      dst[k] = base + (jn * st.ns * RADIX + jj) * st.s;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < K; k++)
-    if (dst[k] >= 0)
-#pragma unroll
-      for (int r = 0; r < RADIX; r++) buf[lds_pad(dst[k] + r * st.ns * st.s)] = v[k][r];
-  __syncthreads();
 }
 
 // First stage on the loaded values (no stage twiddle; wl: the factors of a

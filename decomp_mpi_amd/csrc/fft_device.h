@@ -261,16 +261,12 @@ __device__ __forceinline__ int lds_index(int line, int x, int ls) { return line 
 // TW: pointer to the twiddles, typed by where they live (an LDS-qualified
 // pointer reads with LDS instructions; a generic one would use flat loads);
 // CT: compensated twiddle products (complex float).
-// COL: the lines are the columns of the LDS tile (point x of line l at
-// x * ls + pad(l): a plane's second axis), consecutive butterflies on
-// consecutive lines; m_t: magic for T.
-template <typename R, bool INV, int RADIX, int CAP, int NTH, bool CT, typename TW, bool COL = false>
-__device__ __forceinline__ void stage_lds(cx<R> *buf, const StageInfo &si, int T, int ls, TW tw,
-                                          unsigned long long m_t = 0) {
+template <typename R, bool INV, int RADIX, int CAP, int NTH, bool CT, typename TW>
+__device__ __forceinline__ void stage_lds(cx<R> *buf, const StageInfo &si, int T, int ls, TW tw) {
   constexpr int K = (CAP / RADIX + NTH - 1) / NTH;
   const int nr = si.nr, ns = si.ns;
   const int nb = T * nr;
-  auto at = [&](int l, int x) { return COL ? x * ls + lds_pad(l) : l * ls + lds_pad(x); };
+  auto at = [&](int l, int x) { return l * ls + lds_pad(x); };
   cx<R> v[K][RADIX];
   int dst[K];
 #pragma unroll
@@ -278,14 +274,8 @@ __device__ __forceinline__ void stage_lds(cx<R> *buf, const StageInfo &si, int T
     int b = threadIdx.x + k * NTH;
     dst[k] = -1;
     if (b < nb) {
-      int l, j;
-      if constexpr (COL) {
-        j = fdiv(b, m_t);
-        l = b - j * T;
-      } else {
-        l = fdiv(b, si.m_nr);
-        j = b - l * nr;
-      }
+      int l = fdiv(b, si.m_nr);
+      int j = b - l * nr;
       int jn = fdiv(j, si.m_ns);
       int jj = j - jn * ns;
 #pragma unroll

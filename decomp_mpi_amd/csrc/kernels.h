@@ -219,9 +219,8 @@ int launch_scale(const ScaleLaunch &p, void *stream);
 // ---- K3: batched local FFT pass (many transforms, one axis of each) --------
 // A tile holds nl (<= T) lines of N points of one transform: point x of line
 // l at element base + l * (row ? N : 1) + x * ps of that transform's array.
-// row 2: a plane tile -- the last two axes of one transform at once, nl = T
-// rows of N contiguous points (schedule `sched`), then its N columns of T
-// points (schedule `sched2`, tile height N) in the same LDS tile.
+// row 2: a plane tile -- the last two axes of nl consecutive planes of one
+// transform at once (`sched`: the plane schedule).
 struct BatchTile {
   long long base;
   long long ps;
@@ -229,7 +228,14 @@ struct BatchTile {
   int sched;
   int nl;
   int row;
-  int sched2;
+};
+// Planes of n1 rows of n2 points, T of them a tile: the stages of both axes
+// over the tile's linear order, their twiddles at tw_off of the launch's.
+struct BatchPlane {
+  int plane, points;           // n1 * n2, T times that
+  int nstage, fuse_in, fuse_out;
+  int tw_off, ntw;
+  BlockStage st[16];
 };
 // Per (line length, tile height, radix order): stages and twiddles.
 struct BatchSched {
@@ -267,7 +273,9 @@ struct BatchLaunch {
   int dbl, inverse;
   int primes;                  // some schedule has a radix 5, 7, 11 or 13
   int long_lines;              // some schedule's lines are too long for twiddles in LDS
-  int plane;                   // plane tiles (row 2) only: 2 within the line tile's points, 1 larger
+  int plane;                   // plane tiles (row 2) only: 2 up to batch_plane_small() points, 1 larger
+  const BatchPlane *planes;    // their schedules
+  int plane_tw;                // LDS offset of their twiddles
   int any;                     // some schedule has a direct-sum stage (line tiles only)
   long long grid;              // persistent workgroups (tile loop inside)
   size_t lds;
@@ -280,11 +288,13 @@ int launch_copy16(const void *src, void *dst, long long n16, void *stream);
 // schedules, their stage-ordered roots as complex doubles, LDS bytes.
 struct BatchHost {
   std::vector<std::vector<BatchTile>> tiles;
-  // plane tiles (run before tiles[0]): [0] planes within the line tile's
-  // points (the line kernel's shape), [1] larger ones
+  // plane tiles (run before tiles[0]): [0] of planes up to
+  // batch_plane_small() points, [1] of larger ones
   std::vector<BatchTile> planes[2];
   size_t plane_lds[2] = {0, 0};
+  int plane_tw[2] = {0, 0};    // LDS offset of the twiddles
   int plane_primes[2] = {0, 0};
+  std::vector<BatchPlane> plane_sched;
   std::vector<BatchSched> sched;
   std::vector<double> tw;
   size_t lds = 0;
@@ -309,13 +319,13 @@ int batch_tile_height(int N, long long inner, int dbl, int tile_choice);
 size_t batch_lds_bytes(int dbl, int T, int N);
 bool batch_tw_in_lds(int N);
 long long batch_resident_groups(int dbl, int primes, size_t lds);
-// Plane tiles (BatchTile row 2): the most points a plane may hold, the LDS
-// bytes of a plane of T rows of N points (0 when it does not fit: too many
-// points, a side above the LDS-twiddle limit, or over 160 KiB), and the
-// resident workgroups of the large-plane kernel (planes above the line
-// tile's points) for a launch's LDS.
+// Plane tiles (BatchTile row 2): the most points a plane may hold, the most
+// a plane of the 256-thread kernel may, the LDS offset of a tile's twiddles,
+// and the resident workgroups for a launch's LDS.
 int batch_plane_capacity(int dbl);
-size_t batch_plane_lds_bytes(int dbl, int T, int N);
-long long batch_plane_resident_groups(size_t lds);
+int batch_plane_small();
+size_t batch_plane_tw_at(int dbl, int points);
+long long batch_plane_resident_groups(int dbl, int large, size_t lds);
+int launch_batch_planes(const BatchLaunch &p, void *stream);
 
 }  // namespace dm
