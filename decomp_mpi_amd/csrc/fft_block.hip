@@ -155,24 +155,27 @@ __global__ __launch_bounds__(sizeof(R) == 8 ? kThreadsD : kThreadsF, sizeof(R) =
   const int nl = p.line_dim >= 0 ? min(T, p.lines - (int)(tile % p.tiles_u) * T) : 1;
   // both sides' offset tables (the lines' bases of this tile in their
   // dimension's place) and the twiddles
+  const TwG *twg = reinterpret_cast<const TwG *>(p.twiddle);
+  auto put = [&](int i, TwG w) {
+    if constexpr (sizeof(TwL) == sizeof(TwG)) twl[i] = w;
+    else twl[i] = TwL{w.x, w.y};
+  };
+  // (every table's first loads go out together)
+  TwG tw0 = twg[min((int)threadIdx.x, p.ntw - 1)], w0{};
+  const TwG *wtab = reinterpret_cast<const TwG *>(p.wtab);
+  const int q = wtab != nullptr ? (int)(tile / p.tiles_u / p.wdiv % p.wlen) : 0;
+  if (wtab != nullptr) w0 = wtab[min((int)threadIdx.x, p.wn - 1) * q];
   const int line_at = p.line_dim >= 0 ? p.dim[p.line_dim].at : p.ntab - 1;
   for (int i = threadIdx.x; i < p.ntab; i += NTH) {
     const bool l = i >= line_at && i < line_at + T;
     in_off[i] = l ? p.base_in[tile * T + (i - line_at)] : p.off_in[i];
     out_off[i] = l ? p.base_out[tile * T + (i - line_at)] : p.off_out[i];
   }
-  const TwG *twg = reinterpret_cast<const TwG *>(p.twiddle);
-  for (int i = threadIdx.x; i < p.ntw; i += NTH) {
-    if constexpr (sizeof(TwL) == sizeof(TwG)) twl[i] = twg[i];
-    else twl[i] = TwL{twg[i].x, twg[i].y};
-  }
-  if (p.wtab != nullptr) {
-    const TwG *w = reinterpret_cast<const TwG *>(p.wtab);
-    const int q = (int)(tile / p.tiles_u / p.wdiv % p.wlen);
-    for (int x = threadIdx.x; x < p.wn; x += NTH) {
-      if constexpr (sizeof(TwL) == sizeof(TwG)) twl[p.ntw + x] = w[x * q];
-      else twl[p.ntw + x] = TwL{w[x * q].x, w[x * q].y};
-    }
+  if ((int)threadIdx.x < p.ntw) put(threadIdx.x, tw0);
+  for (int i = threadIdx.x + NTH; i < p.ntw; i += NTH) put(i, twg[i]);
+  if (wtab != nullptr) {
+    if ((int)threadIdx.x < p.wn) put(p.ntw + threadIdx.x, w0);
+    for (int x = threadIdx.x + NTH; x < p.wn; x += NTH) put(p.ntw + x, wtab[x * q]);
   }
   __syncthreads();
   const lds_tw<R, CT> *tw = (const lds_tw<R, CT> *)twl;

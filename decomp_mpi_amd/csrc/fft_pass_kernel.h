@@ -28,7 +28,7 @@ using namespace fftdev;
 
 struct Pass {
   FftLaunch p;
-  StageInfo st[16];
+  StageInfo st[kMaxStages];
   unsigned long long m_n, m_t;  // magics for N and T
   int ls;                        // LDS line stride (complex elements)
   int fuse_in;                   // first stage runs on the loaded registers
@@ -73,10 +73,10 @@ struct LineAddr<true> {
   lds_i64 *base;
   __host__ __device__ static size_t bytes(int T, int) { return (size_t)T * sizeof(i64); }
   __device__ void init(char *mem, int, int) { base = (lds_i64 *)(mem); }
-  __device__ void set_line(const FftLaunch &p, const i64 *const *abs, const int *g, int l) {
+  __device__ void set_line(const FftLaunch &p, const i64 *abs, const int *g, int l) {
     i64 a = 0;
     for (int d = 0; d < p.ndim; d++)
-      if (d != p.t) a += abs[d][g[d]];
+      if (d != p.t) a += abs[p.at[d] + g[d]];
     base[l] = a;
   }
   __device__ __forceinline__ i64 at(const FftLaunch &, const FftSide &s, const i64 *absT, int l, int x) const {
@@ -117,11 +117,11 @@ struct LineAddr<false> {
   __device__ void set_line(const FftLaunch &p, const FftSide &s, const int *g, int l, int q) {
     int R = s.posrank[q];
     for (int d = 0; d < p.ndim; d++)
-      if (d != p.t) R += s.rank[d][g[d]];
+      if (d != p.t) R += s.rank[p.at[d] + g[d]];
     const i64 *m = s.strides + (i64)R * p.ndim;
     i64 a = (i64)R * s.slot;
     for (int d = 0; d < p.ndim; d++)
-      if (d != p.t) a += m[d] * s.off[d][g[d]];
+      if (d != p.t) a += m[d] * s.off[p.at[d] + g[d]];
     base[l * np + q] = a;
     str[l * np + q] = m[p.t];
   }
@@ -378,8 +378,8 @@ __global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 4) vo
     }
   __syncthreads();
 
-  const i64 *inT = p.off_in[p.t];
-  const i64 *outT = p.off_out[p.t];
+  const i64 *inT = p.off_in + p.at[p.t];
+  const i64 *outT = p.off_out + p.at[p.t];
   const cx<R> *in = reinterpret_cast<const cx<R> *>(p.in);
   cx<R> *out = reinterpret_cast<cx<R> *>(p.out);
 

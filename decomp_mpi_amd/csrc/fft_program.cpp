@@ -123,7 +123,7 @@ bool axis_supported(int n, int dbl, std::string *why) {
   if (n > cap) {
     snprintf(msg, sizeof msg, "axis length %d exceeds the %d-point tile of the %s pass", n, cap,
              dbl ? "complex-double" : "complex-float");
-  } else if (!choose_radices(n, &rad, true) || (int)rad.size() > 16) {
+  } else if (!choose_radices(n, &rad, true) || (int)rad.size() > kMaxStages) {
     snprintf(msg, sizeof msg, "axis length %d has more than 16 prime factors", n);
   } else {
     return true;
@@ -160,7 +160,7 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     return false;
   }
   std::vector<int> rad;
-  if (!choose_radices(L.N, &rad, true) || (int)rad.size() > 16) {
+  if (!choose_radices(L.N, &rad, true) || (int)rad.size() > kMaxStages) {
     raise_error(comm, "FFT: axis length %d has more than 16 prime factors", L.N);
     return false;
   }
@@ -259,10 +259,15 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   L.inverse = inverse ? 1 : 0;
   L.dbl = dbl;
   L.ctw = (!dbl && ctw) ? 1 : 0;
-  for (int d = 0; d < nd; d++) {
-    pp->in_off[d] = tb.put(I.abs[d].data(), I.abs[d].size() * sizeof(i64));
-    pp->out_off[d] = tb.put(U.abs[d].data(), U.abs[d].size() * sizeof(i64));
-  }
+  // per-axis tables one after another
+  for (int d = 1; d < nd; d++) L.at[d] = L.at[d - 1] + L.L[d - 1];
+  auto joined = [&](const auto &tab) {
+    std::decay_t<decltype(tab[0])> v;
+    for (int d = 0; d < nd; d++) v.insert(v.end(), tab[d].begin(), tab[d].end());
+    return tb.put(v.data(), v.size() * sizeof(v[0]));
+  };
+  pp->in_off = joined(I.abs);
+  pp->out_off = joined(U.abs);
   // rank-dependent strides: owner, local offset and per-rank stride tables
   auto side = [&](const Side &s, FftSide &fs, PendingSide &ps, const std::vector<int> &pos) {
     fs.uniform = s.h.uniform ? 1 : 0;
@@ -310,10 +315,8 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     }
     ps.xt = tb.put(xt.data(), xt.size() * sizeof(int));
     ps.posrank = tb.put(pos.data(), pos.size() * sizeof(int));
-    for (int d = 0; d < nd; d++) {
-      ps.rank[d] = tb.put(s.h.rank_part[d].data(), s.h.L[d] * sizeof(int));
-      ps.off[d] = tb.put(s.h.off[d].data(), s.h.L[d] * sizeof(int));
-    }
+    ps.rank = joined(s.h.rank_part);
+    ps.off = joined(s.h.off);
     ps.strides = tb.put(s.h.strides.data(), s.h.strides.size() * sizeof(i64));
   };
   side(I, L.sin, pp->sin, pos_in);
@@ -507,7 +510,7 @@ bool block_fits(const Side &I, const Side &U, const std::vector<int> &axes, int 
     stages += rad.size();
   }
   for (int l : I.h.L) total *= l;
-  if (stages > 24) return false;
+  if (stages > kBlockStages) return false;
   int T;
   const int u = block_lines(I, axes, dbl, &T);
   // both sides in runs of 128 bytes along the same axis, or the whole array
@@ -702,16 +705,12 @@ void *finalize_passes(dm_comm_t comm, TableBuilder &tb, std::vector<PendingPass>
       out->push_back(L);
       continue;
     }
-    for (int d = 0; d < L.ndim; d++) {
-      L.off_in[d] = (const i64 *)(b + p.in_off[d]);
-      L.off_out[d] = (const i64 *)(b + p.out_off[d]);
-    }
+    L.off_in = (const i64 *)(b + p.in_off);
+    L.off_out = (const i64 *)(b + p.out_off);
     auto side = [&](FftSide &fs, const PendingSide &ps) {
       if (fs.uniform) return;
-      for (int d = 0; d < L.ndim; d++) {
-        fs.rank[d] = (const int *)(b + ps.rank[d]);
-        fs.off[d] = (const int *)(b + ps.off[d]);
-      }
+      fs.rank = (const int *)(b + ps.rank);
+      fs.off = (const int *)(b + ps.off);
       fs.strides = (const i64 *)(b + ps.strides);
       fs.xt = (const int *)(b + ps.xt);
       fs.posrank = (const int *)(b + ps.posrank);

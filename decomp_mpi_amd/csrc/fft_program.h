@@ -40,15 +40,12 @@ struct TableBuilder {
 
 // Table offsets of one side's non-uniform addressing data.
 struct PendingSide {
-  size_t rank[DM_MAX_DIMS];
-  size_t off[DM_MAX_DIMS];
-  size_t strides, xt, posrank;
+  size_t rank, off, strides, xt, posrank;
 };
 
 struct PendingPass {
   FftLaunch L;
-  size_t in_off[DM_MAX_DIMS];
-  size_t out_off[DM_MAX_DIMS];
+  size_t in_off, out_off;
   PendingSide sin, sout;
   long ord_in = -1, ord_out = -1, ord_u = -1, tw = -1;
   long line_in = -1, line_out = -1;

@@ -148,13 +148,11 @@ struct DevLayout {
   int proc_used;
   int uniform;
   int pad_;
-  const int *rank[DM_MAX_DIMS];
-  const int *off[DM_MAX_DIMS];
-  const i64 *addr[DM_MAX_DIMS];   // uniform: m_d * off_d(g)
+  int at[DM_MAX_DIMS];            // first entry of axis d in the per-axis tables
+  const int *rank;
+  const int *off;
+  const i64 *addr;                // uniform: m_d * off_d(g)
   const i64 *strides;             // [proc_used * ndim]
-  const int *pos[DM_MAX_DIMS];    // coordinate -> rank position (index into posrank)
-  const int *posrank[DM_MAX_DIMS];  // distinct owner contributions, ascending
-  const unsigned *part[DM_MAX_DIMS];  // uniform: (rank, addr) pairs, 32 bits each
 };
 
 // Device copy of a HostLayout's tables.
@@ -163,6 +161,9 @@ struct DeviceLayout {
   void *mem = nullptr;
   size_t bytes = 0;
   int np[DM_MAX_DIMS] = {0};      // rank positions per axis
+  const int *pos[DM_MAX_DIMS] = {nullptr};        // coordinate -> rank position (index into posrank)
+  const int *posrank[DM_MAX_DIMS] = {nullptr};    // distinct owner contributions, ascending
+  const unsigned *part[DM_MAX_DIMS] = {nullptr};  // uniform: (rank, addr) pairs, 32 bits each
   void upload(const HostLayout &h);
   void release();
 };

@@ -76,10 +76,15 @@ struct FftSide {
   int lin;                     // one position, local offset x at point x
   const int *xt;               // point x of t: position, local offset
   const int *posrank;          // owner contribution of each position
-  const int *rank[DM_MAX_DIMS];
-  const int *off[DM_MAX_DIMS];
+  const int *rank, *off;       // owner contributions and local offsets, axis d's at FftLaunch::at[d]
   const i64 *strides;          // [proc_used * ndim]
 };
+
+// Most stages of a pass: a line has at most 8192 = 3^8 + ... points, and two
+// factors of two or more share a stage.  (Kernel arguments are copied and
+// fetched with every launch: 1.3 KiB of them cost a 64^3 pencil pass, three
+// launches, 0.5 us each against 0.8 KiB.)
+constexpr int kMaxStages = 8;
 
 struct FftLaunch {
   FftSide sin, sout;           // non-uniform addressing (used when !uniform)
@@ -89,7 +94,7 @@ struct FftLaunch {
   int T;
   int N;
   int nstage;
-  int radix[16];
+  int radix[kMaxStages];
   int in_row, out_row;        // 1: walk memory along t; 0: along u
   int nbatch;
   int batch_axis[DM_MAX_DIMS];
@@ -97,8 +102,8 @@ struct FftLaunch {
   int merge_v, merge_k;        // merge_k > 1: a tile holds all L[u] lines for merge_k consecutive
                                //   values of batch axis merge_v (tiles_u 1; merge_k divides L[v])
   long long nblocks;
-  const i64 *off_in[DM_MAX_DIMS];
-  const i64 *off_out[DM_MAX_DIMS];
+  int at[DM_MAX_DIMS];        // first entry of axis d in the per-axis tables
+  const i64 *off_in, *off_out;  // absolute offsets
   const int *ord_in;          // row mode: t coordinates in input address order (or null)
   const int *ord_out;         // row mode: t coordinates in output address order (or null)
   const int *ord_u;           // tile line l holds u coordinate ord_u[u0 + l] (or u0 + l)
@@ -149,6 +154,7 @@ int fft_line_positions();
 // first.  Element offsets of a point: the sum of its dimensions' table
 // entries, the line dimension's being the tile's line bases.
 #define DM_BLOCK_DIMS 4
+constexpr int kBlockStages = 10;
 struct BlockDim {
   unsigned long long m_n;      // magic for n
   int n;                       // points (lines per tile)
@@ -166,7 +172,7 @@ struct FftBlock {
   int ndim, line_dim;
   BlockDim dim[DM_BLOCK_DIMS];
   int nstage;
-  BlockStage st[24];
+  BlockStage st[kBlockStages];
   int points;                  // of a tile
   int lines, tiles_u;          // length of the line axis, tiles along it
   long long tiles;

@@ -533,9 +533,9 @@ bool enqueue_reshape(dm_comm_t comm, ReshapePlan plan, const void *src, void *ds
   auto side = [&](const dm::DeviceLayout &dl, ReshapeSide &to) {
     const int ax[2] = {pg->a, pg->b};
     for (int i = 0; i < 2; i++) {
-      to.pos[i] = dl.dev.pos[ax[i]];
-      to.posrank[i] = dl.dev.posrank[ax[i]];
-      to.part[i] = dl.dev.part[ax[i]];
+      to.pos[i] = dl.pos[ax[i]];
+      to.posrank[i] = dl.posrank[ax[i]];
+      to.part[i] = dl.part[ax[i]];
       to.np[i] = dl.np[ax[i]];
     }
   };
@@ -641,7 +641,14 @@ void DeviceLayout::upload(const HostLayout &h) {
     bytes += (n + 255) & ~(size_t)255;
     return at;
   };
-  std::vector<size_t> at_rank(h.ndim), at_off(h.ndim), at_addr(h.ndim), at_pos(h.ndim), at_pr(h.ndim), at_part(h.ndim);
+  int points = 0;
+  for (int d = 0; d < h.ndim; d++) {
+    dev.at[d] = points;
+    points += h.L[d];
+  }
+  const size_t at_rank = take(points * sizeof(int)), at_off = take(points * sizeof(int));
+  const size_t at_addr = take(points * sizeof(i64));
+  std::vector<size_t> at_pos(h.ndim), at_pr(h.ndim), at_part(h.ndim);
   std::vector<std::vector<int>> pr(h.ndim);
   for (int d = 0; d < h.ndim; d++) {
     pr[d] = rank_positions(h, d);
@@ -649,20 +656,17 @@ void DeviceLayout::upload(const HostLayout &h) {
     at_pos[d] = take(h.L[d] * sizeof(int));
     at_pr[d] = take(pr[d].size() * sizeof(int));
     at_part[d] = take(2 * h.L[d] * sizeof(unsigned));
-    at_rank[d] = take(h.L[d] * sizeof(int));
-    at_off[d] = take(h.L[d] * sizeof(int));
-    at_addr[d] = take(h.L[d] * sizeof(i64));
   }
   size_t at_str = take(h.strides.size() * sizeof(i64));
   std::vector<char> host(bytes, 0);
   for (int d = 0; d < h.ndim; d++) {
-    memcpy(&host[at_rank[d]], h.rank_part[d].data(), h.L[d] * sizeof(int));
-    memcpy(&host[at_off[d]], h.off[d].data(), h.L[d] * sizeof(int));
+    memcpy(&host[at_rank] + dev.at[d] * sizeof(int), h.rank_part[d].data(), h.L[d] * sizeof(int));
+    memcpy(&host[at_off] + dev.at[d] * sizeof(int), h.off[d].data(), h.L[d] * sizeof(int));
     int *po = (int *)&host[at_pos[d]];
     for (int g = 0; g < h.L[d]; g++)
       po[g] = (int)(std::lower_bound(pr[d].begin(), pr[d].end(), h.rank_part[d][g]) - pr[d].begin());
     memcpy(&host[at_pr[d]], pr[d].data(), pr[d].size() * sizeof(int));
-    i64 *ad = (i64 *)&host[at_addr[d]];
+    i64 *ad = (i64 *)&host[at_addr] + dev.at[d];
     unsigned *pt = (unsigned *)&host[at_part[d]];
     for (int g = 0; g < h.L[d]; g++) {
       ad[g] = h.m[d] * h.off[d][g];
@@ -683,13 +687,13 @@ void DeviceLayout::upload(const HostLayout &h) {
   dev.proc_used = h.proc_used;
   dev.uniform = h.uniform ? 1 : 0;
   for (int d = 0; d < h.ndim; d++) {
-    dev.rank[d] = (const int *)(b + at_rank[d]);
-    dev.off[d] = (const int *)(b + at_off[d]);
-    dev.addr[d] = (const i64 *)(b + at_addr[d]);
-    dev.pos[d] = (const int *)(b + at_pos[d]);
-    dev.posrank[d] = (const int *)(b + at_pr[d]);
-    dev.part[d] = (const unsigned *)(b + at_part[d]);
+    pos[d] = (const int *)(b + at_pos[d]);
+    posrank[d] = (const int *)(b + at_pr[d]);
+    part[d] = (const unsigned *)(b + at_part[d]);
   }
+  dev.rank = (const int *)(b + at_rank);
+  dev.off = (const int *)(b + at_off);
+  dev.addr = (const i64 *)(b + at_addr);
   dev.strides = (const i64 *)(b + at_str);
 }
 

@@ -50,9 +50,9 @@ __device__ __forceinline__ void partial_init(const DevLayout &Lt, const ReshapeL
     int d = p.batch_axis[k];
     int g = (int)(bidx % p.L[d]);
     bidx /= p.L[d];
-    q.rank += Lt.rank[d][g];
-    if (UNIFORM) q.addr += Lt.addr[d][g];
-    else q.off[k] = Lt.off[d][g];
+    q.rank += Lt.rank[Lt.at[d] + g];
+    if (UNIFORM) q.addr += Lt.addr[Lt.at[d] + g];
+    else q.off[k] = Lt.off[Lt.at[d] + g];
   }
 }
 
@@ -62,15 +62,15 @@ __device__ __forceinline__ void partial_init(const DevLayout &Lt, const ReshapeL
 template <bool UNIFORM>
 __device__ __forceinline__ i64 locate(const DevLayout &Lt, const ReshapeLaunch &p, const Partial &q,
                                       int a, int ga, int b, int gb, i64 slot) {
-  int R = q.rank + Lt.rank[a][ga] + (b != a ? Lt.rank[b][gb] : 0);
+  int R = q.rank + Lt.rank[Lt.at[a] + ga] + (b != a ? Lt.rank[Lt.at[b] + gb] : 0);
   if (R >= Lt.proc_used) return -1;
   i64 off;
   if (UNIFORM) {
-    off = q.addr + Lt.addr[a][ga] + (b != a ? Lt.addr[b][gb] : 0);
+    off = q.addr + Lt.addr[Lt.at[a] + ga] + (b != a ? Lt.addr[Lt.at[b] + gb] : 0);
   } else {
     const i64 *m = Lt.strides + (i64)R * Lt.ndim;
-    off = m[a] * Lt.off[a][ga];
-    if (b != a) off += m[b] * Lt.off[b][gb];
+    off = m[a] * Lt.off[Lt.at[a] + ga];
+    if (b != a) off += m[b] * Lt.off[Lt.at[b] + gb];
     for (int k = 0; k < p.nbatch; k++) off += m[p.batch_axis[k]] * q.off[k];
   }
   return (i64)R * slot + off;
@@ -118,15 +118,15 @@ __global__ __launch_bounds__(NTHREADS) void reshape_tile2d(ReshapeLaunch p) {
     // uniform source: the tile axes' table entries are loaded once (one per
     // column, one per row) and shared by the NB slices
     const int gbc = min(b0 + tx, Lb - 1);
-    const int rb = p.src.rank[p.b][gbc];
-    const i64 ab = p.src.addr[p.b][gbc];
+    const int rb = p.src.rank[p.src.at[p.b] + gbc];
+    const i64 ab = p.src.addr[p.src.at[p.b] + gbc];
     int ra[RPT];
     i64 aa[RPT];
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
       const int gac = min(a0 + ty + k * ROWS, La - 1);
-      ra[k] = p.src.rank[p.a][gac];
-      aa[k] = p.src.addr[p.a][gac];
+      ra[k] = p.src.rank[p.src.at[p.a] + gac];
+      aa[k] = p.src.addr[p.src.at[p.a] + gac];
     }
 #pragma unroll
     for (int n = 0; n < NB; n++)
@@ -164,15 +164,15 @@ __global__ __launch_bounds__(NTHREADS) void reshape_tile2d(ReshapeLaunch p) {
   i64 d[NB][RPT];
   if constexpr (UD) {
     const int gac = min(a0 + tx, La - 1);
-    const int ra = p.dst.rank[p.a][gac];
-    const i64 aa = p.dst.addr[p.a][gac];
+    const int ra = p.dst.rank[p.dst.at[p.a] + gac];
+    const i64 aa = p.dst.addr[p.dst.at[p.a] + gac];
     int rb[RPT];
     i64 ab[RPT];
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
       const int gbc = min(b0 + ty + k * ROWS, Lb - 1);
-      rb[k] = p.dst.rank[p.b][gbc];
-      ab[k] = p.dst.addr[p.b][gbc];
+      rb[k] = p.dst.rank[p.dst.at[p.b] + gbc];
+      ab[k] = p.dst.addr[p.dst.at[p.b] + gbc];
     }
 #pragma unroll
     for (int n = 0; n < NB; n++)
@@ -315,7 +315,7 @@ struct SideAddr<BYTES, true, NB, OT> {
       const uint2 q = *reinterpret_cast<const uint2 *>(s.part[axis] + 2 * (size_t)g);
       return q.x * (unsigned)slot + q.y * (unsigned)BYTES;
     } else {
-      return (i64)L.rank[d][g] * slot + L.addr[d][g] * BYTES;
+      return (i64)L.rank[L.at[d] + g] * slot + L.addr[L.at[d] + g] * BYTES;
     }
   }
   __device__ __forceinline__ i64 base(int n) const { return batch[n]; }
@@ -340,7 +340,7 @@ struct SideAddr<BYTES, false, NB, OT> {
       const int R = rank + s.posrank[0][qa] + s.posrank[1][qb];
       const i64 *m = L.strides + (i64)R * L.ndim;
       i64 addr = 0;
-      batch_walk(p, bidx, [&](int d, int g) { addr += m[d] * L.off[d][g]; });
+      batch_walk(p, bidx, [&](int d, int g) { addr += m[d] * L.off[L.at[d] + g]; });
       lds_ot *q = tab + 3 * (e * NB + n);
       q[0] = (OT)((i64)R * slot + addr * BYTES);
       q[1] = (OT)(m[p.a] * BYTES);
@@ -349,7 +349,7 @@ struct SideAddr<BYTES, false, NB, OT> {
   }
   // axis: 0 for a, 1 for b
   __device__ __forceinline__ Part part(const ReshapeSide &s, const DevLayout &L, int axis, int d, int g, i64) const {
-    return {s.pos[axis][g], L.off[d][g]};
+    return {s.pos[axis][g], L.off[L.at[d] + g]};
   }
   __device__ __forceinline__ i64 base(int) const { return 0; }
   __device__ __forceinline__ OT at(const ReshapeSide &s, int n, Part a, Part b) const {
@@ -366,10 +366,10 @@ __device__ __forceinline__ void batch_parts(const ReshapeLaunch &p, long long bi
   int rs = 0, rd = 0;
   i64 as = 0, ad = 0;
   batch_walk(p, bidx, [&](int d, int g) {
-    rs += p.src.rank[d][g];
-    rd += p.dst.rank[d][g];
-    if constexpr (US) as += p.src.addr[d][g];
-    if constexpr (UD) ad += p.dst.addr[d][g];
+    rs += p.src.rank[p.src.at[d] + g];
+    rd += p.dst.rank[p.dst.at[d] + g];
+    if constexpr (US) as += p.src.addr[p.src.at[d] + g];
+    if constexpr (UD) ad += p.dst.addr[p.dst.at[d] + g];
   });
   src.init(p.ss, p.src, p, bidx, n, lds, p.src_bytes, rs, as);
   dst.init(p.sd, p.dst, p, bidx, n, lds + (US ? 0 : p.ss.np[0] * p.ss.np[1] * 3 * NB * sizeof(OT)), p.dst_bytes, rd,
