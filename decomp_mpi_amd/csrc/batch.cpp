@@ -29,7 +29,7 @@
 
 namespace {
 
-unsigned long long magic(int d) { return (0x100000000ULL / (unsigned long long)d) + 1ULL; }
+unsigned magic(int d) { return dm::magic_for(d); }
 
 struct PassTables {
   std::vector<dm::BatchTile> tiles;
@@ -155,6 +155,7 @@ void make_batch_sched(int N, int T, int radix_order, BatchSched *out, std::vecto
     S.st[s].ns = ns;
     S.st[s].m_nr = magic(N / R);
     S.st[s].m_ns = magic(ns);
+    stage_steps(&S.st[s]);
     int stride = N / (ns * R);
     for (int r = 1; r < R; r++)
       for (int jj = 0; jj < ns; jj++) {

@@ -51,8 +51,8 @@ __device__ __forceinline__ void gstore(gptr<R> data, long long i, cx<R> v) {
 // Butterfly bi of a stage with nr butterflies per line: row walks put
 // consecutive butterflies of a line on consecutive threads, column walks
 // consecutive lines (so that each butterfly input is one coalesced access).
-__device__ __forceinline__ void bfly(int bi, int row, int nr, unsigned long long m_nr, int T,
-                                     unsigned long long m_t, int &l, int &j) {
+__device__ __forceinline__ void bfly(int bi, int row, int nr, unsigned m_nr, int T,
+                                     unsigned m_t, int &l, int &j) {
   if (row) {
     l = fdiv(bi, m_nr);
     j = bi - l * nr;
@@ -78,9 +78,12 @@ __device__ __forceinline__ void load_first(cx<R> *buf, const BatchSched &S, cons
     int bi = threadIdx.x + q * NTH;
     bfly(min(bi, nb - 1), d.row, nr, st.m_nr, S.T, S.m_t, lk[q], jk[q]);
     ok[q] = bi < nb && lk[q] < d.nl;
+    // (one product, then steps of nr points; absent butterflies read the
+    // tile's first element)
+    const long long a0 = ok[q] ? (long long)lk[q] * lstride + (long long)jk[q] * d.ps : 0;
+    const long long step = ok[q] ? nr * d.ps : 0;
 #pragma unroll
-    for (int r = 0; r < RADIX; r++)
-      a[q][r] = ok[q] ? (long long)lk[q] * lstride + (long long)(jk[q] + r * nr) * d.ps : 0;
+    for (int r = 0; r < RADIX; r++) a[q][r] = a0 + r * step;
   }
   cx<R> v[K][RADIX];
 #pragma unroll
@@ -94,9 +97,10 @@ __device__ __forceinline__ void load_first(cx<R> *buf, const BatchSched &S, cons
       for (int r = 0; r < RADIX; r++) v[q][r] = {0, 0};
     dft<R, INV, RADIX>(v[q]);
     if ((int)threadIdx.x + q * NTH < nb) {
-      const int base = lk[q] * ls, idx = jk[q] * RADIX;
+      // (a power-of-two butterfly's outputs do not straddle a pad)
+      cx<R> *to = buf + lk[q] * ls + lds_pad(jk[q] * RADIX);
 #pragma unroll
-      for (int r = 0; r < RADIX; r++) buf[base + lds_pad(idx + r)] = v[q][r];
+      for (int r = 0; r < RADIX; r++) to[r] = v[q][r];
     }
   }
 }
@@ -116,17 +120,22 @@ __device__ __forceinline__ void last_store(const cx<R> *buf, const BatchSched &S
     bfly(min(bi, nb - 1), d.row, nr, st.m_nr, S.T, S.m_t, l, j);
     const bool ok = bi < nb && l < d.nl;
     cx<R> v[RADIX];
+    if (st.rs) {
+      const cx<R> *from = buf + l * ls + lds_pad(j);
 #pragma unroll
-    for (int r = 0; r < RADIX; r++) v[r] = buf[l * ls + lds_pad(j + r * nr)];
+      for (int r = 0; r < RADIX; r++) v[r] = from[r * st.rs];
+    } else {
+#pragma unroll
+      for (int r = 0; r < RADIX; r++) v[r] = buf[l * ls + lds_pad(j + r * nr)];
+    }
 #pragma unroll
     for (int r = 1; r < RADIX; r++) v[r] = twmul<INV, (sizeof(R) == 4)>(v[r], tw, (nr - 1) + (r - 1) * nr + j);
     dft<R, INV, RADIX>(v);
-    if (ok)
+    if (ok) {
+      const long long at = (long long)l * lstride + (long long)j * d.ps, step = nr * d.ps;
 #pragma unroll
-      for (int r = 0; r < RADIX; r++) {
-        const long long at = (long long)l * lstride + (long long)(j + r * nr) * d.ps;
-        gstore(data, at, v[r]);
-      }
+      for (int r = 0; r < RADIX; r++) gstore(data, at + r * step, v[r]);
+    }
   }
 }
 

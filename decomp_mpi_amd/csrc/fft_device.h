@@ -241,10 +241,13 @@ __device__ __forceinline__ void dft(cx<R> *v) {
   else dft_prime<R, INV, RADIX>(v);
 }
 
-// ---- fast division by runtime constants (numerators below 2^16) -------------
+// ---- fast division by runtime constants (n < 2^16, d <= 2^13) ---------------
+// n / d from m = magic_for(d) = 2^31 / d + 1: (2 n + 1) m / 2^32 is (n + 1/2) /
+// d plus less than 2^-15, and n + 1/2 stays at least 1/2 (so 2^-14 after the
+// division) away from a multiple of d.
 
-__device__ __forceinline__ int fdiv(int n, unsigned long long magic) {
-  return (int)(((unsigned long long)(unsigned)n * magic) >> 32);
+__device__ __forceinline__ int fdiv(int n, unsigned m) {
+  return (int)__umulhi(2u * (unsigned)n + 1u, m);
 }
 
 
@@ -278,8 +281,14 @@ __device__ __forceinline__ void stage_lds(cx<R> *buf, const StageInfo &si, int T
       int j = b - l * nr;
       int jn = fdiv(j, si.m_ns);
       int jj = j - jn * ns;
+      if (si.rs) {
+        const cx<R> *from = buf + at(l, j);
 #pragma unroll
-      for (int r = 0; r < RADIX; r++) v[k][r] = buf[at(l, j + r * nr)];
+        for (int r = 0; r < RADIX; r++) v[k][r] = from[r * si.rs];
+      } else {
+#pragma unroll
+        for (int r = 0; r < RADIX; r++) v[k][r] = buf[at(l, j + r * nr)];
+      }
       if (ns > 1) {
         // stage-ordered table: consecutive jj read consecutive entries
         TW tws = tw + (ns - 1) + jj;
@@ -297,8 +306,18 @@ __device__ __forceinline__ void stage_lds(cx<R> *buf, const StageInfo &si, int T
   for (int k = 0; k < K; k++) {
     if (dst[k] >= 0) {
       int l = dst[k] >> 16, idxd = dst[k] & 0xffff;
+      if (si.ws > 0) {
+        cx<R> *to = buf + at(l, idxd);
 #pragma unroll
-      for (int r = 0; r < RADIX; r++) buf[at(l, idxd + r * ns)] = v[k][r];
+        for (int r = 0; r < RADIX; r++) to[r * si.ws] = v[k][r];
+      } else if (RADIX % 2 == 0 && si.ws < 0) {
+        cx<R> *to = buf + at(l, idxd);
+#pragma unroll
+        for (int r = 0; r < RADIX; r++) to[8 * r + r / 2] = v[k][r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < RADIX; r++) buf[at(l, idxd + r * ns)] = v[k][r];
+      }
     }
   }
   __syncthreads();
@@ -319,7 +338,7 @@ __device__ __forceinline__ void stage_lds_any(cx<R> *buf, const StageInfo &si, i
   constexpr int K = (CAP + NTH - 1) / NTH;
   const int nr = si.nr, ns = si.ns;
   const int items = T * nr * p;  // T * N <= CAP
-  const unsigned long long m_p = 0x100000000ull / (unsigned)p + 1;
+  const unsigned m_p = 0x80000000u / (unsigned)p + 1;
   cx<R> y[K];
   int dst[K];
 #pragma unroll
@@ -373,6 +392,19 @@ __device__ __forceinline__ void gather(cx<R> *v, P src, const i64 *a, bool nt) {
   } else {
 #pragma unroll
     for (int k = 0; k < N; k++) v[k] = src[a[k]];
+  }
+}
+
+// N elements at equal steps from `to`.
+template <int N, typename R>
+__device__ __forceinline__ void store_steps(cx<R> *to, i64 step, const cx<R> *v, bool nt) {
+  typedef R v2 __attribute__((ext_vector_type(2)));
+  if (nt) {
+#pragma unroll
+    for (int k = 0; k < N; k++) __builtin_nontemporal_store(v2{v[k].x, v[k].y}, reinterpret_cast<v2 *>(to + k * step));
+  } else {
+#pragma unroll
+    for (int k = 0; k < N; k++) to[k * step] = v[k];
   }
 }
 

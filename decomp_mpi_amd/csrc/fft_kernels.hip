@@ -92,8 +92,19 @@ int launch_fft_pass(const FftLaunch &p, void *stream) {
     P.st[s].ns = ns;
     P.st[s].m_nr = magic_for(p.N / r);
     P.st[s].m_ns = magic_for(ns);
+    stage_steps(&P.st[s]);
     ns *= r;
   }
+  // Step between a fused stage's points where it is one number: along an
+  // affine side, or over whole runs of an axis in equal blocks.
+  auto step = [](const FftSide &s, int nr) -> i64 {
+    if (!s.uniform) return 0;
+    if (s.aff) return nr * s.aff;
+    if (s.jump && (nr & s.rmask) == 0) return (i64)(nr >> s.rsh) * s.jump;
+    return 0;
+  };
+  P.step_in = P.fuse_in ? step(p.sin, P.st[0].nr) : 0;
+  P.step_out = P.fuse_out ? step(p.sout, P.st[p.nstage - 1].nr) : 0;
   const long long all = fft_pass_tiles(p);
   if (p.nblocks <= 0) {  // the whole pass
     P.p.nblocks = all;

@@ -29,22 +29,14 @@ using namespace fftdev;
 struct Pass {
   FftLaunch p;
   StageInfo st[kMaxStages];
-  unsigned long long m_n, m_t;  // magics for N and T
+  unsigned m_n, m_t;  // magics for N and T
+  i64 step_in, step_out;         // offset between the points of a fused stage's butterfly (0: look up each)
   int ls;                        // LDS line stride (complex elements)
   int fuse_in;                   // first stage runs on the loaded registers
   int fuse_out;                  // last stage stores straight from registers
   int xcd_pair;                  // tiles sharing 128-byte rows, run back to back on one XCD
   int tw_lds;                    // twiddle table copied to LDS
 };
-
-template <typename R, bool INV, int RADIX, int CAP, int NTH, bool CT, typename TW>
-__device__ __forceinline__ void stage(cx<R> *buf, const Pass &P, int s, TW tw) {
-  stage_lds<R, INV, RADIX, CAP, NTH, CT>(buf, P.st[s], P.p.T, P.ls, tw);
-}
-template <typename R, bool INV, int CAP, int NTH, bool CT, typename TW, typename RT>
-__device__ __forceinline__ void stage_any(cx<R> *buf, const Pass &P, int s, TW tw, RT roots) {
-  stage_lds_any<R, INV, CAP, NTH, CT>(buf, P.st[s], P.p.radix[s], P.p.T, P.ls, tw, roots);
-}
 
 // Per-line address data of one side of a tile (in LDS).
 //   uniform:     base[l] = sum over axes other than t of abs[d][g_d]
@@ -232,8 +224,8 @@ __device__ __forceinline__ void element(const Pass &P, int row, const int *ord, 
 // column walks put consecutive threads on consecutive lines, row walks on
 // consecutive butterflies of a line, so each input/output index r of the
 // butterfly is one coalesced access across the wave.
-__device__ __forceinline__ void butterfly_of(int bi, int row, int nr, unsigned long long m_nr, int T,
-                                             unsigned long long m_t, int &l, int &j) {
+__device__ __forceinline__ void butterfly_of(int bi, int row, int nr, unsigned m_nr, int T,
+                                             unsigned m_t, int &l, int &j) {
   if (row) {
     l = fdiv(bi, m_nr);
     j = bi - l * nr;
@@ -263,8 +255,14 @@ __device__ __forceinline__ void load_first_stage(cx<R> *buf, const Pass &P, cons
     butterfly_of(bc, p.in_row, nr, si.m_nr, p.T, P.m_t, lk[q], jk[q]);
     ok[q] = bi < nb && lk[q] < nl;
     int ls = ok[q] ? lk[q] : 0;
+    if (P.step_in) {
+      const i64 a0 = lin.at(p, p.sin, inT, ls, jk[q]);
 #pragma unroll
-    for (int r = 0; r < RADIX; r++) a[q][r] = lin.at(p, p.sin, inT, ls, jk[q] + r * nr);
+      for (int r = 0; r < RADIX; r++) a[q][r] = a0 + r * P.step_in;
+    } else {
+#pragma unroll
+      for (int r = 0; r < RADIX; r++) a[q][r] = lin.at(p, p.sin, inT, ls, jk[q] + r * nr);
+    }
   }
   cx<R> v[K][RADIX];
   gather<K * RADIX>(&v[0][0], in, &a[0][0], p.stream_in);
@@ -275,9 +273,10 @@ __device__ __forceinline__ void load_first_stage(cx<R> *buf, const Pass &P, cons
       for (int r = 0; r < RADIX; r++) v[q][r] = {0, 0};
     dft<R, INV, RADIX>(v[q]);
     if (threadIdx.x + q * NTH < nb) {
-      int base = lk[q] * P.ls, idxd = jk[q] * RADIX;
+      // (a power-of-two butterfly's outputs do not straddle a pad)
+      cx<R> *to = buf + lk[q] * P.ls + lds_pad(jk[q] * RADIX);
 #pragma unroll
-      for (int r = 0; r < RADIX; r++) buf[base + lds_pad(idxd + r)] = v[q][r];
+      for (int r = 0; r < RADIX; r++) to[r] = v[q][r];
     }
   }
 }
@@ -298,6 +297,13 @@ __device__ __forceinline__ void last_stage_store(const cx<R> *buf, const Pass &P
   cx<R> v[K][RADIX];
   i64 a[K][RADIX];
   bool ok[K];
+  // (AFF: known when compiled, so that no branch sits between the twiddle
+  // products and the stores)
+  const bool even = UOUT && CT ? AFF : P.step_out != 0;
+  auto lout_form = [&](const FftSide &s, const i64 *tab, int l, int x) -> i64 {
+    if constexpr (UOUT && CT) return lout.template at_form<AFF>(s, tab, l, x);
+    else return 0;
+  };
 #pragma unroll
   for (int q = 0; q < K; q++) {
     int bi = threadIdx.x + q * NTH;
@@ -306,20 +312,30 @@ __device__ __forceinline__ void last_stage_store(const cx<R> *buf, const Pass &P
     butterfly_of(bc, p.out_row, nr, si.m_nr, p.T, P.m_t, l, j);
     ok[q] = bi < nb && l < nl;
     int base = l * P.ls;
+    if (si.rs) {
+      const cx<R> *from = buf + base + lds_pad(j);
 #pragma unroll
-    for (int r = 0; r < RADIX; r++) v[q][r] = buf[base + lds_pad(j + r * nr)];
+      for (int r = 0; r < RADIX; r++) v[q][r] = from[r * si.rs];
+    } else {
+#pragma unroll
+      for (int r = 0; r < RADIX; r++) v[q][r] = buf[base + lds_pad(j + r * nr)];
+    }
     // in the last stage ns = nr, so j % ns = j (stage-ordered table)
 #pragma unroll
     for (int r = 1; r < RADIX; r++) v[q][r] = twmul<INV, CT>(v[q][r], tw, (nr - 1) + (r - 1) * nr + j);
     dft<R, INV, RADIX>(v[q]);
     int ls = ok[q] ? l : 0;
+    if (even) {
+      // evenly stepped: an address pair for the butterfly, formed after it
+      const i64 a0 = UOUT && CT ? lout_form(p.sout, outT, ls, j) : lout.at(p, p.sout, outT, ls, j);
+      if (ok[q]) store_steps<RADIX>(out + a0, P.step_out, v[q], p.stream_out);
+    } else {
 #pragma unroll
-    for (int r = 0; r < RADIX; r++) {
-      if constexpr (UOUT && CT) a[q][r] = lout.template at_form<AFF>(p.sout, outT, ls, j + r * nr);
-      else a[q][r] = lout.at(p, p.sout, outT, ls, j + r * nr);
+      for (int r = 0; r < RADIX; r++)
+        a[q][r] = UOUT && CT ? lout_form(p.sout, outT, ls, j + r * nr) : lout.at(p, p.sout, outT, ls, j + r * nr);
     }
   }
-  scatter<K * RADIX, RADIX>(out, &a[0][0], &v[0][0], ok, p.stream_out);
+  if (!even) scatter<K * RADIX, RADIX>(out, &a[0][0], &v[0][0], ok, p.stream_out);
 }
 
 // One tile per workgroup.  Loads and stores run in three branch-free
@@ -422,24 +438,29 @@ __global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 4) vo
     // device table, p per such stage in stage order (the first stage is
     // never one when s0 = 1: the fused first stage is a power of two)
     int roff = p.N;
+    const int ls = P.ls;
     for (int s = s0; s < s1; s++) {
-      switch (p.radix[s]) {
-        case 2: stage<R, INV, 2, CAP, NTH, CT>(buf, P, s, tw); break;
-        case 3: if constexpr (!POW2) stage<R, INV, 3, CAP, NTH, CT>(buf, P, s, tw); break;
-        case 4: stage<R, INV, 4, CAP, NTH, CT>(buf, P, s, tw); break;
-        case 5: if constexpr (!POW2) stage<R, INV, 5, CAP, NTH, CT>(buf, P, s, tw); break;
-        case 7: if constexpr (!POW2) stage<R, INV, 7, CAP, NTH, CT>(buf, P, s, tw); break;
-        case 8: stage<R, INV, 8, CAP, NTH, CT>(buf, P, s, tw); break;
-        case 11: if constexpr (!POW2) stage<R, INV, 11, CAP, NTH, CT>(buf, P, s, tw); break;
-        case 13: if constexpr (!POW2) stage<R, INV, 13, CAP, NTH, CT>(buf, P, s, tw); break;
-        case 16: stage<R, INV, 16, CAP, NTH, CT>(buf, P, s, tw); break;
+      // (copies: with every stage form referring to the kernel arguments the
+      // compiler keeps them in scratch)
+      const StageInfo si = P.st[s];
+      const int radix = p.radix[s];
+      switch (radix) {
+        case 2: stage_lds<R, INV, 2, CAP, NTH, CT>(buf, si, T, ls, tw); break;
+        case 3: if constexpr (!POW2) stage_lds<R, INV, 3, CAP, NTH, CT>(buf, si, T, ls, tw); break;
+        case 4: stage_lds<R, INV, 4, CAP, NTH, CT>(buf, si, T, ls, tw); break;
+        case 5: if constexpr (!POW2) stage_lds<R, INV, 5, CAP, NTH, CT>(buf, si, T, ls, tw); break;
+        case 7: if constexpr (!POW2) stage_lds<R, INV, 7, CAP, NTH, CT>(buf, si, T, ls, tw); break;
+        case 8: stage_lds<R, INV, 8, CAP, NTH, CT>(buf, si, T, ls, tw); break;
+        case 11: if constexpr (!POW2) stage_lds<R, INV, 11, CAP, NTH, CT>(buf, si, T, ls, tw); break;
+        case 13: if constexpr (!POW2) stage_lds<R, INV, 13, CAP, NTH, CT>(buf, si, T, ls, tw); break;
+        case 16: stage_lds<R, INV, 16, CAP, NTH, CT>(buf, si, T, ls, tw); break;
         default:
           if constexpr (ANY) {
             if constexpr (sizeof(R) == 4 && !CT)
-              stage_any<R, INV, CAP, NTH, CT>(buf, P, s, tw, tw_hi{reinterpret_cast<const cx<R> *>(twg)} + roff);
+              stage_lds_any<R, INV, CAP, NTH, CT>(buf, si, radix, T, ls, tw, tw_hi{reinterpret_cast<const cx<R> *>(twg)} + roff);
             else
-              stage_any<R, INV, CAP, NTH, CT>(buf, P, s, tw, twg + roff);
-            roff += p.radix[s];
+              stage_lds_any<R, INV, CAP, NTH, CT>(buf, si, radix, T, ls, tw, twg + roff);
+            roff += radix;
           }
           break;
       }
@@ -488,8 +509,6 @@ __global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 4) vo
     scatter<V, 1>(out, a, w, ok, p.stream_out);
   }
 }
-
-inline unsigned long long magic_for(int d) { return (0x100000000ULL / (unsigned long long)d) + 1ULL; }
 
 // Big tiles: 8 lines of 512 complex doubles on 512 threads (two such
 // workgroups share a CU), 16 lines of 512 complex floats on 1024 threads.

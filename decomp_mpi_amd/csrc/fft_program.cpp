@@ -532,7 +532,7 @@ bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int 
   const int nd = I.h.ndim;
   int T;
   const int u = block_lines(I, axes, dbl, &T);
-  auto magic = [](int d) { return (0x100000000ULL / (unsigned long long)d) + 1ULL; };
+  auto magic = [](int d) { return magic_for(d); };
   // the tile's dimensions, innermost first: by the input's strides
   std::vector<int> dims = axes;
   if (u >= 0) dims.push_back(u);

@@ -49,13 +49,25 @@ constexpr int kReshapePairs = 512;  // (a position, b position) pairs of a side 
 // Launchers return 0 or the HIP error code of the launch (hipError_t).
 int launch_reshape(const ReshapeLaunch &p, void *stream);
 
+// Divisor d as the kernels' fdiv takes it.
+inline unsigned magic_for(int d) { return 0x80000000u / (unsigned)d + 1u; }
+
 // Stage s of a line of N points: nr = N / radix butterflies per line, ns =
 // product of the earlier radices (Stockham span), magics for both.
+// rs, ws: LDS step between a butterfly's inputs and between its outputs where
+// that is one number (nr, ns a multiple of 16: the pad of one element in 16
+// grows evenly), else 0; ws -1: ns 8, outputs of an even radix 8 apart with a
+// pad after every second.
 struct StageInfo {
-  unsigned long long m_nr;   // magic for N / radix
-  unsigned long long m_ns;   // magic for Ns
+  unsigned m_nr;   // magic for N / radix
+  unsigned m_ns;   // magic for Ns
   int nr, ns;
+  int rs, ws;
 };
+inline void stage_steps(StageInfo *s) {
+  s->rs = s->nr % 16 == 0 ? s->nr + s->nr / 16 : 0;
+  s->ws = s->ns % 16 == 0 ? s->ns + s->ns / 16 : (s->ns == 8 ? -1 : 0);
+}
 
 // ---- K2: batched 1D FFT pass -----------------------------------------------
 // Lines along axis t of an ndim array.  With equal strides on every rank
@@ -156,12 +168,12 @@ int fft_line_positions();
 #define DM_BLOCK_DIMS 4
 constexpr int kBlockStages = 10;
 struct BlockDim {
-  unsigned long long m_n;      // magic for n
+  unsigned m_n;      // magic for n
   int n;                       // points (lines per tile)
   int at;                      // first entry in the offset tables
 };
 struct BlockStage {
-  unsigned long long m_s, m_nr, m_ns;
+  unsigned m_s, m_nr, m_ns;
   int dim, radix;
   int s;                       // the dimension's stride in the tile
   int span;                    // s times its points
@@ -247,7 +259,7 @@ struct BatchPlane {
 struct BatchSched {
   int N, T, nstage, tw_off;    // tw_off: start of the stage-ordered roots
   int radix[16];
-  unsigned long long m_n, m_t;
+  unsigned m_n, m_t;
   StageInfo st[16];
 };
 // A segment: the pass over one axis of one transform, described by its
