@@ -221,19 +221,7 @@ struct dm_split_ext {
   bool custom_out = false;  // out is the caller's (dm_split_set_output)
   int ctw = 1;              // complex float: compensated twiddle products
   dm_phased_program ph;
-  std::vector<hipEvent_t> events;  // timing events, made once (a 16^3 call 21.7 us, 23.4 with them made per call)
 };
-
-// The plan's first n timing events (null where one cannot be made).
-static hipEvent_t *plan_events(SplitPlan plan, size_t n) {
-  std::vector<hipEvent_t> &ev = plan->ext->events;
-  while (ev.size() < n) {
-    hipEvent_t e = nullptr;
-    (void)hipEventCreate(&e);
-    ev.push_back(e);
-  }
-  return ev.data();
-}
 
 static void program_release(dm_fft_program &p) {
   if (p.mem) dm::device_free(p.mem);
@@ -913,8 +901,11 @@ static void run_phased(SplitPlan plan, int direction) {
   char *w1 = w0 + (size_t)plan->extent * es;
   ReshapePlan a_to_b = plan->A_to_B ? plan->A_to_B : ph.a_to_b;
   ReshapePlan b_to_a = plan->B_to_A ? plan->B_to_A : ph.b_to_a;
-  hipEvent_t *ev = timed ? plan_events(plan, 2) : nullptr;
-  hipEvent_t e0 = timed ? ev[0] : nullptr, e1 = timed ? ev[1] : nullptr;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (timed) {
+    (void)hipEventCreate(&e0);
+    (void)hipEventCreate(&e1);
+  }
   bool ok = true;
   double total = 0;
   auto phase = [&](int timer, const std::function<bool()> &work) {
@@ -961,7 +952,11 @@ static void run_phased(SplitPlan plan, int direction) {
     phase(FFT_1, passes(ph.st1_bwd));
     phase(RESHAPE_1, [&]() { return dm::enqueue_reshape(plan->comm, plan->A_to_start, st1_buf, plan->src, s); });
   }
-  if (timed) plan->times[ALL] += total;
+  if (timed) {
+    plan->times[ALL] += total;
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+  }
 }
 
 // ---------------------------------------------------------------- planner
@@ -1342,8 +1337,12 @@ static void run_program(SplitPlan plan, dm_fft_program &prog, int t_first, int t
   void *s = dm::world_stream(w);
   size_t n = prog.passes.size();
   bool timed = !w->async;
-  hipEvent_t *ev = timed ? plan_events(plan, n + 1) : nullptr;
-  if (timed) (void)hipEventRecord(ev[0], (hipStream_t)s);
+  std::vector<hipEvent_t> ev;
+  if (timed) {
+    ev.resize(n + 1);
+    for (auto &e : ev) (void)hipEventCreate(&e);
+    (void)hipEventRecord(ev[0], (hipStream_t)s);
+  }
   bool ok = true;
   for (size_t i = 0; i < n && ok; i++) {
     ok = launch_pass(plan->comm, prog, i, s);
@@ -1352,6 +1351,7 @@ static void run_program(SplitPlan plan, dm_fft_program &prog, int t_first, int t
   if (!timed) return;
   if (!ok) {
     (void)hipStreamSynchronize((hipStream_t)s);
+    for (auto &e : ev) (void)hipEventDestroy(e);
     return;
   }
   (void)hipEventSynchronize(ev[n]);
@@ -1363,6 +1363,7 @@ static void run_program(SplitPlan plan, dm_fft_program &prog, int t_first, int t
     total += ms * 1e-3;
   }
   plan->times[ALL] += total;
+  for (auto &e : ev) (void)hipEventDestroy(e);
 }
 
 // split_fft.c:622-744.  Forward: start layout in dat -> output layout in
@@ -1500,8 +1501,6 @@ extern "C" void freeSplitPlan(SplitPlan plan) {
     program_release(plan->ext->fwd);
     program_release(plan->ext->bwd);
     phased_release(plan->ext->ph);
-    for (hipEvent_t e : plan->ext->events)
-      if (e) (void)hipEventDestroy(e);
     delete plan->ext;
   }
   freeDecomp(plan->B_flipped);
