@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <new>
 #include <numeric>
 
 #include "logger.h"
@@ -132,10 +133,23 @@ bool axis_supported(int n, int dbl, std::string *why) {
   return false;
 }
 
+size_t TableBuilder::space(size_t bytes) {
+  const size_t at = host.n, need = at + ((bytes + 255) & ~(size_t)255);
+  if (need > host.cap) {
+    const size_t cap = std::max(need, host.cap + host.cap / 2);
+    char *p = (char *)realloc(host.p, cap);
+    if (p == nullptr) throw std::bad_alloc();
+    host.p = p;
+    host.cap = cap;
+  }
+  memset(host.p + at + bytes, 0, need - at - bytes);
+  host.n = need;
+  return at;
+}
+
 size_t TableBuilder::put(const void *src, size_t bytes) {
-  size_t at = host.size();
-  host.resize(at + ((bytes + 255) & ~(size_t)255), 0);
-  memcpy(&host[at], src, bytes);
+  const size_t at = space(bytes);
+  memcpy(host.p + at, src, bytes);
   return at;
 }
 
@@ -337,7 +351,6 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     const long long nlines = (long long)L.tiles_u * batch * L.T;
     const size_t wi = I.h.uniform ? 1 : 2 * pos_in.size(), wo = U.h.uniform ? 1 : 2 * pos_out.size();
     if (L.merge_k == 1 && ((I.h.uniform && U.h.uniform && nlines * 16 <= (64LL << 20)) || np_most > fft_line_positions())) {
-      std::vector<i64> bi(nlines * wi), bo(nlines * wo);
       const std::vector<int> *ou = nullptr;
       if (pp->ord_u >= 0) ou = &((out_row ? I : U).order[u]);
       std::vector<int> g(nd, 0);
@@ -361,11 +374,12 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
       std::vector<int> cu(nu, 0);
       for (int l = 0; l < nu && u >= 0; l++)
         if (l < I.h.L[u]) cu[l] = ou ? (*ou)[l] : l;
-      auto fill = [&](const Side &s, const std::vector<int> &pos, size_t w, std::vector<i64> &to) {
+      auto fill = [&](const Side &s, const std::vector<int> &pos, size_t w) {
+        const size_t where = tb.space(nlines * w * sizeof(i64));
         std::vector<i64> au(nu, 0);
         for (int l = 0; l < nu && u >= 0; l++) au[l] = s.abs[u][cu[l]];
         std::fill(g.begin(), g.end(), 0);
-        i64 *at = to.data();
+        i64 *at = (i64 *)(tb.host.data() + where);
         for (long long b = 0; b < batch; b++) {
           if (s.h.uniform) {
             i64 base = 0;
@@ -384,11 +398,10 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
             g[d] = 0;
           }
         }
+        return (long)where;
       };
-      fill(I, pos_in, wi, bi);
-      fill(U, pos_out, wo, bo);
-      pp->line_in = (long)tb.put(bi.data(), bi.size() * sizeof(i64));
-      pp->line_out = (long)tb.put(bo.data(), bo.size() * sizeof(i64));
+      pp->line_in = fill(I, pos_in, wi);
+      pp->line_out = fill(U, pos_out, wo);
     }
   }
   // Twiddles in stage order: stage s (Ns = product of the earlier radices,
@@ -637,18 +650,21 @@ bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int 
   B.tiles = nbatch * B.tiles_u;
   const int nu = B.tiles_u * T;
   auto fill = [&](const Side &s) {
-    std::vector<i64> to((size_t)nbatch * nu);
+    const size_t where = tb.space((size_t)nbatch * nu * sizeof(i64));
+    i64 *to = (i64 *)(tb.host.data() + where);
     std::vector<int> g(nd, 0);
+    std::vector<i64> along(nu, 0);
+    for (int l = 0; l < nu && u >= 0; l++) along[l] = s.abs[u][l < B.lines ? I.order[u][l] : 0];
     for (long long b = 0; b < nbatch; b++) {
       i64 base = 0;
       for (int d : batch) base += s.abs[d][g[d]];
-      for (int l = 0; l < nu; l++) to[b * nu + l] = base + (u < 0 ? 0 : s.abs[u][l < B.lines ? I.order[u][l] : 0]);
+      for (int l = 0; l < nu; l++) to[b * nu + l] = base + along[l];
       for (size_t k = batch.size(); k-- > 0;) {
         if (++g[batch[k]] < s.h.L[batch[k]]) break;
         g[batch[k]] = 0;
       }
     }
-    return tb.put(to.data(), to.size() * sizeof(i64));
+    return where;
   };
   pb->base_in = fill(I);
   pb->base_out = fill(U);

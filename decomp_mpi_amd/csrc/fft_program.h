@@ -1,6 +1,7 @@
 // Building FFT pass programs from layouts (shared by the split plan, the
 // per-axis FFT and the batched transforms).
 #pragma once
+#include <cstdlib>
 #include <string>
 #include <vector>
 
@@ -34,7 +35,21 @@ void twiddle_image(const double *w, size_t n, int dbl, void *dst);
 
 // Host image of the device tables of a program.
 struct TableBuilder {
-  std::vector<char> host;
+  // Grown by realloc and not cleared: the line bases of a 512^3 program are
+  // tens of megabytes.
+  struct Image {
+    char *p = nullptr;
+    size_t n = 0, cap = 0;
+    Image() = default;
+    Image(const Image &) = delete;
+    Image &operator=(const Image &) = delete;
+    ~Image() { free(p); }
+    char *data() const { return p; }
+    size_t size() const { return n; }
+    bool empty() const { return n == 0; }
+  } host;
+  // Space for bytes at a 256-byte boundary: its offset.
+  size_t space(size_t bytes);
   size_t put(const void *src, size_t bytes);
 };
 

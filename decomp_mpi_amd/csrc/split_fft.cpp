@@ -681,12 +681,12 @@ static bool compile_plan(SplitPlan plan, bool inverse) {
 // split, so that a tile's lines can run along a whole other axis (long
 // contiguous rows, many lines per tile).  Fastest axis first.
 static bool compile_stage(SplitPlan plan, const dm::HostLayout &h, std::vector<int> axes, bool stage1,
-                          bool inverse, void *buf, i64 slot, dm_fft_program *prog) {
+                          void *buf, i64 slot, dm_fft_program *prog) {
   dm_split_ext *x = plan->ext;
   prog->passes.clear();
   prog->blocks.clear();
   prog->mem = nullptr;
-  prog->inverse = inverse ? 1 : 0;
+  prog->inverse = 0;
   if (axes.empty()) return true;
   std::stable_sort(axes.begin(), axes.end(), [&](int a, int b) { return h.m[a] < h.m[b]; });
   dm::TableBuilder tb;
@@ -707,7 +707,7 @@ static bool compile_stage(SplitPlan plan, const dm::HostLayout &h, std::vector<i
       dm::Side side = dm::make_side(sh, slot);
       if (!dm::block_fits(side, side, subs, x->dbl)) continue;
       dm::PendingBlock b;
-      if (!dm::plan_block(side, side, subs, x->dbl, inverse, buf, buf, tb, &b, x->ctw)) continue;
+      if (!dm::plan_block(side, side, subs, x->dbl, false, buf, buf, tb, &b, x->ctw)) continue;
       pb.push_back(b);
       dm::PendingPass p;
       memset(&p.L, 0, sizeof p.L);
@@ -731,10 +731,23 @@ static bool compile_stage(SplitPlan plan, const dm::HostLayout &h, std::vector<i
     dm::Side side = dm::make_side(sh, slot);
     const int sub = stage1 ? 2 * d + 1 : 2 * d;
     pp.emplace_back();
-    if (!dm::plan_pass(plan->comm, side, side, sub, x->dbl, inverse, buf, buf, tb, &pp.back(), x->ctw)) return false;
+    if (!dm::plan_pass(plan->comm, side, side, sub, x->dbl, false, buf, buf, tb, &pp.back(), x->ctw)) return false;
   }
   prog->mem = dm::finalize_passes(plan->comm, tb, pp, &prog->passes, &pb, &prog->blocks);
   return prog->mem != nullptr;
+}
+
+// The backward of a stage: the same passes in place, on the same tables (the
+// forward's), with the inverse transform.  Nothing but the flag differs, and
+// a second set of line bases was most of a plan's first call (512^3 in phase
+// order, both directions: 106 ms with both sets built and tables cleared and
+// copied once more on the way, 32 ms so).
+static void inverse_of(const dm_fft_program &fwd, dm_fft_program *bwd) {
+  *bwd = fwd;
+  bwd->mem = nullptr;
+  bwd->inverse = 1;
+  for (auto &L : bwd->passes) L.inverse = 1;
+  for (auto &B : bwd->blocks) B.inverse = 1;
 }
 
 static bool compile_phased(SplitPlan plan) {
@@ -759,15 +772,13 @@ static bool compile_phased(SplitPlan plan) {
     if (x->A[d] > 1) y_axes.push_back(d);
   }
   void *st1_buf = two ? w1 : w0;
-  if (!compile_stage(plan, hA, z_axes, true, false, st1_buf, wslot, &ph.st1_fwd) ||
-      !compile_stage(plan, hA, z_axes, true, true, st1_buf, wslot, &ph.st1_bwd))
-    return false;
+  if (!compile_stage(plan, hA, z_axes, true, st1_buf, wslot, &ph.st1_fwd)) return false;
+  inverse_of(ph.st1_fwd, &ph.st1_bwd);
   if (two) {
     dm::HostLayout hB = dm::layout_from_decomp(plan->B);
     if (!dm::layout_usable(comm, "B", hB, (size_t)plan->extent)) return false;
-    if (!compile_stage(plan, hB, y_axes, false, false, w0, wslot, &ph.st2_fwd) ||
-        !compile_stage(plan, hB, y_axes, false, true, w0, wslot, &ph.st2_bwd))
-      return false;
+    if (!compile_stage(plan, hB, y_axes, false, w0, wslot, &ph.st2_fwd)) return false;
+    inverse_of(ph.st2_fwd, &ph.st2_bwd);
     if (plan->A_to_B == nullptr) {  // single second stage: the reference has no A -> B plan
       MPI_Datatype base = x->dbl ? &dm_type_c_double_complex : &dm_type_c_float_complex;
       ph.a_to_b = makeReshapePlan(comm, base, plan->A, plan->B);
@@ -828,6 +839,7 @@ static bool compile_phased(SplitPlan plan) {
     // reference's recursion forms it
     std::vector<double> rows_tab;
     std::vector<long long> row_off(nr, 0);
+    rows_tab.reserve(2 * (size_t)max_elems);
     for (int r = 0; r < nr; r++) {
       long long rows = 1;
       for (int d = 0; d < nd - 1; d++) rows *= rt[((size_t)r * nd + d) * 2 + 1];
