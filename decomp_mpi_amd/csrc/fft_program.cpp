@@ -206,6 +206,22 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   };
   const std::vector<int> pos_in = positions(I), pos_out = positions(U);
   const int np_most = (int)std::max(std::max(pos_in.size(), pos_out.size()), (size_t)1);
+  // Small arrays: lines per tile are halved while a pass has fewer than 192
+  // tiles for the 256 CUs and rows of 64 bytes stay.  What is left to win
+  // there is the latency of one tile, which falls with its points per thread
+  // (64^3 complex double over pencils 22.0 -> 20.1 us a transform, 61x21x100
+  // on 12 ranks 182 -> 104, 75x200 on 6 62 -> 43).  At 256 tiles
+  // 2940x576 lost (145 -> 153 us: rows of half the width for nothing, all
+  // CUs were busy); at 512 and 1024 arrays of a million points did (71 -> 87
+  // and 105 us for 256x208x72).
+  long long lines = 1;
+  for (int d = 0; d < nd; d++)
+    if (d != t) lines *= I.h.L[d];
+  auto spread = [&](int T) {
+    const int least = 64 / (dbl ? 16 : 8);
+    while (T > least && lines / T < 192) T = (T + 1) / 2;
+    return T;
+  };
   if (u >= 0) {
     // column walk at a line stride of 64 KiB or more: wide rows pay for the
     // lower occupancy of the wide tile -- for lines of 256 points or more
@@ -216,7 +232,7 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
                                (!out_row && (size_t)U.h.m[t] * es >= (64u << 10)));
     static const bool nowide = getenv("DM_NO_WIDE") != nullptr;
     int tcap = fft_tile_capacity(dbl, !(in_row && out_row), wide && !nowide);
-    L.T = std::max(1, std::min(std::min(tcap / L.N, I.h.L[u]), 512));
+    L.T = spread(std::max(1, std::min(std::min(tcap / L.N, I.h.L[u]), 512)));
     // per-line address data of a non-uniform side: 16 KiB of LDS at most
     // (a side with more positions than that reads its line table)
     if (np_most > 1) L.T = std::max(1, std::min(L.T, fft_line_positions() / np_most));
@@ -249,7 +265,7 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   L.merge_v = -1;
   L.merge_k = 1;
   if (u >= 0 && L.nbatch > 0 && in_row && out_row) {
-    const int per = std::min(fft_tile_capacity(dbl, 0) / L.N, 512);
+    const int per = spread(std::min(fft_tile_capacity(dbl, 0) / L.N, 512));
     const int lu = I.h.L[u];
     const int v = L.batch_axis[L.nbatch - 1];
     if (2 * lu <= per && np_most == 1) {
