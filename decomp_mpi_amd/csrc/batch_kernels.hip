@@ -254,15 +254,15 @@ __global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 4) vo
       int roff = N;
       for (int s = s0; s < s1; s++) {
         switch (S.radix[s]) {
-          case 2: stage_lds<R, INV, 2, CAP, NTH, CT>(buf, S.st[s], T, ls, tw); break;
-          case 3: stage_lds<R, INV, 3, CAP, NTH, CT>(buf, S.st[s], T, ls, tw); break;
-          case 4: stage_lds<R, INV, 4, CAP, NTH, CT>(buf, S.st[s], T, ls, tw); break;
-          case 5: if constexpr (PRIMES) stage_lds<R, INV, 5, CAP, NTH, CT>(buf, S.st[s], T, ls, tw); break;
-          case 7: if constexpr (PRIMES) stage_lds<R, INV, 7, CAP, NTH, CT>(buf, S.st[s], T, ls, tw); break;
-          case 8: stage_lds<R, INV, 8, CAP, NTH, CT>(buf, S.st[s], T, ls, tw); break;
-          case 11: if constexpr (PRIMES) stage_lds<R, INV, 11, CAP, NTH, CT>(buf, S.st[s], T, ls, tw); break;
-          case 13: if constexpr (PRIMES) stage_lds<R, INV, 13, CAP, NTH, CT>(buf, S.st[s], T, ls, tw); break;
-          case 16: stage_lds<R, INV, 16, CAP, NTH, CT>(buf, S.st[s], T, ls, tw); break;
+          case 2: stage_lds<R, INV, 2, CAP, NTH, CT, false>(buf, S.st[s], T, ls, tw); break;
+          case 3: stage_lds<R, INV, 3, CAP, NTH, CT, false>(buf, S.st[s], T, ls, tw); break;
+          case 4: stage_lds<R, INV, 4, CAP, NTH, CT, false>(buf, S.st[s], T, ls, tw); break;
+          case 5: if constexpr (PRIMES) stage_lds<R, INV, 5, CAP, NTH, CT, false>(buf, S.st[s], T, ls, tw); break;
+          case 7: if constexpr (PRIMES) stage_lds<R, INV, 7, CAP, NTH, CT, false>(buf, S.st[s], T, ls, tw); break;
+          case 8: stage_lds<R, INV, 8, CAP, NTH, CT, false>(buf, S.st[s], T, ls, tw); break;
+          case 11: if constexpr (PRIMES) stage_lds<R, INV, 11, CAP, NTH, CT, false>(buf, S.st[s], T, ls, tw); break;
+          case 13: if constexpr (PRIMES) stage_lds<R, INV, 13, CAP, NTH, CT, false>(buf, S.st[s], T, ls, tw); break;
+          case 16: stage_lds<R, INV, 16, CAP, NTH, CT, false>(buf, S.st[s], T, ls, tw); break;
           default:
             if constexpr (ANY) {
               stage_lds_any<R, INV, CAP, NTH, CT>(buf, S.st[s], S.radix[s], T, ls, tw, twall + S.tw_off + roff);

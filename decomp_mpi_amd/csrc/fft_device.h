@@ -264,7 +264,10 @@ __device__ __forceinline__ int lds_index(int line, int x, int ls) { return line 
 // TW: pointer to the twiddles, typed by where they live (an LDS-qualified
 // pointer reads with LDS instructions; a generic one would use flat loads);
 // CT: compensated twiddle products (complex float).
-template <typename R, bool INV, int RADIX, int CAP, int NTH, bool CT, typename TW>
+// STEPS: the evenly stepped LDS addresses of StageInfo::rs and ws.  The
+// batched line kernel goes without: the second form of each loop cost
+// 1-2% there (103 complex-float 3D transforms 278 us with it, 274 without).
+template <typename R, bool INV, int RADIX, int CAP, int NTH, bool CT, bool STEPS = true, typename TW>
 __device__ __forceinline__ void stage_lds(cx<R> *buf, const StageInfo &si, int T, int ls, TW tw) {
   constexpr int K = (CAP / RADIX + NTH - 1) / NTH;
   const int nr = si.nr, ns = si.ns;
@@ -281,7 +284,7 @@ __device__ __forceinline__ void stage_lds(cx<R> *buf, const StageInfo &si, int T
       int j = b - l * nr;
       int jn = fdiv(j, si.m_ns);
       int jj = j - jn * ns;
-      if (si.rs) {
+      if (STEPS && si.rs) {
         const cx<R> *from = buf + at(l, j);
 #pragma unroll
         for (int r = 0; r < RADIX; r++) v[k][r] = from[r * si.rs];
@@ -306,11 +309,11 @@ __device__ __forceinline__ void stage_lds(cx<R> *buf, const StageInfo &si, int T
   for (int k = 0; k < K; k++) {
     if (dst[k] >= 0) {
       int l = dst[k] >> 16, idxd = dst[k] & 0xffff;
-      if (si.ws > 0) {
+      if (STEPS && si.ws > 0) {
         cx<R> *to = buf + at(l, idxd);
 #pragma unroll
         for (int r = 0; r < RADIX; r++) to[r * si.ws] = v[k][r];
-      } else if (RADIX % 2 == 0 && si.ws < 0) {
+      } else if (STEPS && RADIX % 2 == 0 && si.ws < 0) {
         cx<R> *to = buf + at(l, idxd);
 #pragma unroll
         for (int r = 0; r < RADIX; r++) to[8 * r + r / 2] = v[k][r];
