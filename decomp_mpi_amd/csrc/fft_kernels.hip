@@ -113,6 +113,7 @@ int launch_fft_pass(const FftLaunch &p, void *stream) {
   if (P.p.nblocks <= 0) return 0;
   if (P.p.tile_base < 0 || P.p.tile_base + P.p.nblocks > all) return (int)hipErrorInvalidValue;
   size_t lds = fft_lds_bytes(p);
+  if (lds > kLdsBytes) return (int)hipErrorInvalidValue;
   hipStream_t s = (hipStream_t)stream;
   bool pow2 = true, any = false;
   for (int i = 0; i < p.nstage; i++) {

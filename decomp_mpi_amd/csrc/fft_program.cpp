@@ -205,6 +205,12 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     return v;
   };
   const std::vector<int> pos_in = positions(I), pos_out = positions(U);
+  L.sin.uniform = I.h.uniform ? 1 : 0;
+  L.sin.np = (int)pos_in.size();
+  L.sout.uniform = U.h.uniform ? 1 : 0;
+  L.sout.np = (int)pos_out.size();
+  L.dbl = dbl;
+  L.ctw = (!dbl && ctw) ? 1 : 0;
   const int np_most = (int)std::max(std::max(pos_in.size(), pos_out.size()), (size_t)1);
   // Small arrays: lines per tile are halved while a pass has fewer than 192
   // tiles for the 256 CUs and rows of 64 bytes stay.  What is left to win
@@ -231,11 +237,16 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     bool wide = L.N >= 256 && ((!in_row && (size_t)I.h.m[t] * es >= (64u << 10)) ||
                                (!out_row && (size_t)U.h.m[t] * es >= (64u << 10)));
     static const bool nowide = getenv("DM_NO_WIDE") != nullptr;
-    int tcap = fft_tile_capacity(dbl, !(in_row && out_row), wide && !nowide);
-    L.T = spread(std::max(1, std::min(std::min(tcap / L.N, I.h.L[u]), 512)));
-    // per-line address data of a non-uniform side: 16 KiB of LDS at most
-    // (a side with more positions than that reads its line table)
-    if (np_most > 1) L.T = std::max(1, std::min(L.T, fft_line_positions() / np_most));
+    auto height = [&](bool w) {
+      const int T = spread(std::max(1, std::min(std::min(fft_tile_capacity(dbl, !(in_row && out_row), w) / L.N, I.h.L[u]), 512)));
+      // per-line address data of a non-uniform side: 16 KiB of LDS at most
+      // (a side with more positions than that reads its line table)
+      return np_most > 1 ? std::max(1, std::min(T, fft_line_positions() / np_most)) : T;
+    };
+    L.T = height(wide && !nowide);
+    // the wide tile (136 KiB and up to 16 of twiddles) leaves no room for the
+    // line data of many positions; the other tiles do: at most 118 KiB in all
+    if (fft_lds_bytes(L) > kLdsBytes) L.T = height(false);
     L.tiles_u = (I.h.L[u] + L.T - 1) / L.T;
   } else {
     L.T = 1;
@@ -287,8 +298,6 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     return false;
   }
   L.inverse = inverse ? 1 : 0;
-  L.dbl = dbl;
-  L.ctw = (!dbl && ctw) ? 1 : 0;
   // per-axis tables one after another
   for (int d = 1; d < nd; d++) L.at[d] = L.at[d - 1] + L.L[d - 1];
   auto joined = [&](const auto &tab) {
@@ -300,7 +309,6 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   pp->out_off = joined(U.abs);
   // rank-dependent strides: owner, local offset and per-rank stride tables
   auto side = [&](const Side &s, FftSide &fs, PendingSide &ps, const std::vector<int> &pos) {
-    fs.uniform = s.h.uniform ? 1 : 0;
     fs.proc_used = s.h.proc_used;
     fs.slot = s.slot;
     // offsets along t affine (x * m_t: axis t local to every rank, in
@@ -336,7 +344,6 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     }
     if (s.h.uniform) return;
     std::vector<int> xt(2 * (size_t)L.N);
-    fs.np = (int)pos.size();
     fs.lin = fs.np == 1;
     for (int x = 0; x < L.N; x++) {
       xt[2 * (size_t)x] = (int)(std::lower_bound(pos.begin(), pos.end(), s.h.rank_part[t][x]) - pos.begin());

@@ -159,6 +159,10 @@ int launch_fft_pass(const FftLaunch &p, void *stream);
 int fft_tile_capacity(int dbl, int column, int wide = 0);
 // (line, position) entries a non-uniform side of a tile keeps in LDS.
 int fft_line_positions();
+// LDS a workgroup of the pass takes: its tile, the line data of both sides
+// (uniform, np) and the twiddles.  At most kLdsBytes, or the launch is refused.
+constexpr size_t kLdsBytes = 160 * 1024;
+size_t fft_lds_bytes(const FftLaunch &p);
 
 // ---- K5: several whole axes in one pass ------------------------------------
 // A tile holds every point of the transformed dimensions times n lines of

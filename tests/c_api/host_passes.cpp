@@ -1,0 +1,74 @@
+// The FFT pass planner against its kernels' limits, without a GPU: passes
+// are planned from real decompositions through the library's own internal
+// headers, and what the launch would ask for is checked here.
+// Usage: host_passes <check>; prints OK.
+#include <cstdio>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "block_decomp.h"
+#include "fft_program.h"
+
+static int failures = 0;
+
+// Packed blocks of shape over grid.
+struct Layout {
+  MPI_Comm comm;
+  Decomp d;
+  dm::HostLayout h;
+  Layout(const std::vector<int> &shape, const std::vector<int> &grid) {
+    int ranks = 1;
+    for (int g : grid) ranks *= g;
+    comm = dm_world_create(ranks);
+    std::vector<DimDecomp> dims;
+    for (size_t i = 0; i < shape.size(); i++) dims.push_back(makeBlockDecomp(shape[i], grid[i]));
+    d = makePackedDecomp(comm, (int)shape.size(), dims.data());
+    h = dm::layout_from_decomp(d);
+  }
+  ~Layout() {
+    freeDecomp(d);
+    dm_world_free(comm);
+  }
+  dm::Side side() const {
+    i64 most = 1;
+    for (i64 e : h.slot_extent) most = e > most ? e : most;
+    return dm::make_side(h, most);
+  }
+};
+
+// A workgroup's LDS, for every combination of line length, rank positions
+// along the line and uneven sides; the middle axis makes a side uneven, the
+// last axis the line stride (64 KiB or more with 130 points).
+static void lds() {
+  for (int n : {256, 360, 512, 729, 1000, 1024, 2048, 4096})
+    for (int np : {1, 2, 16, 20, 32, 34, 47, 64, 68, 100, 128, 146, 256}) {
+      if (np > n / 2) continue;
+      const Layout even({n, 66, 130}, {1, 2, 1}), uneven({n, 65, 130}, {np, 2, 1}), local({n, 65, 130}, {1, 1, 1});
+      const dm::Side e = local.side(), s = uneven.side();
+      for (int form = 0; form < 3; form++)
+        for (int dbl : {0, 1}) {
+          dm::TableBuilder tb;
+          dm::PendingPass pp;
+          if (!dm::plan_pass(uneven.comm, form == 1 ? e : s, form == 0 ? e : s, 0, dbl, false, nullptr, nullptr, tb, &pp)) {
+            printf("no pass: n %d np %d form %d dbl %d\n", n, np, form, dbl);
+            failures++;
+            continue;
+          }
+          const size_t need = dm::fft_lds_bytes(pp.L);
+          if (need > 160 * 1024 || pp.L.T < 1) {
+            printf("%zu bytes of LDS: n %d np %d form %d dbl %d T %d\n", need, n, np, form, dbl, pp.L.T);
+            failures++;
+          }
+        }
+    }
+}
+
+int main(int argc, char **argv) {
+  dm_set_error_mode(1);
+  const std::string check = argc > 1 ? argv[1] : "";
+  if (check == "lds") lds();
+  else return 2;
+  if (failures == 0) printf("OK\n");
+  return failures != 0;
+}
