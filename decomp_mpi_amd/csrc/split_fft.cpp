@@ -787,8 +787,11 @@ static bool compile_phased(SplitPlan plan) {
     }
   }
   // twiddle tables of every rank position, rows in position order, and the
-  // per-rank (first row, count) table with the A layout's strides
-  ph.has_twiddle = two && plan->twiddle != nullptr;
+  // per-rank (first row, count) table with the A layout's strides.  An axis
+  // with both factors has w != 1 at y = z = 1, on whichever rank holds it
+  // (plan->twiddle is the view rank's own table, NULL where that is all ones).
+  ph.has_twiddle = false;
+  for (int d = 0; d < nd; d++) ph.has_twiddle = ph.has_twiddle || (two && x->A[d] > 1 && x->B[d] > 1);
   if (ph.has_twiddle) {
     std::vector<std::vector<double>> tabs(nd);
     std::vector<std::vector<int>> first(nd);
