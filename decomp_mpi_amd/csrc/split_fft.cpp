@@ -215,7 +215,7 @@ struct dm_split_ext {
   Decomp start = nullptr;   // caller's (aliased)
   Decomp out = nullptr;     // B_flipped, or A for single-stage plans (owned by the plan)
   bool use_first = false;   // single stage: output in the A decomposition
-  dm_fft_program fwd, bwd;  // each built for its first run
+  dm_fft_program fwd, bwd;  // built for the first run of either
   bool phased = false;      // run in the reference's phase order
   bool fused_ok = true;     // every axis fits one pass (else phased only)
   bool custom_out = false;  // out is the caller's (dm_split_set_output)
@@ -637,11 +637,12 @@ static bool bind_buffers(SplitPlan plan, dm::Buffer *bd, size_t *od, dm::Buffer 
   return true;
 }
 
-// Build the fused program of one direction, if it is not there yet.
-static bool compile_plan(SplitPlan plan, bool inverse) {
+// Build the fused programs of both directions, if they are not there yet: a
+// first run in one direction leaves nothing to allocate or copy for the other
+// (which a caller may then record into a graph).
+static bool compile_plan(SplitPlan plan) {
   dm_split_ext *x = plan->ext;
-  dm_fft_program &prog = inverse ? x->bwd : x->fwd;
-  if (prog.mem != nullptr) return true;
+  if (x->fwd.mem != nullptr && x->bwd.mem != nullptr) return true;
   if (!x->fused_ok) {
     raise_error(plan->comm, "split FFT: an axis is longer than one pass tile; this plan runs in phase order only");
     return false;
@@ -658,7 +659,10 @@ static bool compile_plan(SplitPlan plan, bool inverse) {
   char *dat = bd.base + od;
   char *w0 = bw.base + ow;
   char *w1 = w0 + ext * es;
-  if (!compile_direction(plan, inverse, S, O, dat, w0, w1, bw.nranks, &prog)) return false;
+  for (bool inverse : {false, true}) {
+    dm_fft_program &prog = inverse ? x->bwd : x->fwd;
+    if (prog.mem == nullptr && !compile_direction(plan, inverse, S, O, dat, w0, w1, bw.nranks, &prog)) return false;
+  }
   plan->plan_a = &x->fwd;
   plan->plan_b_back = &x->bwd;
   return true;
@@ -1208,7 +1212,7 @@ static double model_cost(SplitPlan p) {
 // Milliseconds of a forward + backward step of plan p (the backward
 // overwrites dat: the caller saves it).
 static double time_plan(SplitPlan p, int reps) {
-  if (p->ext->phased ? !compile_phased(p) : !(compile_plan(p, false) && compile_plan(p, true))) return 1e30;
+  if (p->ext->phased ? !compile_phased(p) : !compile_plan(p)) return 1e30;
   void *s = dm::world_stream(p->comm->world);
   hipEvent_t e0, e1;
   (void)hipEventCreate(&e0);
@@ -1424,7 +1428,7 @@ static void run_split(SplitPlan plan, int direction) {
     if (compile_phased(plan)) run_phased(plan, direction);
     return;
   }
-  if (!compile_plan(plan, direction == FFTW_BACKWARD)) return;
+  if (!compile_plan(plan)) return;
   if (direction == FFTW_FORWARD) run_program(plan, plan->ext->fwd, FFT_1, FFT_2);
   else run_program(plan, plan->ext->bwd, FFT_2, FFT_1);
 }
