@@ -89,38 +89,55 @@ struct LineAddr<true> {
 // reads a point) made such passes latency-bound: the three passes of a 90 x
 // 126 x 100 complex-double transform on 6 ranks took 43, 43 and 25 us, 129
 // us for the whole call; 86 us with a base and a stride per line and
-// position, dense intermediates and two workgroups per CU.
+// position, dense intermediates and two workgroups per CU.  It is left for
+// lines with more positions than LDS is given (np > kLinePositions): LDS
+// holds the line's owner contribution and its local offsets then.
 template <>
 struct LineAddr<false> {
+  static constexpr int kFar = 1 + DM_MAX_DIMS;  // entries a line of the far form
   lds_i64 *base;
   lds_i64 *str;
-  const i64 *tab;  // more positions than LDS is given: the tile's host table
   int np;
   __host__ __device__ static size_t bytes(int T, int np) {
-    return np > kLinePositions ? 0 : (size_t)T * np * 2 * sizeof(i64);
+    return np > kLinePositions ? (size_t)T * kFar * sizeof(i64) : (size_t)T * np * 2 * sizeof(i64);
   }
   __device__ void init(char *mem, int T, int n) {
     base = (lds_i64 *)(mem);
-    str = base + T * n;
-    tab = nullptr;
+    str = base + T * n;  // (not used by the far form)
     np = n;
   }
-  // line l on position q along t (g: the line's coordinates)
-  __device__ void set_line(const FftLaunch &p, const FftSide &s, const int *g, int l, int q) {
-    int R = s.posrank[q];
+  // line l through the coordinates g
+  __device__ void set_line(const FftLaunch &p, const FftSide &s, const int *g, int l) {
+    int R0 = 0;
     for (int d = 0; d < p.ndim; d++)
-      if (d != p.t) R += s.rank[p.at[d] + g[d]];
-    const i64 *m = s.strides + (i64)R * p.ndim;
-    i64 a = (i64)R * s.slot;
-    for (int d = 0; d < p.ndim; d++)
-      if (d != p.t) a += m[d] * s.off[p.at[d] + g[d]];
-    base[l * np + q] = a;
-    str[l * np + q] = m[p.t];
+      if (d != p.t) R0 += s.rank[p.at[d] + g[d]];
+    if (np > kLinePositions) {
+      base[l * kFar] = R0;
+      for (int d = 0; d < p.ndim; d++) base[l * kFar + 1 + d] = d != p.t ? s.off[p.at[d] + g[d]] : 0;
+      return;
+    }
+    for (int q = 0; q < np; q++) {
+      const int R = R0 + s.posrank[q];
+      const i64 *m = s.strides + (i64)R * p.ndim;
+      i64 a = (i64)R * s.slot;
+      for (int d = 0; d < p.ndim; d++)
+        if (d != p.t) a += m[d] * s.off[p.at[d] + g[d]];
+      base[l * np + q] = a;
+      str[l * np + q] = m[p.t];
+    }
   }
-  __device__ __forceinline__ i64 at(const FftLaunch &, const FftSide &s, const i64 *, int l, int x) const {
+  // point x, at its local offset, of line l in the far form
+  __device__ i64 far(const FftLaunch &p, const FftSide &s, int l, int x, int off) const {
+    const int R = (int)base[l * kFar] + s.rank[p.at[p.t] + x];
+    const i64 *m = s.strides + (i64)R * p.ndim;
+    i64 a = (i64)R * s.slot + off * m[p.t];
+    for (int d = 0; d < p.ndim; d++) a += m[d] * base[l * kFar + 1 + d];
+    return a;
+  }
+  __device__ __forceinline__ i64 at(const FftLaunch &p, const FftSide &s, const i64 *, int l, int x) const {
     if (s.lin) return base[l] + (i64)x * str[l];  // axis t local to every rank, in order
+    if (np > kLinePositions) return far(p, s, l, x, s.xt[2 * x + 1]);
     const int k = l * np + s.xt[2 * x];
-    if (np > kLinePositions) return tab[2 * k] + (i64)s.xt[2 * x + 1] * tab[2 * k + 1];
     return base[k] + (i64)s.xt[2 * x + 1] * str[k];
   }
 };
@@ -137,41 +154,15 @@ __device__ __forceinline__ int setup_lines(const FftLaunch &p, long long tile, L
   const int u0 = tu * T;
   const int mk = p.merge_k;
   const int nlines = mk > 1 ? T : (p.u >= 0 ? min(T, p.L[p.u] - u0) : 1);
-  if (p.line_in_tab != nullptr) {  // precomputed line bases
-    // (both sides' loads go out together: one latency)
-    if constexpr (UIN && UOUT) {
+  if constexpr (UIN && UOUT) {
+    if (p.line_in_tab != nullptr) {  // precomputed line bases
+      // (both sides' loads go out together: one latency)
       for (int l = threadIdx.x; l < T; l += NTHR) {
         lin.base[l] = p.line_in_tab[tile * T + l];
         lout.base[l] = p.line_out_tab[tile * T + l];
       }
-    } else {
-      const int ni = UIN ? T : T * lin.np, no = UOUT ? T : T * lout.np;
-      const i64 *ti = p.line_in_tab + tile * (UIN ? ni : 2 * ni);
-      const i64 *to = p.line_out_tab + tile * (UOUT ? no : 2 * no);
-      if constexpr (!UIN) lin.tab = ti;
-      if constexpr (!UOUT) lout.tab = to;
-      for (int k = threadIdx.x; k < max(ni, no); k += NTHR) {
-        const int ki = min(k, ni - 1), ko = min(k, no - 1);
-        i64 bi, bo, si = 0, so = 0;
-        if constexpr (UIN) bi = ti[ki];
-        else bi = ti[2 * ki], si = ti[2 * ki + 1];
-        if constexpr (UOUT) bo = to[ko];
-        else bo = to[2 * ko], so = to[2 * ko + 1];
-        if constexpr (UIN) {
-          if (k < ni) lin.base[k] = bi;
-        } else if (k < ni && lin.np <= kLinePositions) {
-          lin.base[k] = bi;
-          lin.str[k] = si;
-        }
-        if constexpr (UOUT) {
-          if (k < no) lout.base[k] = bo;
-        } else if (k < no && lout.np <= kLinePositions) {
-          lout.base[k] = bo;
-          lout.str[k] = so;
-        }
-      }
+      return nlines;
     }
-    return nlines;
   }
   long long bid = tile / p.tiles_u;
   int gb[DM_MAX_DIMS];
@@ -198,11 +189,9 @@ __device__ __forceinline__ int setup_lines(const FftLaunch &p, long long tile, L
       g[p.u] = (l < nlines) ? (p.ord_u ? p.ord_u[u0 + l] : u0 + l) : 0;
     }
     if constexpr (UIN) lin.set_line(p, p.off_in, g, l);
-    else
-      for (int q = 0; q < lin.np; q++) lin.set_line(p, p.sin, g, l, q);
+    else lin.set_line(p, p.sin, g, l);
     if constexpr (UOUT) lout.set_line(p, p.off_out, g, l);
-    else
-      for (int q = 0; q < lout.np; q++) lout.set_line(p, p.sout, g, l, q);
+    else lout.set_line(p, p.sout, g, l);
   }
   return nlines;
 }

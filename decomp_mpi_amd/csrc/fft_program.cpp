@@ -240,7 +240,8 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     auto height = [&](bool w) {
       const int T = spread(std::max(1, std::min(std::min(fft_tile_capacity(dbl, !(in_row && out_row), w) / L.N, I.h.L[u]), 512)));
       // per-line address data of a non-uniform side: 16 KiB of LDS at most
-      // (a side with more positions than that reads its line table)
+      // (a side with more positions than that forms its addresses point by
+      // point)
       return np_most > 1 ? std::max(1, std::min(T, fft_line_positions() / np_most)) : T;
     };
     L.T = height(wide && !nowide);
@@ -368,53 +369,28 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   // Per-tile line bases for uniform sides: one coalesced load per tile in
   // the kernel instead of a chain of lookups (bounded to 64 MiB of tables).
   // Non-uniform sides form theirs in the kernel (90 x 126 x 100 on 6 ranks:
-  // 86 us against 81 with tables, but 371 against 566 for a first pass),
-  // unless they have more positions than LDS holds.
+  // 86 us against 81 with tables, but 371 against 566 for a first pass).
   {
     const long long nlines = (long long)L.tiles_u * batch * L.T;
-    const size_t wi = I.h.uniform ? 1 : 2 * pos_in.size(), wo = U.h.uniform ? 1 : 2 * pos_out.size();
-    if (L.merge_k == 1 && ((I.h.uniform && U.h.uniform && nlines * 16 <= (64LL << 20)) || np_most > fft_line_positions())) {
+    if (L.merge_k == 1 && I.h.uniform && U.h.uniform && nlines * 16 <= (64LL << 20)) {
       const std::vector<int> *ou = nullptr;
       if (pp->ord_u >= 0) ou = &((out_row ? I : U).order[u]);
-      std::vector<int> g(nd, 0);
-      // the line through g: its base, or its base and stride per position
-      auto put = [&](const Side &s, const std::vector<int> &pos, i64 *to) {
-        int R0 = 0;
-        for (int d = 0; d < nd; d++)
-          if (d != t) R0 += s.h.rank_part[d][g[d]];
-        for (size_t q = 0; q < pos.size(); q++) {
-          const int R = R0 + pos[q];
-          const i64 *m = &s.h.strides[(size_t)R * nd];
-          i64 a = (i64)R * s.slot;
-          for (int d = 0; d < nd; d++)
-            if (d != t) a += m[d] * s.h.off[d][g[d]];
-          to[2 * q] = a;
-          to[2 * q + 1] = m[t];
-        }
-      };
-      // u coordinate of every line of a row of tiles, its offsets in both
+      // u coordinate of every line of a row of tiles
       const int nu = L.tiles_u * L.T;
-      std::vector<int> cu(nu, 0);
+      std::vector<int> cu(nu, 0), g(nd, 0);
       for (int l = 0; l < nu && u >= 0; l++)
         if (l < I.h.L[u]) cu[l] = ou ? (*ou)[l] : l;
-      auto fill = [&](const Side &s, const std::vector<int> &pos, size_t w) {
-        const size_t where = tb.space(nlines * w * sizeof(i64));
+      auto fill = [&](const Side &s) {
+        const size_t where = tb.space(nlines * sizeof(i64));
         std::vector<i64> au(nu, 0);
         for (int l = 0; l < nu && u >= 0; l++) au[l] = s.abs[u][cu[l]];
         std::fill(g.begin(), g.end(), 0);
         i64 *at = (i64 *)(tb.host.data() + where);
         for (long long b = 0; b < batch; b++) {
-          if (s.h.uniform) {
-            i64 base = 0;
-            for (int k = 0; k < L.nbatch; k++) base += s.abs[L.batch_axis[k]][g[L.batch_axis[k]]];
-            for (int l = 0; l < nu; l++) at[l] = base + au[l];
-          } else {
-            for (int l = 0; l < nu; l++) {
-              if (u >= 0) g[u] = cu[l];
-              put(s, pos, at + l * w);
-            }
-          }
-          at += nu * w;
+          i64 base = 0;
+          for (int k = 0; k < L.nbatch; k++) base += s.abs[L.batch_axis[k]][g[L.batch_axis[k]]];
+          for (int l = 0; l < nu; l++) at[l] = base + au[l];
+          at += nu;
           for (int k = L.nbatch - 1; k >= 0; k--) {  // the next batch coordinate
             const int d = L.batch_axis[k];
             if (++g[d] < I.h.L[d]) break;
@@ -423,8 +399,8 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
         }
         return (long)where;
       };
-      pp->line_in = fill(I, pos_in, wi);
-      pp->line_out = fill(U, pos_out, wo);
+      pp->line_in = fill(I);
+      pp->line_out = fill(U);
     }
   }
   // Twiddles in stage order: stage s (Ns = product of the earlier radices,

@@ -119,9 +119,8 @@ struct FftLaunch {
   const int *ord_in;          // row mode: t coordinates in input address order (or null)
   const int *ord_out;         // row mode: t coordinates in output address order (or null)
   const int *ord_u;           // tile line l holds u coordinate ord_u[u0 + l] (or u0 + l)
-  const i64 *line_in_tab;     // base offset of line l of tile b at [b * T + l]; non-uniform sides:
-  const i64 *line_out_tab;    //   (base, stride along t) of position q at 2 * ((b * T + l) * np + q)
-                              //   (both null: computed from the per-axis tables)
+  const i64 *line_in_tab;     // uniform sides: base offset of line l of tile b at [b * T + l]
+  const i64 *line_out_tab;    //   (both null: computed from the per-axis tables)
   const void *twiddle;        // stage-ordered roots (N 16-byte entries, twiddle_image): stage with
                               //   Ns earlier points and radix R holds w^(jj*r*N/(Ns*R)) at
                               //   (Ns-1) + (r-1)*Ns + jj

@@ -64,10 +64,27 @@ static void lds() {
     }
 }
 
+// Tables of a pass: within the 64 MiB that the line bases of uniform sides
+// may take, however many rank positions a line crosses.
+static void tables() {
+  const Layout uneven({64, 2101, 128}, {1, 1100, 1}), local({64, 2101, 128}, {1, 1, 1});
+  const dm::Side s = uneven.side(), e = local.side();
+  for (int form = 0; form < 4; form++) {
+    dm::TableBuilder tb;
+    dm::PendingPass pp;
+    if (!dm::plan_pass(uneven.comm, form & 1 ? e : s, form & 2 ? e : s, 1, 1, false, nullptr, nullptr, tb, &pp) ||
+        tb.host.size() > (size_t)64 << 20) {
+      printf("%zu bytes of tables, form %d\n", tb.host.size(), form);
+      failures++;
+    }
+  }
+}
+
 int main(int argc, char **argv) {
   dm_set_error_mode(1);
   const std::string check = argc > 1 ? argv[1] : "";
   if (check == "lds") lds();
+  else if (check == "tables") tables();
   else return 2;
   if (failures == 0) printf("OK\n");
   return failures != 0;

@@ -76,3 +76,8 @@ def axis_fft(C, shape, axis, gin, gout, dbl):
 ])
 def test_line_data_beside_wide_tile(C, shape, gin, gout, dbl):
     axis_fft(C, shape, 0, gin, gout, dbl)
+
+
+@pytest.mark.parametrize("dbl", [True, False])
+def test_more_positions_than_lds_on_both_sides(C, dbl):
+    axis_fft(C, (6, 2101, 5), 1, (1, 1100, 1), (1, 1100, 1), dbl)

@@ -32,3 +32,8 @@ def run(driver, check):
 def test_workgroup_lds(driver):
     """No pass asks for more than the 160 KiB of LDS that a workgroup has."""
     run(driver, "lds")
+
+
+def test_table_bytes(driver):
+    """A pass's tables stay bounded with more rank positions than LDS holds."""
+    run(driver, "tables")
