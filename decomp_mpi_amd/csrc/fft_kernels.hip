@@ -30,8 +30,6 @@ int fft_tile_capacity(int dbl, int column, int wide) {
   return small ? cap / 2 : cap;
 }
 
-int fft_line_positions() { return fftpass::kLinePositions; }
-
 // Twiddle table in LDS: 16 bytes per entry for a complex double or a
 // compensated complex-float pair, 8 for a plain complex float.  A
 // compensated table stays within 8 KiB there, so that two 8192-point
@@ -46,7 +44,7 @@ size_t fft_lds_bytes(const FftLaunch &p) {
   size_t elem = p.dbl ? 16 : 8;
   size_t ls = (size_t)lds_line(p.N);
   auto side = [&](const FftSide &s) {
-    return s.uniform ? LineAddr<true>::bytes(p.T, 1) : LineAddr<false>::bytes(p.T, s.np);
+    return s.uniform ? LineAddr<true>::bytes(p.T, s) : LineAddr<false>::bytes(p.T, s);
   };
   // tile data + per-line address data of both sides
   size_t b = (size_t)p.T * ls * elem + side(p.sin) + side(p.sout);

@@ -53,9 +53,6 @@ using lds_cx = __attribute__((address_space(3))) cx<R>;
 template <typename R, bool CT>
 using lds_tw = __attribute__((address_space(3))) typename tw_local<R, CT>::type;
 
-// Line entries (line, position) a non-uniform side keeps in LDS: 16 KiB.
-constexpr int kLinePositions = 1024;
-
 template <bool UNIFORM>
 struct LineAddr;
 
@@ -63,7 +60,7 @@ template <>
 struct LineAddr<true> {
   static constexpr int np = 1;
   lds_i64 *base;
-  __host__ __device__ static size_t bytes(int T, int) { return (size_t)T * sizeof(i64); }
+  __host__ __device__ static size_t bytes(int T, const FftSide &) { return (size_t)T * sizeof(i64); }
   __device__ void init(char *mem, int, int) { base = (lds_i64 *)(mem); }
   __device__ void set_line(const FftLaunch &p, const i64 *abs, const int *g, int l) {
     i64 a = 0;
@@ -90,16 +87,16 @@ struct LineAddr<true> {
 // 126 x 100 complex-double transform on 6 ranks took 43, 43 and 25 us, 129
 // us for the whole call; 86 us with a base and a stride per line and
 // position, dense intermediates and two workgroups per CU.  It is left for
-// lines with more positions than LDS is given (np > kLinePositions): LDS
-// holds the line's owner contribution and its local offsets then.
+// lines over many positions (FftSide::far): LDS holds the line's owner
+// contribution and its local offsets then.
 template <>
 struct LineAddr<false> {
-  static constexpr int kFar = 1 + DM_MAX_DIMS;  // entries a line of the far form
+  static constexpr int kFar = 2 + DM_MAX_DIMS;  // ints a line of the far form
   lds_i64 *base;
   lds_i64 *str;
   int np;
-  __host__ __device__ static size_t bytes(int T, int np) {
-    return np > kLinePositions ? (size_t)T * kFar * sizeof(i64) : (size_t)T * np * 2 * sizeof(i64);
+  __host__ __device__ static size_t bytes(int T, const FftSide &s) {
+    return s.far ? (size_t)T * kFar * sizeof(int) : (size_t)T * s.np * 2 * sizeof(i64);
   }
   __device__ void init(char *mem, int T, int n) {
     base = (lds_i64 *)(mem);
@@ -111,9 +108,10 @@ struct LineAddr<false> {
     int R0 = 0;
     for (int d = 0; d < p.ndim; d++)
       if (d != p.t) R0 += s.rank[p.at[d] + g[d]];
-    if (np > kLinePositions) {
-      base[l * kFar] = R0;
-      for (int d = 0; d < p.ndim; d++) base[l * kFar + 1 + d] = d != p.t ? s.off[p.at[d] + g[d]] : 0;
+    if (s.far) {
+      lds_int *line = (lds_int *)base + l * kFar;
+      line[0] = R0;
+      for (int d = 0; d < p.ndim; d++) line[1 + d] = d != p.t ? s.off[p.at[d] + g[d]] : 0;
       return;
     }
     for (int q = 0; q < np; q++) {
@@ -126,24 +124,22 @@ struct LineAddr<false> {
       str[l * np + q] = m[p.t];
     }
   }
-  // point x, at its local offset, of line l in the far form
-  __device__ i64 far(const FftLaunch &p, const FftSide &s, int l, int x, int off) const {
-    const int R = (int)base[l * kFar] + s.rank[p.at[p.t] + x];
+  // point x of line l in the far form
+  __device__ i64 far(const FftLaunch &p, const FftSide &s, int l, int x) const {
+    const lds_int *line = (const lds_int *)base + l * kFar;
+    const int R = line[0] + s.rank[p.at[p.t] + x];
     const i64 *m = s.strides + (i64)R * p.ndim;
-    i64 a = (i64)R * s.slot + off * m[p.t];
-    for (int d = 0; d < p.ndim; d++) a += m[d] * base[l * kFar + 1 + d];
+    i64 a = (i64)R * s.slot + m[p.t] * s.off[p.at[p.t] + x];
+    for (int d = 0; d < p.ndim; d++) a += m[d] * line[1 + d];
     return a;
   }
   __device__ __forceinline__ i64 at(const FftLaunch &p, const FftSide &s, const i64 *, int l, int x) const {
     if (s.lin) return base[l] + (i64)x * str[l];  // axis t local to every rank, in order
-    if (np > kLinePositions) return far(p, s, l, x, s.xt[2 * x + 1]);
+    if (s.far) return far(p, s, l, x);
     const int k = l * np + s.xt[2 * x];
     return base[k] + (i64)s.xt[2 * x + 1] * str[k];
   }
 };
-
-// Address data one line of a side holds (LineAddr::bytes' second argument).
-__host__ __device__ __forceinline__ int side_positions(const FftSide &s) { return s.uniform ? 1 : s.np; }
 
 // Tile t -> (tile along u, batch coordinates); fills the per-line address
 // data of both sides for that tile (threads l < T).
@@ -353,9 +349,8 @@ __global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 4) vo
   char *lmem = smem_raw + (size_t)T * P.ls * sizeof(cx<R>);
   LineAddr<UIN> lin;
   LineAddr<UOUT> lout;
-  const int npi = side_positions(p.sin), npo = side_positions(p.sout);
-  lin.init(lmem, T, npi);
-  lout.init(lmem + LineAddr<UIN>::bytes(T, npi), T, npo);
+  lin.init(lmem, T, p.sin.np);
+  lout.init(lmem + LineAddr<UIN>::bytes(T, p.sin), T, p.sout.np);
   // Workgroups are dispatched round-robin over the 8 XCDs.  When a tile's
   // rows are shorter than a 128-byte line, the xcd_pair tiles that share
   // those lines are given to consecutive workgroups of one XCD, so its L2
@@ -371,7 +366,7 @@ __global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 4) vo
   tile += p.tile_base;
   const int nl = setup_lines<UIN, UOUT>(p, tile, lin, lout, T, NTH);
   // twiddle table in LDS after the line data
-  size_t tw_at = (size_t)T * P.ls * sizeof(cx<R>) + LineAddr<UIN>::bytes(T, npi) + LineAddr<UOUT>::bytes(T, npo);
+  size_t tw_at = (size_t)T * P.ls * sizeof(cx<R>) + LineAddr<UIN>::bytes(T, p.sin) + LineAddr<UOUT>::bytes(T, p.sout);
   typedef typename tw_local<R, CT>::type TwL;
   typedef typename tw_global<R>::type TwG;
   TwL *twl = reinterpret_cast<TwL *>(smem_raw + ((tw_at + 15) & ~(size_t)15));

@@ -207,11 +207,15 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   const std::vector<int> pos_in = positions(I), pos_out = positions(U);
   L.sin.uniform = I.h.uniform ? 1 : 0;
   L.sin.np = (int)pos_in.size();
+  L.sin.far = L.sin.np > kLinePositions;
   L.sout.uniform = U.h.uniform ? 1 : 0;
   L.sout.np = (int)pos_out.size();
+  L.sout.far = L.sout.np > kLinePositions;
   L.dbl = dbl;
   L.ctw = (!dbl && ctw) ? 1 : 0;
-  const int np_most = (int)std::max(std::max(pos_in.size(), pos_out.size()), (size_t)1);
+  const int np_most = std::max(std::max(L.sin.np, L.sout.np), 1);
+  // positions per line of the sides that keep their lines' bases in LDS
+  const int np_lds = std::max(std::max(L.sin.far ? 1 : L.sin.np, L.sout.far ? 1 : L.sout.np), 1);
   // Small arrays: lines per tile are halved while a pass has fewer than 192
   // tiles for the 256 CUs and rows of 64 bytes stay.  What is left to win
   // there is the latency of one tile, which falls with its points per thread
@@ -240,9 +244,7 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     auto height = [&](bool w) {
       const int T = spread(std::max(1, std::min(std::min(fft_tile_capacity(dbl, !(in_row && out_row), w) / L.N, I.h.L[u]), 512)));
       // per-line address data of a non-uniform side: 16 KiB of LDS at most
-      // (a side with more positions than that forms its addresses point by
-      // point)
-      return np_most > 1 ? std::max(1, std::min(T, fft_line_positions() / np_most)) : T;
+      return np_lds > 1 ? std::max(1, std::min(T, kLineEntries / np_lds)) : T;
     };
     L.T = height(wide && !nowide);
     // the wide tile (136 KiB and up to 16 of twiddles) leaves no room for the

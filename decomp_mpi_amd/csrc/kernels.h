@@ -86,6 +86,7 @@ struct FftSide {
   // non-uniform sides
   int np;                      // rank positions along t
   int lin;                     // one position, local offset x at point x
+  int far;                     // more than kLinePositions: addresses formed point by point
   const int *xt;               // point x of t: position, local offset
   const int *posrank;          // owner contribution of each position
   const int *rank, *off;       // owner contributions and local offsets, axis d's at FftLaunch::at[d]
@@ -156,10 +157,17 @@ int launch_fft_pass(const FftLaunch &p, void *stream);
 // column walks at a large line stride ("wide") a double one (16 lines of
 // 512 points, 256-byte rows).
 int fft_tile_capacity(int dbl, int column, int wide = 0);
-// (line, position) entries a non-uniform side of a tile keeps in LDS.
-int fft_line_positions();
+// (line, position) entries a non-uniform side of a tile keeps in LDS, at
+// most (16 KiB), and the most positions of one that keeps any.
+// A line's entries are formed one after another, so with more positions
+// that costs more than it saves: 385-point lines of 65 x 66 x 385 complex
+// doubles on 2 x np ranks, both sides uneven, take 25 us with them at np 3,
+// 28 at 6, 30 at 8, 35 at 12, 60 at 16 and 88 at 32, and 29 to 30 at any
+// without.
+constexpr int kLineEntries = 1024;
+constexpr int kLinePositions = 6;
 // LDS a workgroup of the pass takes: its tile, the line data of both sides
-// (uniform, np) and the twiddles.  At most kLdsBytes, or the launch is refused.
+// (uniform, np, far) and the twiddles.  At most kLdsBytes, or the launch is refused.
 constexpr size_t kLdsBytes = 160 * 1024;
 size_t fft_lds_bytes(const FftLaunch &p);
 

@@ -42,7 +42,7 @@ struct Layout {
 // last axis the line stride (64 KiB or more with 130 points).
 static void lds() {
   for (int n : {256, 360, 512, 729, 1000, 1024, 2048, 4096})
-    for (int np : {1, 2, 16, 20, 32, 34, 47, 64, 68, 100, 128, 146, 256}) {
+    for (int np : {1, 2, 6, 7, 16, 20, 32, 34, 47, 64, 68, 100, 128, 146, 256}) {
       if (np > n / 2) continue;
       const Layout even({n, 66, 130}, {1, 2, 1}), uneven({n, 65, 130}, {np, 2, 1}), local({n, 65, 130}, {1, 1, 1});
       const dm::Side e = local.side(), s = uneven.side();

@@ -81,3 +81,16 @@ def test_line_data_beside_wide_tile(C, shape, gin, gout, dbl):
 @pytest.mark.parametrize("dbl", [True, False])
 def test_more_positions_than_lds_on_both_sides(C, dbl):
     axis_fft(C, (6, 2101, 5), 1, (1, 1100, 1), (1, 1100, 1), dbl)
+
+
+@pytest.mark.parametrize("dbl", [True, False])
+@pytest.mark.parametrize("shape,axis,gin,gout", [
+    ((5, 50, 33), 1, (2, 6, 1), (2, 6, 1)),     # the most positions that are kept
+    ((5, 50, 33), 1, (2, 7, 1), (2, 3, 1)),     # one more on one side
+    ((5, 50, 33), 1, (1, 6, 1), (1, 10, 1)),    # and on the other
+    ((9, 300, 8), 1, (2, 7, 1), (2, 100, 1)),
+    ((7, 5, 61), 2, (2, 1, 20), (2, 1, 20)),    # a direct-sum prime, contiguous axis
+    ((385, 65, 66), 0, (12, 2, 1), (12, 2, 1)), # the wide tile
+])
+def test_kept_positions_and_beyond(C, shape, axis, gin, gout, dbl):
+    axis_fft(C, shape, axis, gin, gout, dbl)
