@@ -8,7 +8,7 @@ import pytest
 
 import decomp_mpi_amd as dm
 from helpers import rel_l2
-from test_gpu_fft import TOL32, TOL64
+from test_gpu_fft import TOL32, TOL64, run_split
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +94,17 @@ def test_more_positions_than_lds_on_both_sides(C, dbl):
 ])
 def test_kept_positions_and_beyond(C, shape, axis, gin, gout, dbl):
     axis_fft(C, shape, axis, gin, gout, dbl)
+
+
+@pytest.mark.parametrize("dbl", [True, False])
+@pytest.mark.parametrize("P,shape,grid", [
+    (4, (33, 1024), (2, 2)),       # the longest line of 64-byte rows
+    (4, (33, 1050), (2, 2)),       # one beyond, and blocks of 33 are uneven
+    (12, (26, 3025), (6, 2)),
+    (6, (1050, 35), (3, 2)),       # the long axis last: dense all the same
+    (6, (5, 1100, 14), (1, 3, 2)),
+])
+def test_uneven_intermediates_of_long_lines(C, P, shape, grid, dbl):
+    fwd, rt, _ = run_split(C, P, shape, grid, slab=0, dbl=dbl)
+    tol = TOL64 if dbl else TOL32
+    assert fwd < tol and rt < tol, (fwd, rt)
