@@ -46,6 +46,10 @@ struct ReshapeLaunch {
   int nontemporal;        // owned: non-temporal hint on the element accesses
 };
 constexpr int kReshapePairs = 512;  // (a position, b position) pairs of a side in LDS, at most
+// LDS of the tile a launch of the owned kernels would use, at most kTileLds
+// (what a launch gets without asking for more; 0: not a tile).
+constexpr size_t kTileLds = 64 * 1024;
+size_t reshape_tile_lds(const ReshapeLaunch &p);
 // Launchers return 0 or the HIP error code of the launch (hipError_t).
 int launch_reshape(const ReshapeLaunch &p, void *stream);
 

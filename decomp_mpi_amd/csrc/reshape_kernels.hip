@@ -9,6 +9,8 @@
 // coordinate) plus per-rank memory strides.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace dm {
@@ -513,32 +515,73 @@ hipError_t launch_rows(ReshapeLaunch &p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Tile shapes: 16 elements a thread (8 of 16 bytes), since an element costs
-// more instructions than bytes, with rows of at least 256 bytes on both
-// sides.  Measured us a pass, tile a x b x slices:
-//   512^3 int64 chain (two hops)          64x64 844, 32x64x2 907, 64x32x2 872, 32x32x2 963
-//   400 x 380 x 392 4-byte, permuted      128x64 179, 64x64 204, 64x128 206, 32x32x2 294
-//   400 x 380 x 392 16-byte, permuted     64x32 440, 32x32 490, 32x64 486
-// A tile axis of at most 16 values (the phase order's split axes, 16-byte
-// elements) takes a 16-wide tile and two slices: half of a 32-wide one would
-// stay empty (512^3 phase order, both reshapes 0.96 -> 0.79 and 0.74 ms).
+// Tile shapes (a x b x batch slices).
+//   small   32 x 32 of 16 KiB: the least latency, and little lost where an
+//           axis does not fill its tiles
+//   large   16 elements a thread (8 of 16 bytes), rows of at least 256 bytes
+//           on both sides: an element costs more instructions than bytes
+//   narrow  16 wide, for an axis of at most 16 values (the phase order's
+//           split axes), where a 32-wide tile stays half empty
+// Measured us a pass (large / small / narrow; before there were several: 32 x
+// 32 x 2, element addresses in 64 bits):
+//   512^3 int64 chain, two hops               844 / 963; before 944
+//   400 x 380 x 392 4-byte, permuted          179 / 294
+//   352 x 416 x 256 int64 chain               332 / 360; 368
+//   416 x 352 x 64 int64 chain (72 MB a side) 104 / 109; 117
+//   384 x 64 x 224 int64 chain (42 MB)        70 / 57; 80
+//   512 x 64 x 96 4-byte, permuted (12 MB)    26.5 / 18.8; 22.7
+//   352 x 256 x 96 int64 chain, tiles 3/4 full 91.6 / 78.1; 87.2
+//   512^3 phase order, complex float (calls)  5752 / 3160 / 3160; 5854
+//   256^3 phase order, complex float          1110 / 519 / 463; 923
+//   64^3 phase order, complex float           177 / 141 / 148; 179
+// (the split axes of 512^3 are 16 x 32 points: a large tile is an eighth
+// full.)  Hence: the narrow tile from 32 MiB a side on where an axis is
+// short, the large one from 64 MiB on unless rounding the axes up to it moves
+// a fifth more than rounding them up to the small one, else the small one.
+struct TileForm {
+  int a, b, n;
+};
+constexpr TileForm small_tile(int bytes) { return {32, 32, bytes > 8 ? 1 : 2}; }
+constexpr TileForm large_tile(int bytes) {
+  return bytes == 16 ? TileForm{64, 32, 1} : (bytes == 8 ? TileForm{64, 64, 1} : TileForm{128, 64, 1});
+}
+constexpr TileForm narrow_tile(int bytes, bool along_a) {
+  return along_a ? TileForm{16, 32, bytes == 16 ? 2 : 4} : TileForm{32, 16, bytes == 16 ? 2 : 4};
+}
+// LDS of a tile: the elements and both sides' pair tables.
+size_t tile_lds(const ReshapeLaunch &p, TileForm f) {
+  const int pairs = (p.src.uniform ? 0 : p.ss.np[0] * p.ss.np[1]) + (p.dst.uniform ? 0 : p.sd.np[0] * p.sd.np[1]);
+  return (size_t)f.n * f.a * (f.b + 1) * p.elem_bytes + (size_t)pairs * 3 * f.n * (p.below_4g ? 4 : 8);
+}
+TileForm tile_form(const ReshapeLaunch &p) {
+  const int bytes = p.elem_bytes, la = p.L[p.a], lb = p.L[p.b];
+  const TileForm small = small_tile(bytes);
+  if (bytes == 12 || bytes == 24) return small;
+  double side = bytes;
+  for (int d = 0; d < p.ndim; d++) side *= p.L[d];
+  auto rounded = [&](TileForm f) { return (double)((la + f.a - 1) / f.a * f.a) * ((lb + f.b - 1) / f.b * f.b); };
+  const TileForm large = large_tile(bytes), narrow = narrow_tile(bytes, la <= 16);
+  if (std::min(la, lb) <= 16 && side >= (32 << 20) && tile_lds(p, narrow) <= kTileLds) return narrow;
+  if (side >= (64 << 20) && rounded(large) <= 1.25 * rounded(small)) return large;
+  // (two slices' pair tables of 512 pairs a side in 64 bits: 66 KiB in all)
+  return tile_lds(p, small) <= kTileLds ? small : large;
+}
+
 template <int BYTES, bool US, bool UD>
 hipError_t launch_owned(ReshapeLaunch &p, hipStream_t s) {
   if (p.same_order) {
     if (p.L[p.a] <= 64) return launch_rows<BYTES, US, UD, 64>(p, s);
     return launch_rows<BYTES, US, UD, 256>(p, s);
   }
-  if constexpr (BYTES == 16) {
-    if (p.L[p.a] <= 16) return launch_tile<BYTES, US, UD, 16, 32, 2>(p, s);
-    if (p.L[p.b] <= 16) return launch_tile<BYTES, US, UD, 32, 16, 2>(p, s);
-    return launch_tile<BYTES, US, UD, 64, 32, 1>(p, s);
-  } else if constexpr (BYTES > 8) {
-    return launch_tile<BYTES, US, UD, 32, 32, 1>(p, s);
-  } else if constexpr (BYTES == 8) {
-    return launch_tile<BYTES, US, UD, 64, 64, 1>(p, s);
-  } else {
-    return launch_tile<BYTES, US, UD, 128, 64, 1>(p, s);
+  const TileForm f = tile_form(p);
+  if constexpr (BYTES != 12 && BYTES != 24) {
+    constexpr TileForm large = large_tile(BYTES), na = narrow_tile(BYTES, true), nb = narrow_tile(BYTES, false);
+    if (f.a == na.a) return launch_tile<BYTES, US, UD, na.a, na.b, na.n>(p, s);
+    if (f.b == nb.b) return launch_tile<BYTES, US, UD, nb.a, nb.b, nb.n>(p, s);
+    if (f.a == large.a) return launch_tile<BYTES, US, UD, large.a, large.b, large.n>(p, s);
   }
+  constexpr TileForm small = small_tile(BYTES);
+  return launch_tile<BYTES, US, UD, small.a, small.b, small.n>(p, s);
 }
 
 // ---- coordinates without an owner, or very many rank positions --------------
@@ -577,6 +620,8 @@ hipError_t launch_bytes(ReshapeLaunch &p, hipStream_t s) {
 }
 
 }  // namespace
+
+size_t reshape_tile_lds(const ReshapeLaunch &p) { return p.owned && !p.same_order ? tile_lds(p, tile_form(p)) : 0; }
 
 // Tile counts and grid size are filled here so the host only chooses axes.
 int launch_reshape(const ReshapeLaunch &p0, void *stream) {

@@ -1,6 +1,6 @@
-// The FFT pass planner against its kernels' limits, without a GPU: passes
-// are planned from real decompositions through the library's own internal
-// headers, and what the launch would ask for is checked here.
+// The planners against their kernels' limits, without a GPU: passes are
+// planned from real decompositions through the library's own internal
+// headers, and what a launch would ask for is checked here.
 // Usage: host_passes <check>; prints OK.
 #include <cstdio>
 #include <cstring>
@@ -80,11 +80,44 @@ static void tables() {
   }
 }
 
+// A reshape tile's LDS, for every element size, tile axis length, array size
+// and number of rank positions that the owned kernels take.
+static void reshape() {
+  for (int bytes : {1, 2, 4, 8, 12, 16, 24})
+    for (int la : {8, 16, 17, 64, 500})
+      for (int lb : {8, 16, 17, 64, 500})
+        for (int batch : {1, 100, 10000, 1000000})
+          for (int pairs : {1, 100, dm::kReshapePairs})
+            for (int form = 0; form < 8; form++) {
+              dm::ReshapeLaunch L;
+              memset(&L, 0, sizeof L);
+              L.owned = 1;
+              L.ndim = 3;
+              L.L[0] = batch;
+              L.L[1] = la;
+              L.L[2] = lb;
+              L.a = 1;
+              L.b = 2;
+              L.elem_bytes = bytes;
+              L.src.uniform = form & 1;
+              L.dst.uniform = form >> 1 & 1;
+              L.below_4g = form >> 2 & 1;
+              L.ss.np[0] = L.sd.np[1] = pairs;
+              L.ss.np[1] = L.sd.np[0] = 1;
+              const size_t need = dm::reshape_tile_lds(L);
+              if (need == 0 || need > 64 * 1024) {
+                printf("%zu bytes of LDS: %d bytes, %d x %d x %d, %d pairs, form %d\n", need, bytes, batch, la, lb, pairs, form);
+                failures++;
+              }
+            }
+}
+
 int main(int argc, char **argv) {
   dm_set_error_mode(1);
   const std::string check = argc > 1 ? argv[1] : "";
   if (check == "lds") lds();
   else if (check == "tables") tables();
+  else if (check == "reshape") reshape();
   else return 2;
   if (failures == 0) printf("OK\n");
   return failures != 0;

@@ -1,4 +1,4 @@
-"""The FFT pass planner against its kernels' limits, without a GPU: a driver
+"""The planners against their kernels' limits, without a GPU: a driver
 (tests/c_api/host_passes.cpp) plans passes through the library's internal
 headers and checks what their launches would ask for."""
 import os
@@ -37,3 +37,8 @@ def test_workgroup_lds(driver):
 def test_table_bytes(driver):
     """A pass's tables stay bounded with more rank positions than LDS holds."""
     run(driver, "tables")
+
+
+def test_reshape_tile_lds(driver):
+    """No reshape tile asks for more than 64 KiB of LDS."""
+    run(driver, "reshape")
