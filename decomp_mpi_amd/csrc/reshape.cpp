@@ -544,12 +544,19 @@ bool enqueue_reshape(dm_comm_t comm, ReshapePlan plan, const void *src, void *ds
   L.elem_bytes = pg->word;
   L.below_4g = s.buf.slot * (size_t)s.buf.nranks < ((size_t)1 << 32) && d.buf.slot * (size_t)d.buf.nranks < ((size_t)1 << 32);
   // Data that the memory-side cache holds (256 MB, both sides) is left
-  // there: 28 MB in and out 27 us a pass without the hint, 32 with it;
-  // the 512^3 int64 chain (1 GiB in and out a hop) 897 us without, 860 with.
+  // there; the hint pays from about twice that on (us a hop pair or call):
+  //   288 x 96 x 352 int64 chain, 74 MB a side     149 with it, 89 without
+  //   416 x 64 x 416, 85 MB                        129 and 102
+  //   384 x 192 x 224, 126 MB                      147 and 138
+  //   448 x 256 x 192, 168 MB                      163 and 170
+  //   352 x 416 x 256, 286 MB                      333 and 308
+  //   512^3, 1 GiB                                 860 and 897
+  // and 256^3 phase-order calls, 128 MB complex float 461 and 472, 256 MB
+  // complex double 606 and 624.
   size_t moved = 0;
   for (auto e : pg->src.slot_extent) moved += (size_t)e * pg->word;
   static const bool nont = getenv("DM_NO_NONTEMPORAL") != nullptr;
-  L.nontemporal = nont || 2 * moved <= ((size_t)128 << 20) ? 0 : 1;
+  L.nontemporal = nont || 2 * moved < ((size_t)256 << 20) ? 0 : 1;
   return launch_ok(comm, launch_reshape(L, stream), "reshape kernel launch");
 }
 }  // namespace dm
