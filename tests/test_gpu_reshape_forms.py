@@ -1,7 +1,8 @@
 """The reshape's tile forms at sizes where each is chosen: large tiles (64 MiB
-a side and more) and narrow ones (a tile axis of at most 16 values, 32 MiB and
-more), with remainders along both tile axes and the batch, even and uneven
-ranks.  Bit-exact against the oracle on every destination byte."""
+a side and more) and narrow ones (a tile axis of at most 16 values, 128 MiB
+over the element size and more), with remainders along both tile axes and the
+batch, even and uneven ranks.  Bit-exact against the oracle on every
+destination byte."""
 import pytest
 
 import decomp_mpi_amd as dm
@@ -39,4 +40,4 @@ def test_large(C, elem, grid):
 @pytest.mark.parametrize("shape", [(13, 515), (515, 13), (16, 16)])
 @pytest.mark.parametrize("grid", [(1, 1, 1), (2, 2, 3)])
 def test_narrow(C, elem, shape, grid):
-    permuted(C, elem, shape, grid, 32)
+    permuted(C, elem, shape, grid, 128 // elem)
