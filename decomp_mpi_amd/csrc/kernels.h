@@ -43,7 +43,7 @@ struct ReshapeLaunch {
   i64 dst_bytes;
   int elem_bytes;
   int below_4g;           // owned: both buffers below 4 GiB
-  int nontemporal;        // owned: non-temporal hint on the element accesses
+  int nontemporal;        // non-temporal hint on the element accesses
 };
 constexpr int kReshapePairs = 512;  // (a position, b position) pairs of a side in LDS, at most
 // LDS of the tile a launch of the owned kernels would use, at most kTileLds

@@ -552,11 +552,11 @@ bool enqueue_reshape(dm_comm_t comm, ReshapePlan plan, const void *src, void *ds
   //   352 x 416 x 256, 286 MB                      333 and 308
   //   512^3, 1 GiB                                 860 and 897
   // and 256^3 phase-order calls, 128 MB complex float 461 and 472, 256 MB
-  // complex double 606 and 624.
+  // complex double 606 and 624.  (The general kernels have it always.)
   size_t moved = 0;
   for (auto e : pg->src.slot_extent) moved += (size_t)e * pg->word;
   static const bool nont = getenv("DM_NO_NONTEMPORAL") != nullptr;
-  L.nontemporal = nont || 2 * moved < ((size_t)256 << 20) ? 0 : 1;
+  L.nontemporal = nont || (pg->owned && 2 * moved < ((size_t)256 << 20)) ? 0 : 1;
   return launch_ok(comm, launch_reshape(L, stream), "reshape kernel launch");
 }
 }  // namespace dm

@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kernels.h"
 
@@ -32,6 +33,36 @@ template <> struct Elem<2> { typedef uint16_t T; };
 template <> struct Elem<4> { typedef uint32_t T; };
 template <> struct Elem<8> { typedef uint64_t T; };
 template <> struct Elem<16> { typedef unsigned int T __attribute__((ext_vector_type(4))); };
+
+// 12- and 24-byte elements (three floats, three doubles) move whole: as three
+// separate words each access would use a third of its lines.
+struct E12 { uint32_t x, y, z; };
+struct E24 { uint64_t x, y, z; };
+template <> struct Elem<12> { typedef E12 T; };
+template <> struct Elem<24> { typedef E24 T; };
+
+// One element access.  NT: the non-temporal hint (a template argument: a
+// hinted and a plain access in two branches are merged into one by the
+// compiler, which drops the hint).
+template <bool NT, typename E>
+__device__ __forceinline__ E take(const E *e) {
+  if constexpr (!NT) return *e;
+  else if constexpr (sizeof(E) == 12 || sizeof(E) == 24)
+    return {__builtin_nontemporal_load(&e->x), __builtin_nontemporal_load(&e->y), __builtin_nontemporal_load(&e->z)};
+  else return __builtin_nontemporal_load(e);
+}
+template <bool NT, typename E>
+__device__ __forceinline__ void give(E *e, E v) {
+  if constexpr (!NT) {
+    *e = v;
+  } else if constexpr (sizeof(E) == 12 || sizeof(E) == 24) {
+    __builtin_nontemporal_store(v.x, &e->x);
+    __builtin_nontemporal_store(v.y, &e->y);
+    __builtin_nontemporal_store(v.z, &e->z);
+  } else {
+    __builtin_nontemporal_store(v, e);
+  }
+}
 
 // Per-block partial sums of the batch axes for one layout.
 struct Partial {
@@ -86,7 +117,7 @@ __device__ __forceinline__ i64 locate(const DevLayout &Lt, const ReshapeLaunch &
 // to element 0 of the region when the element is absent), then the LDS (or
 // global) writes.  A load queue that completes in order would otherwise
 // stall each data load behind the next element's table loads.
-template <int BYTES, bool US, bool UD, int NB>
+template <int BYTES, bool US, bool UD, int NB, bool NT>
 __global__ __launch_bounds__(NTHREADS) void reshape_tile2d(ReshapeLaunch p) {
   typedef typename Elem<BYTES>::T E;
   constexpr int RPT = TILE / ROWS;
@@ -153,7 +184,7 @@ __global__ __launch_bounds__(NTHREADS) void reshape_tile2d(ReshapeLaunch p) {
 #pragma unroll
   for (int n = 0; n < NB; n++)
 #pragma unroll
-    for (int k = 0; k < RPT; k++) v[n][k] = __builtin_nontemporal_load(src + (s[n][k] >= 0 ? s[n][k] : 0));
+    for (int k = 0; k < RPT; k++) v[n][k] = take<NT>(src + (s[n][k] >= 0 ? s[n][k] : 0));
 #pragma unroll
   for (int n = 0; n < NB; n++)
 #pragma unroll
@@ -199,11 +230,11 @@ __global__ __launch_bounds__(NTHREADS) void reshape_tile2d(ReshapeLaunch p) {
   for (int n = 0; n < NB; n++)
 #pragma unroll
     for (int k = 0; k < RPT; k++)
-      if (d[n][k] >= 0) __builtin_nontemporal_store(tile[n][tx][ty + k * ROWS], dst + d[n][k]);
+      if (d[n][k] >= 0) give<NT>(dst + d[n][k], tile[n][tx][ty + k * ROWS]);
 }
 
 // 1D runs along axis a (same fastest axis on both sides), phased as above.
-template <int BYTES, bool US, bool UD>
+template <int BYTES, bool US, bool UD, bool NT>
 __global__ __launch_bounds__(NTHREADS) void reshape_run1d(ReshapeLaunch p) {
   typedef typename Elem<BYTES>::T E;
   constexpr int PER = 4;
@@ -229,45 +260,13 @@ __global__ __launch_bounds__(NTHREADS) void reshape_run1d(ReshapeLaunch p) {
   }
   E v[PER];
 #pragma unroll
-  for (int k = 0; k < PER; k++) v[k] = __builtin_nontemporal_load(src + (s[k] >= 0 ? s[k] : 0));
+  for (int k = 0; k < PER; k++) v[k] = take<NT>(src + (s[k] >= 0 ? s[k] : 0));
 #pragma unroll
   for (int k = 0; k < PER; k++)
-    if (d[k] >= 0) __builtin_nontemporal_store(v[k], dst + d[k]);
+    if (d[k] >= 0) give<NT>(dst + d[k], v[k]);
 }
 
 // ---- every coordinate owned on both sides ----------------------------------
-
-// 12- and 24-byte elements (three floats, three doubles) move whole: as three
-// separate words each access would use a third of its lines.
-struct E12 { uint32_t x, y, z; };
-struct E24 { uint64_t x, y, z; };
-template <> struct Elem<12> { typedef E12 T; };
-template <> struct Elem<24> { typedef E24 T; };
-
-// One element access.  NT: the non-temporal hint (a template argument: a
-// hinted and a plain access in two branches are merged into one by the
-// compiler, which drops the hint).
-template <bool NT, typename E>
-__device__ __forceinline__ E take(const char *at) {
-  const E *e = reinterpret_cast<const E *>(at);
-  if constexpr (!NT) return *e;
-  else if constexpr (sizeof(E) == 12 || sizeof(E) == 24)
-    return {__builtin_nontemporal_load(&e->x), __builtin_nontemporal_load(&e->y), __builtin_nontemporal_load(&e->z)};
-  else return __builtin_nontemporal_load(e);
-}
-template <bool NT, typename E>
-__device__ __forceinline__ void give(char *at, E v) {
-  E *e = reinterpret_cast<E *>(at);
-  if constexpr (!NT) {
-    *e = v;
-  } else if constexpr (sizeof(E) == 12 || sizeof(E) == 24) {
-    __builtin_nontemporal_store(v.x, &e->x);
-    __builtin_nontemporal_store(v.y, &e->y);
-    __builtin_nontemporal_store(v.z, &e->z);
-  } else {
-    __builtin_nontemporal_store(v, e);
-  }
-}
 
 // f(axis, coordinate) for every batch axis at batch index bidx (last batch
 // axis fastest); 32-bit divisions while the index fits.
@@ -422,7 +421,7 @@ __global__ __launch_bounds__(NTHREADS) void reshape_tile(ReshapeLaunch p) {
 #pragma unroll
     for (int n = 0; n < NB; n++)
 #pragma unroll
-      for (int k = 0; k < N; k++) v[n][k] = take<NT, E>(p.src_base + src.base(n) + at[n][k]);
+      for (int k = 0; k < N; k++) v[n][k] = take<NT>(reinterpret_cast<const E *>(p.src_base + src.base(n) + at[n][k]));
 #pragma unroll
     for (int n = 0; n < NB; n++)
 #pragma unroll
@@ -447,7 +446,8 @@ __global__ __launch_bounds__(NTHREADS) void reshape_tile(ReshapeLaunch p) {
   for (int n = 0; n < NB; n++)
 #pragma unroll
     for (int k = 0; k < N; k++)
-      if (live[n] && a0 + tx < La && b0 + ty + k * SA < Lb) give<NT, E>(p.dst_base + dst.base(n) + at[n][k], v[n][k]);
+      if (live[n] && a0 + tx < La && b0 + ty + k * SA < Lb) 
+        give<NT>(reinterpret_cast<E *>(p.dst_base + dst.base(n) + at[n][k]), v[n][k]);
 }
 
 // Both sides fastest along a: rows of TX lanes along a, N rows of axis b per
@@ -480,10 +480,10 @@ __global__ __launch_bounds__(NTHREADS) void reshape_rows(ReshapeLaunch p) {
   }
   E v[N];
 #pragma unroll
-  for (int k = 0; k < N; k++) v[k] = take<NT, E>(p.src_base + src.base(0) + from[k]);
+  for (int k = 0; k < N; k++) v[k] = take<NT>(reinterpret_cast<const E *>(p.src_base + src.base(0) + from[k]));
 #pragma unroll
   for (int k = 0; k < N; k++)
-    if (ga < La && (tb * N + k) * SB + ty < Lb) give<NT, E>(p.dst_base + dst.base(0) + to[k], v[k]);
+    if (ga < La && (tb * N + k) * SB + ty < Lb) give<NT>(reinterpret_cast<E *>(p.dst_base + dst.base(0) + to[k]), v[k]);
 }
 
 template <int BYTES, bool US, bool UD, int TA, int TB, int NB>
@@ -494,10 +494,11 @@ hipError_t launch_tile(ReshapeLaunch &p, hipStream_t s) {
   if (p.nblocks <= 0) return hipSuccess;
   const dim3 grid((unsigned)p.nblocks), block(NTHREADS);
   const size_t l4 = side_lds<US, UD, NB, unsigned>(p), l8 = side_lds<US, UD, NB, i64>(p);
-  if (!p.below_4g) hipLaunchKernelGGL((reshape_tile<BYTES, US, UD, TA, TB, NB, i64, true>), grid, block, l8, s, p);
-  else if (p.nontemporal)
+  if (p.below_4g && p.nontemporal)
     hipLaunchKernelGGL((reshape_tile<BYTES, US, UD, TA, TB, NB, unsigned, true>), grid, block, l4, s, p);
-  else hipLaunchKernelGGL((reshape_tile<BYTES, US, UD, TA, TB, NB, unsigned, false>), grid, block, l4, s, p);
+  else if (p.below_4g) hipLaunchKernelGGL((reshape_tile<BYTES, US, UD, TA, TB, NB, unsigned, false>), grid, block, l4, s, p);
+  else if (p.nontemporal) hipLaunchKernelGGL((reshape_tile<BYTES, US, UD, TA, TB, NB, i64, true>), grid, block, l8, s, p);
+  else hipLaunchKernelGGL((reshape_tile<BYTES, US, UD, TA, TB, NB, i64, false>), grid, block, l8, s, p);
   return hipGetLastError();
 }
 template <int BYTES, bool US, bool UD, int TX>
@@ -509,9 +510,10 @@ hipError_t launch_rows(ReshapeLaunch &p, hipStream_t s) {
   if (p.nblocks <= 0) return hipSuccess;
   const dim3 grid((unsigned)p.nblocks), block(NTHREADS);
   const size_t l4 = side_lds<US, UD, 1, unsigned>(p), l8 = side_lds<US, UD, 1, i64>(p);
-  if (!p.below_4g) hipLaunchKernelGGL((reshape_rows<BYTES, US, UD, TX, i64, true>), grid, block, l8, s, p);
-  else if (p.nontemporal) hipLaunchKernelGGL((reshape_rows<BYTES, US, UD, TX, unsigned, true>), grid, block, l4, s, p);
-  else hipLaunchKernelGGL((reshape_rows<BYTES, US, UD, TX, unsigned, false>), grid, block, l4, s, p);
+  if (p.below_4g && p.nontemporal) hipLaunchKernelGGL((reshape_rows<BYTES, US, UD, TX, unsigned, true>), grid, block, l4, s, p);
+  else if (p.below_4g) hipLaunchKernelGGL((reshape_rows<BYTES, US, UD, TX, unsigned, false>), grid, block, l4, s, p);
+  else if (p.nontemporal) hipLaunchKernelGGL((reshape_rows<BYTES, US, UD, TX, i64, true>), grid, block, l8, s, p);
+  else hipLaunchKernelGGL((reshape_rows<BYTES, US, UD, TX, i64, false>), grid, block, l8, s, p);
   return hipGetLastError();
 }
 
@@ -606,8 +608,13 @@ hipError_t launch_typed(ReshapeLaunch &p, hipStream_t s) {
     }
     if (p.nblocks <= 0) return hipSuccess;
     const dim3 grid((unsigned)p.nblocks), block(NTHREADS);
-    if (p.a != p.b) hipLaunchKernelGGL((reshape_tile2d<BYTES, US, UD, tile_slices(BYTES)>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((reshape_run1d<BYTES, US, UD>), grid, block, 0, s, p);
+    auto launch = [&](auto nt) {
+      constexpr bool NT = decltype(nt)::value;
+      if (p.a != p.b) hipLaunchKernelGGL((reshape_tile2d<BYTES, US, UD, tile_slices(BYTES), NT>), grid, block, 0, s, p);
+      else hipLaunchKernelGGL((reshape_run1d<BYTES, US, UD, NT>), grid, block, 0, s, p);
+    };
+    if (p.nontemporal) launch(std::true_type{});
+    else launch(std::false_type{});
     return hipGetLastError();
   }
 }
