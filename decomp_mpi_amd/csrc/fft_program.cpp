@@ -229,7 +229,7 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
     if (d != t) lines *= I.h.L[d];
   auto spread = [&](int T) {
     const int least = 64 / (dbl ? 16 : 8);
-    while (T > least && lines / T < 192) T = (T + 1) / 2;
+    while (T > least && lines / T < 192) T = std::max(least, (T + 1) / 2);
     return T;
   };
   if (u >= 0) {
@@ -279,19 +279,19 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   L.merge_v = -1;
   L.merge_k = 1;
   if (u >= 0 && L.nbatch > 0 && in_row && out_row) {
-    const int per = spread(std::min(fft_tile_capacity(dbl, 0) / L.N, 512));
-    const int lu = I.h.L[u];
-    const int v = L.batch_axis[L.nbatch - 1];
-    if (2 * lu <= per && np_most == 1) {
-      for (int k = per / lu; k >= 2; k--)
-        if (I.h.L[v] % k == 0) {
+    // (the most that leave 192 tiles; fewer tiles than that whatever k is:
+    // the height of small arrays)
+    const int lu = I.h.L[u], v = L.batch_axis[L.nbatch - 1];
+    const int full = std::min(fft_tile_capacity(dbl, 0) / L.N, 512), low = spread(full);
+    if (np_most == 1)
+      for (int k = full / lu; k >= 2; k--)
+        if (I.h.L[v] % k == 0 && (lines / (lu * k) >= 192 || lu * k <= low)) {
           L.merge_v = v;
           L.merge_k = k;
           L.T = lu * k;
           L.tiles_u = 1;
           break;
         }
-    }
   }
   const long long ntiles = fft_pass_tiles(L);
   long long batch = 1;
