@@ -537,11 +537,12 @@ hipError_t launch_rows(ReshapeLaunch &p, hipStream_t s) {
 //   256^3 phase order, complex float          1110 / 519 / 463; 923
 //   64^3 phase order, complex float           177 / 141 / 148; 179
 // (the split axes of 512^3 are 16 x 32 points: a large tile is an eighth
-// full; 215 x 13 x 310 16-byte, 14 MB, 21.2 us small, 19.4 narrow.)  Hence: the
-// narrow tile from 128 MiB over the element size on (8 MiB of 16 bytes, 32
-// MiB of 4) where an axis is short, the large one from 64 MiB a side on unless rounding the
-// axes up to it moves a fifth more than rounding them up to the small one,
-// else the small one.
+// full; 215 x 13 x 310 16-byte, 14 MB, 21.2 us small, 19.4 narrow; calls of
+// 512 x 30 x 30 in phase order, complex double, 7 MB, 193 and 179.)  Hence:
+// where an axis is short the narrow tile, of fewer than 16 bytes from 128
+// MiB over the element size on; the large one from 64 MiB a side on unless
+// rounding the axes up to it moves a fifth more than rounding them up to the
+// small one; else the small one.
 struct TileForm {
   int a, b, n;
 };
@@ -565,7 +566,8 @@ TileForm tile_form(const ReshapeLaunch &p) {
   for (int d = 0; d < p.ndim; d++) side *= p.L[d];
   auto rounded = [&](TileForm f) { return (double)((la + f.a - 1) / f.a * f.a) * ((lb + f.b - 1) / f.b * f.b); };
   const TileForm large = large_tile(bytes), narrow = narrow_tile(bytes, la <= 16);
-  if (std::min(la, lb) <= 16 && side > (double)(128 << 20) / bytes && tile_lds(p, narrow) <= kTileLds) return narrow;
+  if (std::min(la, lb) <= 16 && (bytes == 16 || side > (double)(128 << 20) / bytes) && tile_lds(p, narrow) <= kTileLds)
+    return narrow;
   if (side >= (64 << 20) && rounded(large) <= 1.25 * rounded(small)) return large;
   // (two slices' pair tables of 512 pairs a side in 64 bits: 66 KiB in all)
   return tile_lds(p, small) <= kTileLds ? small : large;
