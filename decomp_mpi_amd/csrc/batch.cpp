@@ -202,7 +202,8 @@ static bool plane_fits(int n1, int n2, int dbl) {
 
 // Schedule of plane tiles: the columns' first stage, the rows' stages, the
 // columns' other ones, a power of two last where there are two.
-static void make_plane_sched(int n1, int n2, int T, int radix_order, BatchPlane *out, std::vector<double> *tw) {
+// Powers of two in butterflies of up to 2^most points.
+static void make_plane_sched(int n1, int n2, int T, int radix_order, int most, BatchPlane *out, std::vector<double> *tw) {
   BatchPlane P{};
   P.plane = n1 * n2;
   P.points = T * n1 * n2;
@@ -222,12 +223,13 @@ static void make_plane_sched(int n1, int n2, int T, int radix_order, BatchPlane 
   };
   std::vector<int> odd, cols, rows;
   int k = odd_pow2(n1, &odd);
-  const int first = (k + 1) / 2, last = k / 2;  // at most 16 each: n1 <= 256
+  const int first = std::min(most, (k + 1) / 2), last = std::min(most, k / 2);
   if (k > 0) cols.push_back(1 << (radix_order == DM_BATCH_RADIX_SMALL_FIRST && last > 0 ? last : first));
+  if (k > first + last) cols.push_back(1 << (k - first - last));  // (n1 <= 256: at most 8 8 4)
   cols.insert(cols.end(), odd.begin(), odd.end());
   if (last > 0) cols.push_back(1 << (radix_order == DM_BATCH_RADIX_SMALL_FIRST ? first : last));
   k = odd_pow2(n2, &rows);
-  for (int left = (k + 3) / 4; left > 0; left--) {
+  for (int left = (k + most - 1) / most; left > 0; left--) {
     const int b = (k + left - 1) / left;
     rows.push_back(1 << b);
     k -= b;
@@ -332,7 +334,7 @@ bool build_batch_host(int count, int ndim, const int *shapes, int dbl, int tile_
       if (it == plane_of.end()) {
         BatchPlane P{};
         std::vector<double> block;
-        make_plane_sched(n1, n2, T, radix_order, &P, &block);
+        make_plane_sched(n1, n2, T, radix_order, k == 0 ? 3 : 4, &P, &block);
         P.tw_off = (int)(h.tw.size() / 2);
         h.tw.insert(h.tw.end(), block.begin(), block.end());
         it = plane_of.emplace(key, (int)h.plane_sched.size()).first;

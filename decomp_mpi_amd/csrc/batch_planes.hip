@@ -5,12 +5,14 @@
 // so an element's offset is its index in the tile.  The columns' first stage
 // runs on the loaded values and their last one before the store (lanes walk
 // contiguous memory in both), the rows' stages between them in LDS: four LDS
-// exchanges for a 64 x 64 plane.  16 points per thread: planes of up to 4096
-// points on 256 threads (several small planes fill a tile), complex-float
-// planes of up to 8192 on 512.  As row stages, then column stages, then a
-// store from LDS, one plane per workgroup, the planes of the 256-transform
-// complex-float batch took 149 and 202 us (3.0 TB/s); 109 and 164 us now (4.0
-// and 3.7 TB/s).
+// exchanges for a 64 x 64 plane.  512 threads: planes of up to 4096 points at
+// 8 points per thread with butterflies of up to 8 (several small planes fill
+// a tile), complex-float planes of up to 8192 at 16.  At 16 points per thread
+// on 256 the small tile's odd radices ran one after another in too few waves:
+// two complex-double 3D transforms of odd lengths 30 us a batch, 27 at 8, and
+// 1126 and 1101 us for 153 of them.  As row stages, then column stages, then
+// a store from LDS, one plane per workgroup, the planes of the 256-transform
+// complex-float batch took 149 and 202 us (3.0 TB/s).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,6 +24,8 @@ namespace dm {
 namespace {
 
 using namespace fftdev;
+
+constexpr int NTH = 512;
 
 template <typename R>
 using gptr = __attribute__((address_space(1))) cx<R> *;  // global memory
@@ -42,9 +46,9 @@ __device__ __forceinline__ BlockStage stage_of(const cplane &S, int i) {
   return st;
 }
 
-template <typename R, bool INV, int RADIX, int NTH>
+template <typename R, bool INV, int RADIX, int PER>
 __device__ __forceinline__ void plane_load(cx<R> *buf, const BlockStage &st, gptr<R> data, int points, int live) {
-  constexpr int K = kPer / RADIX;
+  constexpr int K = (PER + RADIX - 1) / RADIX;
   const int nb = points / RADIX;
   cx<R> v[K][RADIX];
   int e[K], j[K];
@@ -67,10 +71,10 @@ __device__ __forceinline__ void plane_load(cx<R> *buf, const BlockStage &st, gpt
     }
 }
 
-template <typename R, bool INV, int RADIX, int NTH, bool CT>
+template <typename R, bool INV, int RADIX, bool CT, int PER>
 __device__ __forceinline__ void plane_store(const cx<R> *buf, const BlockStage &st, gptr<R> data, int points, int live,
                                             const lds_tw<R, CT> *tw) {
-  constexpr int K = kPer / RADIX;
+  constexpr int K = (PER + RADIX - 1) / RADIX;
   const int nb = points / RADIX;
 #pragma unroll
   for (int k = 0; k < K; k++) {
@@ -94,9 +98,10 @@ __device__ __forceinline__ void plane_store(const cx<R> *buf, const BlockStage &
   }
 }
 
-// MX: schedules with odd radices.  WPS: waves per SIMD that LDS allows.
-template <typename R, bool INV, int NTH, bool MX, int WPS>
-__global__ __launch_bounds__(NTH, WPS) void batch_plane_kernel(BatchLaunch p) {
+// MX: schedules with odd radices.  Two workgroups per CU by LDS, three of
+// complex-float planes of up to 4096 points.
+template <typename R, bool INV, int PER, bool MX>
+__global__ __launch_bounds__(NTH, 4) void batch_plane_kernel(BatchLaunch p) {
   constexpr bool CT = sizeof(R) == 4;  // compensated twiddle products
   typedef typename tw_local<R, CT>::type Tw;
   extern __shared__ __align__(16) char smem[];
@@ -115,22 +120,22 @@ __global__ __launch_bounds__(NTH, WPS) void batch_plane_kernel(BatchLaunch p) {
     if (S.fuse_in) {
       const BlockStage st = stage_of(S, 0);
       switch (st.radix) {
-        case 2: plane_load<R, INV, 2, NTH>(buf, st, data, points, live); break;
-        case 4: plane_load<R, INV, 4, NTH>(buf, st, data, points, live); break;
-        case 8: plane_load<R, INV, 8, NTH>(buf, st, data, points, live); break;
-        case 16: plane_load<R, INV, 16, NTH>(buf, st, data, points, live); break;
+        case 2: plane_load<R, INV, 2, PER>(buf, st, data, points, live); break;
+        case 4: plane_load<R, INV, 4, PER>(buf, st, data, points, live); break;
+        case 8: plane_load<R, INV, 8, PER>(buf, st, data, points, live); break;
+        case 16: if constexpr (PER == 16) plane_load<R, INV, 16, PER>(buf, st, data, points, live); break;
         default: break;
       }
       s0 = 1;
     } else {
-      cx<R> v[kPer];
+      cx<R> v[PER];
 #pragma unroll
-      for (int k = 0; k < kPer; k++) {
+      for (int k = 0; k < PER; k++) {
         const int e = threadIdx.x + k * NTH, at = e < live ? e : 0;
         v[k] = {data[at].x, data[at].y};
       }
 #pragma unroll
-      for (int k = 0; k < kPer; k++) {
+      for (int k = 0; k < PER; k++) {
         const int e = threadIdx.x + k * NTH;
         if (e < points) buf[lds_pad(e)] = v[k];
       }
@@ -139,30 +144,30 @@ __global__ __launch_bounds__(NTH, WPS) void batch_plane_kernel(BatchLaunch p) {
     for (int s = s0; s < s1; s++) {
       const BlockStage st = stage_of(S, s);
       switch (st.radix) {
-        case 2: block_stage<R, INV, 2, NTH, CT>(buf, st, points, tw); break;
-        case 4: block_stage<R, INV, 4, NTH, CT>(buf, st, points, tw); break;
-        case 8: block_stage<R, INV, 8, NTH, CT>(buf, st, points, tw); break;
-        case 16: block_stage<R, INV, 16, NTH, CT>(buf, st, points, tw); break;
-        case 3: if constexpr (MX) block_stage<R, INV, 3, NTH, CT>(buf, st, points, tw); break;
-        case 5: if constexpr (MX) block_stage<R, INV, 5, NTH, CT>(buf, st, points, tw); break;
-        case 7: if constexpr (MX) block_stage<R, INV, 7, NTH, CT>(buf, st, points, tw); break;
-        case 11: if constexpr (MX) block_stage<R, INV, 11, NTH, CT>(buf, st, points, tw); break;
-        case 13: if constexpr (MX) block_stage<R, INV, 13, NTH, CT>(buf, st, points, tw); break;
+        case 2: block_stage<R, INV, 2, NTH, CT, PER>(buf, st, points, tw); break;
+        case 4: block_stage<R, INV, 4, NTH, CT, PER>(buf, st, points, tw); break;
+        case 8: block_stage<R, INV, 8, NTH, CT, PER>(buf, st, points, tw); break;
+        case 16: if constexpr (PER == 16) block_stage<R, INV, 16, NTH, CT, PER>(buf, st, points, tw); break;
+        case 3: if constexpr (MX) block_stage<R, INV, 3, NTH, CT, PER>(buf, st, points, tw); break;
+        case 5: if constexpr (MX) block_stage<R, INV, 5, NTH, CT, PER>(buf, st, points, tw); break;
+        case 7: if constexpr (MX) block_stage<R, INV, 7, NTH, CT, PER>(buf, st, points, tw); break;
+        case 11: if constexpr (MX) block_stage<R, INV, 11, NTH, CT, PER>(buf, st, points, tw); break;
+        case 13: if constexpr (MX) block_stage<R, INV, 13, NTH, CT, PER>(buf, st, points, tw); break;
         default: break;
       }
     }
     if (S.fuse_out) {
       const BlockStage st = stage_of(S, nst - 1);
       switch (st.radix) {
-        case 2: plane_store<R, INV, 2, NTH, CT>(buf, st, data, points, live, tw); break;
-        case 4: plane_store<R, INV, 4, NTH, CT>(buf, st, data, points, live, tw); break;
-        case 8: plane_store<R, INV, 8, NTH, CT>(buf, st, data, points, live, tw); break;
-        case 16: plane_store<R, INV, 16, NTH, CT>(buf, st, data, points, live, tw); break;
+        case 2: plane_store<R, INV, 2, CT, PER>(buf, st, data, points, live, tw); break;
+        case 4: plane_store<R, INV, 4, CT, PER>(buf, st, data, points, live, tw); break;
+        case 8: plane_store<R, INV, 8, CT, PER>(buf, st, data, points, live, tw); break;
+        case 16: if constexpr (PER == 16) plane_store<R, INV, 16, CT, PER>(buf, st, data, points, live, tw); break;
         default: break;
       }
     } else {
 #pragma unroll
-      for (int k = 0; k < kPer; k++) {
+      for (int k = 0; k < PER; k++) {
         const int e = threadIdx.x + k * NTH;
         if (e < live) {
           const cx<R> w = buf[lds_pad(e)];
@@ -175,9 +180,9 @@ __global__ __launch_bounds__(NTH, WPS) void batch_plane_kernel(BatchLaunch p) {
   }
 }
 
-template <typename R, bool INV, int NTH, bool MX, int WPS>
+template <typename R, bool INV, int PER, bool MX>
 hipError_t launch_typed(const BatchLaunch &p, hipStream_t s) {
-  auto k = batch_plane_kernel<R, INV, NTH, MX, WPS>;
+  auto k = batch_plane_kernel<R, INV, PER, MX>;
   // once per kernel (a thread-safe static)
   static const hipError_t attr =
       hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -185,11 +190,11 @@ hipError_t launch_typed(const BatchLaunch &p, hipStream_t s) {
   hipLaunchKernelGGL(k, dim3((unsigned)p.grid), dim3(NTH), p.lds, s, p);
   return hipGetLastError();
 }
-template <typename R, int NTH, int WPS>
+template <typename R, int PER>
 hipError_t launch_forms(const BatchLaunch &p, hipStream_t s) {
   if (p.primes)
-    return p.inverse ? launch_typed<R, true, NTH, true, WPS>(p, s) : launch_typed<R, false, NTH, true, WPS>(p, s);
-  return p.inverse ? launch_typed<R, true, NTH, false, WPS>(p, s) : launch_typed<R, false, NTH, false, WPS>(p, s);
+    return p.inverse ? launch_typed<R, true, PER, true>(p, s) : launch_typed<R, false, PER, true>(p, s);
+  return p.inverse ? launch_typed<R, true, PER, false>(p, s) : launch_typed<R, false, PER, false>(p, s);
 }
 
 constexpr int kSmall = 4096, kLarge = 8192;
@@ -203,21 +208,21 @@ size_t batch_plane_tw_at(int dbl, int points) {
   return ((size_t)(lds_pad(points - 1) + 1) * (dbl ? 16 : 8) + 15) & ~(size_t)15;
 }
 
-// Persistent grids: four 256-thread or two 512-thread workgroups per CU (two
-// of complex double), fewer if LDS says so.
+// Persistent grids: two workgroups per CU by registers, three of
+// complex-float planes of up to 4096 points, fewer if LDS says so.
 long long batch_plane_resident_groups(int dbl, int large, size_t lds) {
   int dev = 0, cus = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (cus <= 0) cus = 256;
-  return (long long)cus * std::max(1, std::min(dbl || large ? 2 : 4, (int)((160 * 1024) / std::max<size_t>(lds, 1))));
+  return (long long)cus * std::max(1, std::min(dbl || large ? 2 : 3, (int)((160 * 1024) / std::max<size_t>(lds, 1))));
 }
 
 int launch_batch_planes(const BatchLaunch &p, void *stream) {
   if (p.ntiles <= 0 || p.grid <= 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  if (p.plane == 1) return p.dbl ? (int)hipErrorInvalidValue : (int)launch_forms<float, 512, 4>(p, s);
-  return (int)(p.dbl ? launch_forms<double, 256, 2>(p, s) : launch_forms<float, 256, 4>(p, s));
+  if (p.plane == 1) return p.dbl ? (int)hipErrorInvalidValue : (int)launch_forms<float, 16>(p, s);
+  return (int)(p.dbl ? launch_forms<double, 8>(p, s) : launch_forms<float, 8>(p, s));
 }
 
 }  // namespace dm

@@ -7,7 +7,7 @@
 namespace dm {
 namespace fftdev {
 
-constexpr int kPer = 16;  // points per thread
+constexpr int kPer = 16;  // points per thread (of most tiles)
 template <typename R, bool CT>
 using lds_tw = __attribute__((address_space(3))) typename tw_local<R, CT>::type;
 
@@ -20,9 +20,9 @@ __device__ __forceinline__ void butterfly(const BlockStage &st, int b, int *base
   *base = outer * st.span + inner;
 }
 
-template <typename R, bool INV, int RADIX, int NTH, bool CT>
+template <typename R, bool INV, int RADIX, int NTH, bool CT, int PER = kPer>
 __device__ __forceinline__ void block_stage(cx<R> *buf, const BlockStage &st, int points, const lds_tw<R, CT> *tw) {
-  constexpr int K = (kPer + RADIX - 1) / RADIX;
+  constexpr int K = (PER + RADIX - 1) / RADIX;
   const int nb = points / RADIX;
   cx<R> v[K][RADIX];
   int dst[K];

@@ -306,7 +306,8 @@ struct BatchLaunch {
   int dbl, inverse;
   int primes;                  // some schedule has a radix 5, 7, 11 or 13
   int long_lines;              // some schedule's lines are too long for twiddles in LDS
-  int plane;                   // plane tiles (row 2) only: 2 up to batch_plane_small() points, 1 larger
+  int plane;                   // plane tiles (row 2) only: 2 up to batch_plane_small() points (butterflies of
+                               //   up to 8), 1 larger
   const BatchPlane *planes;    // their schedules
   int plane_tw;                // LDS offset of their twiddles
   int any;                     // some schedule has a direct-sum stage (line tiles only)
@@ -353,8 +354,8 @@ size_t batch_lds_bytes(int dbl, int T, int N);
 bool batch_tw_in_lds(int N);
 long long batch_resident_groups(int dbl, int primes, size_t lds);
 // Plane tiles (BatchTile row 2): the most points a plane may hold, the most
-// a plane of the 256-thread kernel may, the LDS offset of a tile's twiddles,
-// and the resident workgroups for a launch's LDS.
+// a plane of the small tile may, the LDS offset of a tile's twiddles, and
+// the resident workgroups for a launch's LDS.
 int batch_plane_capacity(int dbl);
 int batch_plane_small();
 size_t batch_plane_tw_at(int dbl, int points);
