@@ -318,6 +318,20 @@ bool build_batch_host(int count, int ndim, const int *shapes, int dbl, int tile_
     return id;
   };
   h.tiles.assign(ndim, std::vector<BatchTile>());
+  // Points of a tile of several small planes: a tile for each of the 256 CUs
+  // before any is filled, a point for each of its 512 threads at least (20 x
+  // 100 x 143 and 22 x 25 x 18 complex doubles: 46.1 us with full tiles, 40.4
+  // so; 5 of 45 x 60 and smaller planes 66.7 and 64.4; at a thousand tiles 19
+  // transforms lose, 97.0 and 99.9).
+  long long small_points = 0;
+  for (int i = 0; i < count && tile_choice == DM_BATCH_TILE_PLANES && ndim >= 2; i++) {
+    const int *n = &shapes[(size_t)i * ndim];
+    if (!plane_fits(n[ndim - 2], n[ndim - 1], dbl) || n[ndim - 2] * n[ndim - 1] > batch_plane_small()) continue;
+    long long points = 1;
+    for (int d = 0; d < ndim; d++) points *= n[d];
+    small_points += points;
+  }
+  const int tile_points = (int)std::min<long long>(std::max(small_points / 256, 512LL), batch_plane_small());
   std::map<std::tuple<int, int, int>, int> plane_of;  // (n1, n2, T) -> plane schedule
   int plane_ntw[2] = {0, 0};
   for (int i = 0; i < count; i++) {
@@ -328,7 +342,7 @@ bool build_batch_host(int count, int ndim, const int *shapes, int dbl, int tile_
       long long outer = 1;
       for (int e = 0; e < ndim - 2; e++) outer *= n[e];
       const int k = plane <= batch_plane_small() ? 0 : 1;
-      const int T = (int)std::min<long long>(outer, (k == 0 ? batch_plane_small() : plane) / plane);
+      const int T = (int)std::min<long long>(outer, std::max(k == 0 ? tile_points : 0, plane) / plane);
       const auto key = std::make_tuple(n1, n2, T);
       auto it = plane_of.find(key);
       if (it == plane_of.end()) {
