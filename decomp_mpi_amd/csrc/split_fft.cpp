@@ -840,12 +840,13 @@ static bool compile_phased(SplitPlan plan) {
     // 256-thread workgroups: one chunk of one row (the last axis) each, or
     // several whole rows when the rows are shorter (the kernel's mapping)
     const int block = 256;
-    long long max_blocks = 0;
+    long long max_blocks = 0, all_rows = 0;
     for (int r = 0; r < nr; r++) {
       long long rows = 1;
       for (int d = 0; d < nd - 1; d++) rows *= rt[((size_t)r * nd + d) * 2 + 1];
       const long long inner = rt[((size_t)r * nd + nd - 1) * 2 + 1];
       if (rows <= 0 || inner <= 0) continue;  // a rank with an empty block
+      all_rows += rows;
       const long long need = inner >= block ? rows * ((inner + block - 1) / block)
                                             : (rows + block / inner - 1) / (block / inner);
       max_blocks = std::max(max_blocks, need);
@@ -855,7 +856,7 @@ static bool compile_phased(SplitPlan plan) {
     // reference's recursion forms it
     std::vector<double> rows_tab;
     std::vector<long long> row_off(nr, 0);
-    rows_tab.reserve(2 * (size_t)max_elems);
+    rows_tab.reserve(2 * (size_t)all_rows);
     for (int r = 0; r < nr; r++) {
       long long rows = 1;
       for (int d = 0; d < nd - 1; d++) rows *= rt[((size_t)r * nd + d) * 2 + 1];
