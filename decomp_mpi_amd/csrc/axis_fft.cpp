@@ -8,6 +8,7 @@
 // transform along `axis`, write the output decomposition.
 #include <algorithm>
 #include <cstring>
+#include <new>
 
 #include "internal.h"
 #include "fft_program.h"
@@ -56,6 +57,45 @@ extern "C" void dm_free_axis_fft(struct dm_axis_fft *p) {
   delete p;
 }
 
+// The pass for these buffers (offsets oi, oo in bi, bo).
+static bool compile_axis(dm_axis_fft *p, const void *in, void *out, const dm::Buffer &bi, size_t oi, const dm::Buffer &bo,
+                         size_t oo) {
+  dm_comm_t comm = p->in->comm;
+  const size_t es = p->dbl ? 16 : 8;
+  if (p->mem) dm::device_free(p->mem);
+  p->mem = nullptr;
+  dm::HostLayout hi = dm::layout_from_decomp(p->in), ho = dm::layout_from_decomp(p->out);
+  if (bi.nranks < hi.proc_used || bo.nranks < ho.proc_used) {
+    raise_error(comm, "dm_run_axis_fft: buffers have fewer rank slots than the decompositions use");
+    return false;
+  }
+  size_t ri = (bi.slot - oi) / es, ro = (bo.slot - oo) / es;
+  if (!dm::layout_usable(comm, "input", hi, ri) || !dm::layout_usable(comm, "output", ho, ro)) return false;
+  if (bi.base == bo.base) {
+    size_t ei = 0, eo = 0;
+    for (auto e : hi.slot_extent) ei = std::max(ei, (size_t)e * es);
+    for (auto e : ho.slot_extent) eo = std::max(eo, (size_t)e * es);
+    bool overlap = oi < oo + eo && oo < oi + ei;
+    // in place is safe only when both sides are the same layout: every
+    // tile then writes exactly the addresses it read
+    if (overlap && !(oi == oo && equivalent(p->in, p->out))) {
+      raise_error(comm, "dm_run_axis_fft: input and output overlap with different layouts");
+      return false;
+    }
+  }
+  dm::Side si = dm::make_side(hi, (i64)(bi.slot / es)), so = dm::make_side(ho, (i64)(bo.slot / es));
+  dm::TableBuilder tb;
+  std::vector<dm::PendingPass> pp(1);
+  if (!dm::plan_pass(comm, si, so, p->axis, p->dbl, p->inverse, bi.base + oi, bo.base + oo, tb, &pp[0])) return false;
+  p->mem = dm::finalize_passes(comm, tb, pp, &p->passes);
+  if (p->mem == nullptr) return false;
+  p->in_ptr = in;
+  p->out_ptr = out;
+  p->in_slot = bi.slot;
+  p->out_slot = bo.slot;
+  return true;
+}
+
 extern "C" int dm_run_axis_fft(struct dm_axis_fft *p, const void *in, void *out) {
   if (p == nullptr) return DM_ERR_ARG;
   dm_comm_t comm = p->in->comm;
@@ -73,38 +113,12 @@ extern "C" int dm_run_axis_fft(struct dm_axis_fft *p, const void *in, void *out)
   }
   if (p->mem == nullptr || p->in_ptr != in || p->out_ptr != out || p->in_slot != bi.slot ||
       p->out_slot != bo.slot) {
-    if (p->mem) dm::device_free(p->mem);
-    p->mem = nullptr;
-    dm::HostLayout hi = dm::layout_from_decomp(p->in), ho = dm::layout_from_decomp(p->out);
-    if (bi.nranks < hi.proc_used || bo.nranks < ho.proc_used) {
-      raise_error(comm, "dm_run_axis_fft: buffers have fewer rank slots than the decompositions use");
+    try {
+      if (!compile_axis(p, in, out, bi, oi, bo, oo)) return DM_ERR_ARG;
+    } catch (const std::bad_alloc &) {
+      raise_error(comm, "dm_run_axis_fft: no host memory for the pass's tables");
       return DM_ERR_ARG;
     }
-    size_t ri = (bi.slot - oi) / es, ro = (bo.slot - oo) / es;
-    if (!dm::layout_usable(comm, "input", hi, ri) || !dm::layout_usable(comm, "output", ho, ro)) return DM_ERR_ARG;
-    if (bi.base == bo.base) {
-      size_t ei = 0, eo = 0;
-      for (auto e : hi.slot_extent) ei = std::max(ei, (size_t)e * es);
-      for (auto e : ho.slot_extent) eo = std::max(eo, (size_t)e * es);
-      bool overlap = oi < oo + eo && oo < oi + ei;
-      // in place is safe only when both sides are the same layout: every
-      // tile then writes exactly the addresses it read
-      if (overlap && !(oi == oo && equivalent(p->in, p->out))) {
-        raise_error(comm, "dm_run_axis_fft: input and output overlap with different layouts");
-        return DM_ERR_ARG;
-      }
-    }
-    dm::Side si = dm::make_side(hi, (i64)(bi.slot / es)), so = dm::make_side(ho, (i64)(bo.slot / es));
-    dm::TableBuilder tb;
-    std::vector<dm::PendingPass> pp(1);
-    if (!dm::plan_pass(comm, si, so, p->axis, p->dbl, p->inverse, bi.base + oi, bo.base + oo, tb, &pp[0]))
-      return DM_ERR_ARG;
-    p->mem = dm::finalize_passes(comm, tb, pp, &p->passes);
-    if (p->mem == nullptr) return DM_ERR_ARG;
-    p->in_ptr = in;
-    p->out_ptr = out;
-    p->in_slot = bi.slot;
-    p->out_slot = bo.slot;
   }
   void *s = dm::world_stream(comm->world);
   for (auto &L : p->passes)

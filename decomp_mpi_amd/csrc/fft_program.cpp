@@ -159,8 +159,8 @@ static bool is_identity(const std::vector<int> &o) {
   return true;
 }
 
-bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, bool inverse, const void *in,
-               void *out, TableBuilder &tb, PendingPass *pp, int ctw) {
+static bool plan_pass_tables(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, bool inverse,
+                             const void *in, void *out, TableBuilder &tb, PendingPass *pp, int ctw) {
   int nd = I.h.ndim;
   FftLaunch &L = pp->L;
   memset(&L, 0, sizeof L);
@@ -455,6 +455,16 @@ bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, boo
   return true;
 }
 
+bool plan_pass(dm_comm_t comm, const Side &I, const Side &U, int t, int dbl, bool inverse, const void *in,
+               void *out, TableBuilder &tb, PendingPass *pp, int ctw) {
+  try {
+    return plan_pass_tables(comm, I, U, t, dbl, inverse, in, out, tb, pp, ctw);
+  } catch (const std::bad_alloc &) {  // the callers are C entry points
+    raise_error(comm, "FFT: no host memory for the tables of the pass over axis %d", t);
+    return false;
+  }
+}
+
 // Radices of a block pass stage by stage: powers of two in 16s, 8s and 4s
 // (a 16-point axis is one butterfly of a thread's 16 points).
 static bool block_radices(int n, std::vector<int> *out) {
@@ -539,8 +549,8 @@ bool block_fits(const Side &I, const Side &U, const std::vector<int> &axes, int 
   return total / points * 16 <= (64LL << 20);  // the line bases
 }
 
-bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int dbl, bool inverse, const void *in,
-                void *out, TableBuilder &tb, PendingBlock *pb, int ctw, int wq) {
+static bool plan_block_tables(const Side &I, const Side &U, const std::vector<int> &axes, int dbl, bool inverse,
+                              const void *in, void *out, TableBuilder &tb, PendingBlock *pb, int ctw, int wq) {
   FftBlock &B = pb->B;
   memset(&B, 0, sizeof B);
   const int nd = I.h.ndim;
@@ -691,6 +701,15 @@ bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int 
   B.out = out;
   fft_block_lds(&B);
   return B.lds <= 160 * 1024 && B.tiles < (1LL << 31);
+}
+
+bool plan_block(const Side &I, const Side &U, const std::vector<int> &axes, int dbl, bool inverse, const void *in,
+                void *out, TableBuilder &tb, PendingBlock *pb, int ctw, int wq) {
+  try {
+    return plan_block_tables(I, U, axes, dbl, inverse, in, out, tb, pb, ctw, wq);
+  } catch (const std::bad_alloc &) {
+    return false;
+  }
 }
 
 void *finalize_passes(dm_comm_t comm, TableBuilder &tb, std::vector<PendingPass> &pp,

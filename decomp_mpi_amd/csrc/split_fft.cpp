@@ -24,6 +24,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <memory>
+#include <new>
 #include <numeric>
 #include <string>
 
@@ -1434,11 +1435,17 @@ static void run_split(SplitPlan plan, int direction) {
   }
   dm::check_device(plan->comm);
   if (dm::error_pending() && dm::error_mode() == 1) return;
+  bool ready = false;
+  try {
+    ready = plan->ext->phased ? compile_phased(plan) : compile_plan(plan);
+  } catch (const std::bad_alloc &) {
+    raise_error(plan->comm, "runSplitPlan: no host memory for the plan's tables");
+  }
+  if (!ready) return;
   if (plan->ext->phased) {
-    if (compile_phased(plan)) run_phased(plan, direction);
+    run_phased(plan, direction);
     return;
   }
-  if (!compile_plan(plan)) return;
   if (direction == FFTW_FORWARD) run_program(plan, plan->ext->fwd, FFT_1, FFT_2);
   else run_program(plan, plan->ext->bwd, FFT_2, FFT_1);
 }

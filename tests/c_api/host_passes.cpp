@@ -2,6 +2,9 @@
 // planned from real decompositions through the library's own internal
 // headers, and what a launch would ask for is checked here.
 // Usage: host_passes <check>; prints OK.
+#include <sys/resource.h>
+#include <unistd.h>
+
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -112,12 +115,44 @@ static void reshape() {
             }
 }
 
+// Planning under a limit on the address space: an error, not an exception
+// through the C interface.
+static void memory() {
+  const Layout many({1 << 20, 4, 1}, {1, 1, 1});
+  const dm::Side t = many.side();
+  struct rlimit lim;
+  getrlimit(RLIMIT_AS, &lim);
+  const struct rlimit before = lim;
+  FILE *f = fopen("/proc/self/statm", "r");
+  long pages = 0;
+  if (f == nullptr || fscanf(f, "%ld", &pages) != 1) failures++;
+  if (f != nullptr) fclose(f);
+  lim.rlim_cur = (rlim_t)pages * sysconf(_SC_PAGESIZE) + (4 << 20);  // 4 MiB more than now
+  setrlimit(RLIMIT_AS, &lim);
+  {
+    dm::TableBuilder tb;
+    dm::PendingPass pp;
+    // 2^20 lines of 4 points: 16 MiB of line bases
+    if (dm::plan_pass(many.comm, t, t, 1, 1, false, nullptr, nullptr, tb, &pp) || !dm::error_pending()) {
+      printf("a pass was planned within 4 MiB, or without an error\n");
+      failures++;
+    }
+    dm::PendingBlock pb;
+    if (dm::plan_block(t, t, {1}, 1, false, nullptr, nullptr, tb, &pb, 1)) {
+      printf("a block pass was planned within 4 MiB\n");
+      failures++;
+    }
+  }
+  setrlimit(RLIMIT_AS, &before);
+}
+
 int main(int argc, char **argv) {
   dm_set_error_mode(1);
   const std::string check = argc > 1 ? argv[1] : "";
   if (check == "lds") lds();
   else if (check == "tables") tables();
   else if (check == "reshape") reshape();
+  else if (check == "memory") memory();
   else return 2;
   if (failures == 0) printf("OK\n");
   return failures != 0;

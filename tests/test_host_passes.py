@@ -42,3 +42,8 @@ def test_table_bytes(driver):
 def test_reshape_tile_lds(driver):
     """No reshape tile asks for more than 64 KiB of LDS."""
     run(driver, "reshape")
+
+
+def test_out_of_host_memory(driver):
+    """Tables that do not fit in memory make an error, not an exception."""
+    run(driver, "memory")
