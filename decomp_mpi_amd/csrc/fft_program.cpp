@@ -125,7 +125,7 @@ bool axis_supported(int n, int dbl, std::string *why) {
     snprintf(msg, sizeof msg, "axis length %d exceeds the %d-point tile of the %s pass", n, cap,
              dbl ? "complex-double" : "complex-float");
   } else if (!choose_radices(n, &rad, true) || (int)rad.size() > kMaxStages) {
-    snprintf(msg, sizeof msg, "axis length %d has more than 16 prime factors", n);
+    snprintf(msg, sizeof msg, "axis length %d takes more than %d stages", n, kMaxStages);
   } else {
     return true;
   }
@@ -175,7 +175,7 @@ static bool plan_pass_tables(dm_comm_t comm, const Side &I, const Side &U, int t
   }
   std::vector<int> rad;
   if (!choose_radices(L.N, &rad, true) || (int)rad.size() > kMaxStages) {
-    raise_error(comm, "FFT: axis length %d has more than 16 prime factors", L.N);
+    raise_error(comm, "FFT: axis length %d takes more than %d stages", L.N, kMaxStages);
     return false;
   }
   L.nstage = (int)rad.size();

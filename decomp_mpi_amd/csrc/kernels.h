@@ -97,10 +97,11 @@ struct FftSide {
   const i64 *strides;          // [proc_used * ndim]
 };
 
-// Most stages of a pass: a line has at most 8192 = 3^8 + ... points, and two
-// factors of two or more share a stage.  (Kernel arguments are copied and
-// fetched with every launch: 1.3 KiB of them cost a 64^3 pencil pass, three
-// launches, 0.5 us each against 0.8 KiB.)
+// Most stages of a pass: no length within a tile (8192 points) takes more
+// (6561 = 3^8 and 4374 = 2 * 3^7 take 8; factors of two share stages of three
+// or four).  Kernel arguments are copied and fetched with every launch: 1.3
+// KiB of them cost a 64^3 pencil pass, three launches, 0.5 us each against
+// 0.8 KiB.
 constexpr int kMaxStages = 8;
 
 struct FftLaunch {

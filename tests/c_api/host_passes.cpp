@@ -146,6 +146,21 @@ static void memory() {
   setrlimit(RLIMIT_AS, &before);
 }
 
+// Every line length within a tile: a schedule of its stages that fits the
+// launch arguments and multiplies to the length.
+static void stages() {
+  for (int n = 1; n <= dm::fft_tile_capacity(0, 1); n++) {
+    std::vector<int> rad;
+    long long m = 1;
+    const bool ok = dm::choose_radices(n, &rad, true);
+    for (int r : rad) m *= r;
+    if (!ok || m != n || (int)rad.size() > dm::kMaxStages) {
+      printf("length %d: %zu stages\n", n, rad.size());
+      failures++;
+    }
+  }
+}
+
 int main(int argc, char **argv) {
   dm_set_error_mode(1);
   const std::string check = argc > 1 ? argv[1] : "";
@@ -153,6 +168,7 @@ int main(int argc, char **argv) {
   else if (check == "tables") tables();
   else if (check == "reshape") reshape();
   else if (check == "memory") memory();
+  else if (check == "stages") stages();
   else return 2;
   if (failures == 0) printf("OK\n");
   return failures != 0;

@@ -47,3 +47,8 @@ def test_reshape_tile_lds(driver):
 def test_out_of_host_memory(driver):
     """Tables that do not fit in memory make an error, not an exception."""
     run(driver, "memory")
+
+
+def test_stages(driver):
+    """No length within a tile takes more stages than a launch holds."""
+    run(driver, "stages")
