@@ -409,7 +409,7 @@ static bool plan_pass_tables(dm_comm_t comm, const Side &I, const Side &U, int t
   // radix R) holds w^(jj * r * N / (Ns * R)) for r = 1..R-1, jj < Ns at
   // index (Ns - 1) + (r - 1) * Ns + jj, so the lanes of a wave (consecutive
   // jj) read consecutive entries.  The stages telescope to N - 1 entries.
-  std::vector<double> root = roots(L.N);
+  const std::vector<double> &root = tb.root->of(L.N);
   std::vector<double> w(2 * (size_t)L.N, 0.0);
   {
     int ns = 1;
@@ -603,7 +603,7 @@ static bool plan_block_tables(const Side &I, const Side &U, const std::vector<in
     std::vector<int> rad;
     block_radices(n, &rad);
     if (a == 0 && rad.size() > 1 && (rad[0] & (rad[0] - 1)) != 0) std::reverse(rad.begin(), rad.end());
-    const std::vector<double> root = roots(n);
+    const std::vector<double> &root = tb.root->of(n);
     int ns = 1;
     for (int r : rad) {
       BlockStage st{};
@@ -687,7 +687,7 @@ static bool plan_block_tables(const Side &I, const Side &U, const std::vector<in
     B.wdiv = 1;
     for (auto k = at + 1; k != batch.end(); ++k) B.wdiv *= I.h.L[*k];
     const int N = B.wn * B.wlen;
-    const std::vector<double> w = roots(N);
+    const std::vector<double> &w = tb.root->of(N);
     std::vector<char> wi((size_t)N * 16);
     twiddle_image(w.data(), N, dbl, wi.data());
     pb->wtab = (long)tb.put(wi.data(), wi.size());

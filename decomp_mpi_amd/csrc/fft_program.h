@@ -2,6 +2,7 @@
 // per-axis FFT and the batched transforms).
 #pragma once
 #include <cstdlib>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -33,8 +34,22 @@ std::vector<double> roots(int n);
 // third word; the fourth word is 0).
 void twiddle_image(const double *w, size_t n, int dbl, void *dst);
 
+// roots(n) of the lengths asked for, each formed once (4096 of them take 0.75
+// ms, the better part of a small plan's first call).
+struct RootTables {
+  std::map<int, std::vector<double>> made;
+  const std::vector<double> &of(int n) {
+    std::vector<double> &w = made[n];
+    if (w.empty()) w = roots(n);
+    return w;
+  }
+};
+
 // Host image of the device tables of a program.
 struct TableBuilder {
+  TableBuilder() = default;
+  explicit TableBuilder(RootTables &shared) : root(&shared) {}
+  RootTables own, *root = &own;
   // Grown by realloc and not cleared: the line bases of a 512^3 program are
   // tens of megabytes.
   struct Image {

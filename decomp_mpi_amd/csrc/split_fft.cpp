@@ -362,7 +362,7 @@ static int long_factor(int n, int dbl, i64 stride, int row_bytes) {
 // place.
 static bool compile_split_axes(SplitPlan plan, bool inverse, const dm::Side &first, const dm::Side &last,
                                const std::vector<int> &axes, void *src, void *dst, void *w1, int slots,
-                               i64 wslot, dm_fft_program *prog) {
+                               i64 wslot, dm::RootTables &roots, dm_fft_program *prog) {
   dm_split_ext *x = plan->ext;
   const int nd = x->ndim, f = first.h.fastest;
   if (!first.h.uniform || !last.h.uniform || last.h.fastest != f || axes.size() < 2 || x->L[f] < 16) return false;
@@ -411,7 +411,7 @@ static bool compile_split_axes(SplitPlan plan, bool inverse, const dm::Side &fir
     h.rank_part[fs][U.order[fs][i]] = owner[i];
   }
   const dm::Side M = dm::make_side(h, wslot);
-  dm::TableBuilder tb;
+  dm::TableBuilder tb(roots);
   std::vector<dm::PendingPass> pp;
   std::vector<dm::PendingBlock> pb;
   // the passes: f, then the others by stride (a split axis: z, then y)
@@ -459,7 +459,7 @@ static bool compile_split_axes(SplitPlan plan, bool inverse, const dm::Side &fir
 // tiles are disjoint, and such a pass reads and writes one layout).
 // slots: rank slots of the workspace buffer.
 static bool compile_direction(SplitPlan plan, bool inverse, const dm::Side &S, const dm::Side &O, void *dat,
-                              void *w0, void *w1, int slots, dm_fft_program *prog) {
+                              void *w0, void *w1, int slots, dm::RootTables &roots, dm_fft_program *prog) {
   dm_split_ext *x = plan->ext;
   int nd = x->ndim;
   std::vector<int> axes;
@@ -525,7 +525,7 @@ static bool compile_direction(SplitPlan plan, bool inverse, const dm::Side &S, c
       order = fallback_order();
     }
   }
-  dm::TableBuilder tb;
+  dm::TableBuilder tb(roots);
   // Small arrays: every axis in one block pass, or the two fastest in one
   // and the third in a line pass over rows of the first (one pass less: a 16^3
   // forward on 4 ranks 49 -> 24 us, 400 x 60 x 60 complex double forward and
@@ -544,7 +544,7 @@ static bool compile_direction(SplitPlan plan, bool inverse, const dm::Side &S, c
       return prog->mem != nullptr;
     };
     memset(&pp[0].L, 0, sizeof pp[0].L);
-    if (compile_split_axes(plan, inverse, first, last, axes, src, dst, w1, slots, wslot, prog)) return true;
+    if (compile_split_axes(plan, inverse, first, last, axes, src, dst, w1, slots, wslot, roots, prog)) return true;
     if (n >= 2 && dm::block_fits(first, last, axes, x->dbl) &&
         dm::plan_block(first, last, axes, x->dbl, inverse, src, dst, tb, &pb[0], x->ctw))
       return finish();
@@ -647,12 +647,16 @@ static bool bind_buffers(SplitPlan plan, dm::Buffer *bd, size_t *od, dm::Buffer 
   return true;
 }
 
-// Build the fused programs of both directions, if they are not there yet: a
-// first run in one direction leaves nothing to allocate or copy for the other
-// (which a caller may then record into a graph).
-static bool compile_plan(SplitPlan plan) {
+// Build the fused programs, the given direction's first, and call `between`
+// once that one is there.  Both are built for the first run of either, so
+// that it leaves nothing to allocate or copy for the other (which a caller
+// may then record into a graph).
+static bool compile_plan(SplitPlan plan, bool inverse, const std::function<void()> &between) {
   dm_split_ext *x = plan->ext;
-  if (x->fwd.mem != nullptr && x->bwd.mem != nullptr) return true;
+  if (x->fwd.mem != nullptr && x->bwd.mem != nullptr) {
+    between();
+    return true;
+  }
   if (!x->fused_ok) {
     raise_error(plan->comm, "split FFT: an axis is longer than one pass tile; this plan runs in phase order only");
     return false;
@@ -669,10 +673,14 @@ static bool compile_plan(SplitPlan plan) {
   char *dat = bd.base + od;
   char *w0 = bw.base + ow;
   char *w1 = w0 + ext * es;
-  for (bool inverse : {false, true}) {
-    dm_fft_program &prog = inverse ? x->bwd : x->fwd;
-    if (prog.mem == nullptr && !compile_direction(plan, inverse, S, O, dat, w0, w1, bw.nranks, &prog)) return false;
-  }
+  dm::RootTables roots;
+  auto build = [&](bool inv) {
+    dm_fft_program &prog = inv ? x->bwd : x->fwd;
+    return prog.mem != nullptr || compile_direction(plan, inv, S, O, dat, w0, w1, bw.nranks, roots, &prog);
+  };
+  if (!build(inverse)) return false;
+  between();
+  if (!build(!inverse)) return false;
   plan->plan_a = &x->fwd;
   plan->plan_b_back = &x->bwd;
   return true;
@@ -1223,7 +1231,7 @@ static double model_cost(SplitPlan p) {
 // Milliseconds of a forward + backward step of plan p (the backward
 // overwrites dat: the caller saves it).
 static double time_plan(SplitPlan p, int reps) {
-  if (p->ext->phased ? !compile_phased(p) : !compile_plan(p)) return 1e30;
+  if (p->ext->phased ? !compile_phased(p) : !compile_plan(p, false, [] {})) return 1e30;
   void *s = dm::world_stream(p->comm->world);
   hipEvent_t e0, e1;
   (void)hipEventCreate(&e0);
@@ -1362,39 +1370,48 @@ static SplitPlan autotune_search(int dbl, Decomp start, void *dat, int length, v
 
 // ---------------------------------------------------------------- executor
 
-static void run_program(SplitPlan plan, dm_fft_program &prog, int t_first, int t_rest) {
-  dm_world *w = plan->comm->world;
-  void *s = dm::world_stream(w);
-  size_t n = prog.passes.size();
-  bool timed = !w->async;
-  std::vector<hipEvent_t> ev;
-  if (timed) {
-    ev.resize(n + 1);
-    for (auto &e : ev) (void)hipEventCreate(&e);
-    (void)hipEventRecord(ev[0], (hipStream_t)s);
-  }
+// One run of a program: its passes enqueued; waited for, and their times
+// added, where the world is synchronous.
+struct ProgramRun {
+  SplitPlan plan;
+  dm_fft_program &prog;
+  int t_first, t_rest;
+  std::vector<hipEvent_t> ev = {};
   bool ok = true;
-  for (size_t i = 0; i < n && ok; i++) {
-    ok = launch_pass(plan->comm, prog, i, s);
-    if (timed) (void)hipEventRecord(ev[i + 1], (hipStream_t)s);
+
+  void enqueue() {
+    void *s = dm::world_stream(plan->comm->world);
+    const size_t n = prog.passes.size();
+    const bool timed = !plan->comm->world->async;
+    if (timed) {
+      ev.resize(n + 1);
+      for (auto &e : ev) (void)hipEventCreate(&e);
+      (void)hipEventRecord(ev[0], (hipStream_t)s);
+    }
+    for (size_t i = 0; i < n && ok; i++) {
+      ok = launch_pass(plan->comm, prog, i, s);
+      if (timed) (void)hipEventRecord(ev[i + 1], (hipStream_t)s);
+    }
   }
-  if (!timed) return;
-  if (!ok) {
-    (void)hipStreamSynchronize((hipStream_t)s);
+  void finish() {
+    if (ev.empty()) return;
+    const size_t n = prog.passes.size();
+    if (ok) {
+      (void)hipEventSynchronize(ev[n]);
+      double total = 0;
+      for (size_t i = 0; i < n; i++) {
+        float ms = 0;
+        (void)hipEventElapsedTime(&ms, ev[i], ev[i + 1]);
+        plan->times[prog.passes[i].pass_index == 0 ? t_first : t_rest] += ms * 1e-3;
+        total += ms * 1e-3;
+      }
+      plan->times[ALL] += total;
+    } else {
+      (void)hipStreamSynchronize((hipStream_t)dm::world_stream(plan->comm->world));
+    }
     for (auto &e : ev) (void)hipEventDestroy(e);
-    return;
   }
-  (void)hipEventSynchronize(ev[n]);
-  double total = 0;
-  for (size_t i = 0; i < n; i++) {
-    float ms = 0;
-    (void)hipEventElapsedTime(&ms, ev[i], ev[i + 1]);
-    plan->times[prog.passes[i].pass_index == 0 ? t_first : t_rest] += ms * 1e-3;
-    total += ms * 1e-3;
-  }
-  plan->times[ALL] += total;
-  for (auto &e : ev) (void)hipEventDestroy(e);
-}
+};
 
 // split_fft.c:622-744.  Forward: start layout in dat -> output layout in
 // work.  Backward: the exact (unnormalised) inverse, output layout in work ->
@@ -1435,19 +1452,19 @@ static void run_split(SplitPlan plan, int direction) {
   }
   dm::check_device(plan->comm);
   if (dm::error_pending() && dm::error_mode() == 1) return;
-  bool ready = false;
+  const bool inverse = direction == FFTW_BACKWARD;
+  // (a first run's passes go out before the other direction's are built)
+  ProgramRun run{plan, inverse ? plan->ext->bwd : plan->ext->fwd, inverse ? FFT_2 : FFT_1, inverse ? FFT_1 : FFT_2};
   try {
-    ready = plan->ext->phased ? compile_phased(plan) : compile_plan(plan);
+    if (plan->ext->phased) {
+      if (compile_phased(plan)) run_phased(plan, direction);
+      return;
+    }
+    compile_plan(plan, inverse, [&] { run.enqueue(); });
   } catch (const std::bad_alloc &) {
     raise_error(plan->comm, "runSplitPlan: no host memory for the plan's tables");
   }
-  if (!ready) return;
-  if (plan->ext->phased) {
-    run_phased(plan, direction);
-    return;
-  }
-  if (direction == FFTW_FORWARD) run_program(plan, plan->ext->fwd, FFT_1, FFT_2);
-  else run_program(plan, plan->ext->bwd, FFT_2, FFT_1);
+  run.finish();
 }
 
 extern "C" int dm_split_set_output(SplitPlan plan, Decomp out) {
