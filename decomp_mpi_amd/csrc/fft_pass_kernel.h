@@ -87,7 +87,7 @@ struct LineAddr<true> {
 // 126 x 100 complex-double transform on 6 ranks took 43, 43 and 25 us, 129
 // us for the whole call; 86 us with a base and a stride per line and
 // position, dense intermediates and two workgroups per CU.  It is left for
-// lines over many positions (FftSide::far): LDS holds the line's owner
+// lines over many positions (FftSide::form 2): LDS holds the line's owner
 // contribution and its local offsets then.
 template <>
 struct LineAddr<false> {
@@ -96,7 +96,7 @@ struct LineAddr<false> {
   lds_i64 *str;
   int np;
   __host__ __device__ static size_t bytes(int T, const FftSide &s) {
-    return s.far ? (size_t)T * kFar * sizeof(int) : (size_t)T * s.np * 2 * sizeof(i64);
+    return s.form == 2 ? (size_t)T * kFar * sizeof(int) : (size_t)T * s.np * 2 * sizeof(i64);
   }
   __device__ void init(char *mem, int T, int n) {
     base = (lds_i64 *)(mem);
@@ -108,7 +108,7 @@ struct LineAddr<false> {
     int R0 = 0;
     for (int d = 0; d < p.ndim; d++)
       if (d != p.t) R0 += s.rank[p.at[d] + g[d]];
-    if (s.far) {
+    if (s.form == 2) {
       lds_int *line = (lds_int *)base + l * kFar;
       line[0] = R0;
       for (int d = 0; d < p.ndim; d++) line[1 + d] = d != p.t ? s.off[p.at[d] + g[d]] : 0;
@@ -130,16 +130,31 @@ struct LineAddr<false> {
     const int R = line[0] + s.rank[p.at[p.t] + x];
     const i64 *m = s.strides + (i64)R * p.ndim;
     i64 a = (i64)R * s.slot + m[p.t] * s.off[p.at[p.t] + x];
+#pragma unroll 1
     for (int d = 0; d < p.ndim; d++) a += m[d] * line[1 + d];
     return a;
   }
-  __device__ __forceinline__ i64 at(const FftLaunch &p, const FftSide &s, const i64 *, int l, int x) const {
-    if (s.lin) return base[l] + (i64)x * str[l];  // axis t local to every rank, in order
-    if (s.far) return far(p, s, l, x);
-    const int k = l * np + s.xt[2 * x];
-    return base[k] + (i64)s.xt[2 * x + 1] * str[k];
+  // the point in a given form (FftSide::form)
+  template <int FORM>
+  __device__ __forceinline__ i64 at_form(const FftLaunch &p, const FftSide &s, int l, int x) const {
+    if constexpr (FORM == 1) return base[l] + (i64)x * str[l];  // axis t local to every rank, in order
+    else if constexpr (FORM == 2) return far(p, s, l, x);
+    else {
+      const int k = l * np + s.xt[2 * x];
+      return base[k] + (i64)s.xt[2 * x + 1] * str[k];
+    }
   }
 };
+
+// f(a point's offset as a function of line and point) for a non-uniform
+// side's lines; the form is chosen once, around f's loops (a choice per point
+// cost the pencils of uneven ranks 4 to 10%).
+template <typename F>
+__device__ __forceinline__ void with_points(const LineAddr<false> &la, const FftLaunch &p, const FftSide &s, F f) {
+  if (s.form == 2) f([&](int l, int x) { return la.template at_form<2>(p, s, l, x); });
+  else if (s.form == 1) f([&](int l, int x) { return la.template at_form<1>(p, s, l, x); });
+  else f([&](int l, int x) { return la.template at_form<0>(p, s, l, x); });
+}
 
 // Tile t -> (tile along u, batch coordinates); fills the per-line address
 // data of both sides for that tile (threads l < T).
@@ -239,16 +254,25 @@ __device__ __forceinline__ void load_first_stage(cx<R> *buf, const Pass &P, cons
     int bc = min(bi, nb - 1);
     butterfly_of(bc, p.in_row, nr, si.m_nr, p.T, P.m_t, lk[q], jk[q]);
     ok[q] = bi < nb && lk[q] < nl;
-    int ls = ok[q] ? lk[q] : 0;
-    if (P.step_in) {
-      const i64 a0 = lin.at(p, p.sin, inT, ls, jk[q]);
+    if constexpr (UIN) {
+      int ls = ok[q] ? lk[q] : 0;
+      if (P.step_in) {
+        const i64 a0 = lin.at(p, p.sin, inT, ls, jk[q]);
 #pragma unroll
-      for (int r = 0; r < RADIX; r++) a[q][r] = a0 + r * P.step_in;
-    } else {
+        for (int r = 0; r < RADIX; r++) a[q][r] = a0 + r * P.step_in;
+      } else {
 #pragma unroll
-      for (int r = 0; r < RADIX; r++) a[q][r] = lin.at(p, p.sin, inT, ls, jk[q] + r * nr);
+        for (int r = 0; r < RADIX; r++) a[q][r] = lin.at(p, p.sin, inT, ls, jk[q] + r * nr);
+      }
     }
   }
+  if constexpr (!UIN)
+    with_points(lin, p, p.sin, [&](auto at) {
+#pragma unroll
+      for (int q = 0; q < K; q++)
+#pragma unroll
+        for (int r = 0; r < RADIX; r++) a[q][r] = at(ok[q] ? lk[q] : 0, jk[q] + r * nr);
+    });
   cx<R> v[K][RADIX];
   gather<K * RADIX>(&v[0][0], in, &a[0][0], p.stream_in);
 #pragma unroll
@@ -284,7 +308,7 @@ __device__ __forceinline__ void last_stage_store(const cx<R> *buf, const Pass &P
   bool ok[K];
   // (AFF: known when compiled, so that no branch sits between the twiddle
   // products and the stores)
-  const bool even = UOUT && CT ? AFF : P.step_out != 0;
+  const bool even = UOUT && (CT ? AFF : P.step_out != 0);
   auto lout_form = [&](const FftSide &s, const i64 *tab, int l, int x) -> i64 {
     if constexpr (UOUT && CT) return lout.template at_form<AFF>(s, tab, l, x);
     else return 0;
@@ -309,17 +333,29 @@ __device__ __forceinline__ void last_stage_store(const cx<R> *buf, const Pass &P
 #pragma unroll
     for (int r = 1; r < RADIX; r++) v[q][r] = twmul<INV, CT>(v[q][r], tw, (nr - 1) + (r - 1) * nr + j);
     dft<R, INV, RADIX>(v[q]);
-    int ls = ok[q] ? l : 0;
-    if (even) {
-      // evenly stepped: an address pair for the butterfly, formed after it
-      const i64 a0 = UOUT && CT ? lout_form(p.sout, outT, ls, j) : lout.at(p, p.sout, outT, ls, j);
-      if (ok[q]) store_steps<RADIX>(out + a0, P.step_out, v[q], p.stream_out);
-    } else {
+    if constexpr (UOUT) {
+      int ls = ok[q] ? l : 0;
+      if (even) {
+        // evenly stepped: an address pair for the butterfly, formed after it
+        const i64 a0 = CT ? lout_form(p.sout, outT, ls, j) : lout.at(p, p.sout, outT, ls, j);
+        if (ok[q]) store_steps<RADIX>(out + a0, P.step_out, v[q], p.stream_out);
+      } else {
 #pragma unroll
-      for (int r = 0; r < RADIX; r++)
-        a[q][r] = UOUT && CT ? lout_form(p.sout, outT, ls, j + r * nr) : lout.at(p, p.sout, outT, ls, j + r * nr);
+        for (int r = 0; r < RADIX; r++)
+          a[q][r] = CT ? lout_form(p.sout, outT, ls, j + r * nr) : lout.at(p, p.sout, outT, ls, j + r * nr);
+      }
     }
   }
+  if constexpr (!UOUT)
+    with_points(lout, p, p.sout, [&](auto at) {
+#pragma unroll
+      for (int q = 0; q < K; q++) {
+        int l, j;
+        butterfly_of(min((int)threadIdx.x + q * NTH, nb - 1), p.out_row, nr, si.m_nr, p.T, P.m_t, l, j);
+#pragma unroll
+        for (int r = 0; r < RADIX; r++) a[q][r] = at(ok[q] ? l : 0, j + r * nr);
+      }
+    });
   if (!even) scatter<K * RADIX, RADIX>(out, &a[0][0], &v[0][0], ok, p.stream_out);
 }
 
@@ -397,15 +433,24 @@ __global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 4) vo
     i64 a[V];
     int sl[V];
     bool ok[V];
-#pragma unroll
-    for (int k = 0; k < V; k++) {
+    // element k of this thread: its place in the tile and on its side
+    auto place = [&](int k, auto at) {
       int e = threadIdx.x + k * NTH;
       int ec = min(e, tot - 1);
       int l, x;
       element(P, p.in_row, p.ord_in, ec, l, x);
       ok[k] = e < tot && l < nl;
       sl[k] = e < tot ? lds_index(l, x, P.ls) : -1;
-      a[k] = lin.at(p, p.sin, inT, ok[k] ? l : 0, x);
+      a[k] = at(ok[k] ? l : 0, x);
+    };
+    if constexpr (UIN) {
+#pragma unroll
+      for (int k = 0; k < V; k++) place(k, [&](int l, int x) { return lin.at(p, p.sin, inT, l, x); });
+    } else {
+      with_points(lin, p, p.sin, [&](auto at) {
+#pragma unroll
+        for (int k = 0; k < V; k++) place(k, at);
+      });
     }
     cx<R> v[V];
     gather<V>(v, in, a, p.stream_in);
@@ -477,15 +522,24 @@ __global__ __launch_bounds__(NTH, (sizeof(R) == 4 && CAP / NTH == 8) ? 8 : 4) vo
     i64 a[V];
     int sl[V];
     bool ok[V];
-#pragma unroll
-    for (int k = 0; k < V; k++) {
+    // element k of this thread: its place in the tile and on its side
+    auto place = [&](int k, auto at) {
       int e = threadIdx.x + k * NTH;
       int ec = min(e, tot - 1);
       int l, x;
       element(P, p.out_row, p.ord_out, ec, l, x);
       ok[k] = e < tot && l < nl;
       sl[k] = lds_index(l, x, P.ls);
-      a[k] = lout.at(p, p.sout, outT, ok[k] ? l : 0, x);
+      a[k] = at(ok[k] ? l : 0, x);
+    };
+    if constexpr (UOUT) {
+#pragma unroll
+      for (int k = 0; k < V; k++) place(k, [&](int l, int x) { return lout.at(p, p.sout, outT, l, x); });
+    } else {
+      with_points(lout, p, p.sout, [&](auto at) {
+#pragma unroll
+        for (int k = 0; k < V; k++) place(k, at);
+      });
     }
     cx<R> w[V];
 #pragma unroll

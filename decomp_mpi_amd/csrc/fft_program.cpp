@@ -207,15 +207,15 @@ static bool plan_pass_tables(dm_comm_t comm, const Side &I, const Side &U, int t
   const std::vector<int> pos_in = positions(I), pos_out = positions(U);
   L.sin.uniform = I.h.uniform ? 1 : 0;
   L.sin.np = (int)pos_in.size();
-  L.sin.far = L.sin.np > kLinePositions;
+  L.sin.form = L.sin.np > kLinePositions ? 2 : 0;
   L.sout.uniform = U.h.uniform ? 1 : 0;
   L.sout.np = (int)pos_out.size();
-  L.sout.far = L.sout.np > kLinePositions;
+  L.sout.form = L.sout.np > kLinePositions ? 2 : 0;
   L.dbl = dbl;
   L.ctw = (!dbl && ctw) ? 1 : 0;
   const int np_most = std::max(std::max(L.sin.np, L.sout.np), 1);
   // positions per line of the sides that keep their lines' bases in LDS
-  const int np_lds = std::max(std::max(L.sin.far ? 1 : L.sin.np, L.sout.far ? 1 : L.sout.np), 1);
+  const int np_lds = std::max(std::max(L.sin.form == 2 ? 1 : L.sin.np, L.sout.form == 2 ? 1 : L.sout.np), 1);
   // Small arrays: lines per tile are halved while a pass has fewer than 192
   // tiles for the 256 CUs and rows of 64 bytes stay.  What is left to win
   // there is the latency of one tile, which falls with its points per thread
@@ -347,12 +347,13 @@ static bool plan_pass_tables(dm_comm_t comm, const Side &I, const Side &U, int t
     }
     if (s.h.uniform) return;
     std::vector<int> xt(2 * (size_t)L.N);
-    fs.lin = fs.np == 1;
+    bool in_order = fs.np == 1;
     for (int x = 0; x < L.N; x++) {
       xt[2 * (size_t)x] = (int)(std::lower_bound(pos.begin(), pos.end(), s.h.rank_part[t][x]) - pos.begin());
       xt[2 * (size_t)x + 1] = s.h.off[t][x];
-      fs.lin = fs.lin && s.h.off[t][x] == x;
+      in_order = in_order && s.h.off[t][x] == x;
     }
+    if (in_order) fs.form = 1;
     ps.xt = tb.put(xt.data(), xt.size() * sizeof(int));
     ps.posrank = tb.put(pos.data(), pos.size() * sizeof(int));
     ps.rank = joined(s.h.rank_part);

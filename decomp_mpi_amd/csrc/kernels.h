@@ -89,8 +89,8 @@ struct FftSide {
   int rsh, rmask;              //   (x >> rsh) * jump + (x & rmask) * rstride; else the table
   // non-uniform sides
   int np;                      // rank positions along t
-  int lin;                     // one position, local offset x at point x
-  int far;                     // more than kLinePositions: addresses formed point by point
+  int form;                    // 1: one position, local offset x at point x; 2: more than
+                               //   kLinePositions, addresses formed point by point; else 0
   const int *xt;               // point x of t: position, local offset
   const int *posrank;          // owner contribution of each position
   const int *rank, *off;       // owner contributions and local offsets, axis d's at FftLaunch::at[d]
@@ -172,7 +172,7 @@ int fft_tile_capacity(int dbl, int column, int wide = 0);
 constexpr int kLineEntries = 1024;
 constexpr int kLinePositions = 6;
 // LDS a workgroup of the pass takes: its tile, the line data of both sides
-// (uniform, np, far) and the twiddles.  At most kLdsBytes, or the launch is refused.
+// (uniform, np, form) and the twiddles.  At most kLdsBytes, or the launch is refused.
 constexpr size_t kLdsBytes = 160 * 1024;
 size_t fft_lds_bytes(const FftLaunch &p);
 
