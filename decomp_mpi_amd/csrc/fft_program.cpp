@@ -217,19 +217,27 @@ static bool plan_pass_tables(dm_comm_t comm, const Side &I, const Side &U, int t
   // positions per line of the sides that keep their lines' bases in LDS
   const int np_lds = std::max(std::max(L.sin.form == 2 ? 1 : L.sin.np, L.sout.form == 2 ? 1 : L.sout.np), 1);
   // Small arrays: lines per tile are halved while a pass has fewer than 192
-  // tiles for the 256 CUs and rows of 64 bytes stay.  What is left to win
+  // tiles for the 256 CUs and its rows are longer than 64 bytes (so 5 complex
+  // doubles become 3; stopping at 64 bytes exactly, 8 lines for 6, a forward
+  // of 68x8x24 complex floats took 43.5 us for 40.5).  What is left to win
   // there is the latency of one tile, which falls with its points per thread
   // (64^3 complex double over pencils 22.0 -> 20.1 us a transform, 61x21x100
   // on 12 ranks 182 -> 104, 75x200 on 6 62 -> 43).  At 256 tiles
   // 2940x576 lost (145 -> 153 us: rows of half the width for nothing, all
   // CUs were busy); at 512 and 1024 arrays of a million points did (71 -> 87
-  // and 105 us for 256x208x72).
+  // and 105 us for 256x208x72).  Fewer points than one complex-double tile
+  // holds are left in it: more workgroups only fetch the code more often
+  // (steps of 104x8 complex doubles 32.6 -> 28.4 us whole, 78x16 complex
+  // floats 36.5 -> 32.9; 128x44, 5632 points, 41.9 whole and 35.9 spread),
+  // unless a direct-sum stage has work for them (45x79 complex floats 109 us
+  // a forward whole, 52 spread).
   long long lines = 1;
   for (int d = 0; d < nd; d++)
     if (d != t) lines *= I.h.L[d];
   auto spread = [&](int T) {
     const int least = 64 / (dbl ? 16 : 8);
-    while (T > least && lines / T < 192) T = std::max(least, (T + 1) / 2);
+    if (lines * L.N < 4096 && std::all_of(rad.begin(), rad.end(), has_radix_kernel)) return T;
+    while (T > least && lines / T < 192) T = (T + 1) / 2;
     return T;
   };
   if (u >= 0) {

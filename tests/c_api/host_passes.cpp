@@ -161,6 +161,31 @@ static void stages() {
   }
 }
 
+// Workgroups of passes over few lines: as many as tiles hold the lines where
+// the whole array is less than 4096 points; more from there on, and where a
+// direct-sum stage has work for them.
+static void few_lines() {
+  const struct {
+    int n, lines;
+    bool whole;
+  } at[] = {{32, 127, true}, {32, 128, false}, {3, 100, true}, {104, 8, true}, {8, 104, true}, {1000, 4, true},
+            {256, 16, false}, {79, 45, false}, {106, 38, false}};
+  for (const auto &c : at)
+    for (int t : {0, 1})
+      for (int dbl : {0, 1}) {
+        const Layout l(t == 0 ? std::vector<int>{c.n, c.lines} : std::vector<int>{c.lines, c.n}, {1, 1});
+        const dm::Side s = l.side();
+        dm::TableBuilder tb;
+        dm::PendingPass pp;
+        const int most = dm::fft_tile_capacity(dbl, t == 0) / c.n, held = (c.lines + most - 1) / most;
+        if (!dm::plan_pass(l.comm, s, s, t, dbl, false, nullptr, nullptr, tb, &pp) || (pp.L.tiles_u == held) != c.whole) {
+          printf("%d lines of %d along axis %d, dbl %d: %lld tiles, %d hold them\n", c.lines, c.n, t, dbl,
+                 (long long)pp.L.tiles_u, held);
+          failures++;
+        }
+      }
+}
+
 int main(int argc, char **argv) {
   dm_set_error_mode(1);
   const std::string check = argc > 1 ? argv[1] : "";
@@ -169,6 +194,7 @@ int main(int argc, char **argv) {
   else if (check == "reshape") reshape();
   else if (check == "memory") memory();
   else if (check == "stages") stages();
+  else if (check == "few_lines") few_lines();
   else return 2;
   if (failures == 0) printf("OK\n");
   return failures != 0;

@@ -108,3 +108,16 @@ def test_uneven_intermediates_of_long_lines(C, P, shape, grid, dbl):
     fwd, rt, _ = run_split(C, P, shape, grid, slab=0, dbl=dbl)
     tol = TOL64 if dbl else TOL32
     assert fwd < tol and rt < tol, (fwd, rt)
+
+
+@pytest.mark.parametrize("dbl", [True, False])
+@pytest.mark.parametrize("shape,axis,gin,gout", [
+    ((32, 127), 0, (2, 1), (1, 3)),  # the most points that are not spread over workgroups
+    ((127, 32), 1, (3, 1), (1, 2)),
+    ((32, 128), 0, (2, 1), (1, 3)),  # one line more
+    ((104, 8), 0, (1, 1), (1, 1)),
+    ((1, 2, 2), 1, (1, 1, 1), (1, 1, 1)),
+    ((79, 45), 0, (2, 4), (2, 4)),   # a direct-sum prime: spread all the same
+])
+def test_passes_over_few_lines(C, shape, axis, gin, gout, dbl):
+    axis_fft(C, shape, axis, gin, gout, dbl)

@@ -52,3 +52,8 @@ def test_out_of_host_memory(driver):
 def test_stages(driver):
     """No length within a tile takes more stages than a launch holds."""
     run(driver, "stages")
+
+
+def test_workgroups_of_few_lines(driver):
+    """A pass over less than 4096 points is not spread over workgroups."""
+    run(driver, "few_lines")
