@@ -225,18 +225,19 @@ static bool plan_pass_tables(dm_comm_t comm, const Side &I, const Side &U, int t
   // on 12 ranks 182 -> 104, 75x200 on 6 62 -> 43).  At 256 tiles
   // 2940x576 lost (145 -> 153 us: rows of half the width for nothing, all
   // CUs were busy); at 512 and 1024 arrays of a million points did (71 -> 87
-  // and 105 us for 256x208x72).  Fewer points than one complex-double tile
-  // holds are left in it: more workgroups only fetch the code more often
-  // (steps of 104x8 complex doubles 32.6 -> 28.4 us whole, 78x16 complex
-  // floats 36.5 -> 32.9; 128x44, 5632 points, 41.9 whole and 35.9 spread),
-  // unless a direct-sum stage has work for them (45x79 complex floats 109 us
-  // a forward whole, 52 spread).
+  // and 105 us for 256x208x72).  Less than 20 KiB of points stay in one tile:
+  // more workgroups only fetch the code more often.  Forwards spread and
+  // whole: 84x14 complex floats 35.7 and 33.7 us, 78x20 34.9 and 32.5, 65x35
+  // 38.7 and 37.5; beyond, 96x30 36.8 and 38.0, 27x125 38.7 and 40.7; complex
+  // doubles 90x12 28.1 and 28.3, 105x15 36.7 and 39.3, 45x45 38.4 and 42.6.
+  // A direct-sum stage has work for more workgroups (45x79 complex floats
+  // 52 and 109).
   long long lines = 1;
   for (int d = 0; d < nd; d++)
     if (d != t) lines *= I.h.L[d];
   auto spread = [&](int T) {
     const int least = 64 / (dbl ? 16 : 8);
-    if (lines * L.N < 4096 && std::all_of(rad.begin(), rad.end(), has_radix_kernel)) return T;
+    if (lines * L.N * (dbl ? 16 : 8) < (20 << 10) && std::all_of(rad.begin(), rad.end(), has_radix_kernel)) return T;
     while (T > least && lines / T < 192) T = (T + 1) / 2;
     return T;
   };

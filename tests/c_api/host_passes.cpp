@@ -162,14 +162,15 @@ static void stages() {
 }
 
 // Workgroups of passes over few lines: as many as tiles hold the lines where
-// the whole array is less than 4096 points; more from there on, and where a
+// the whole array is less than 20 KiB; more from there on, and where a
 // direct-sum stage has work for them.
 static void few_lines() {
   const struct {
     int n, lines;
-    bool whole;
-  } at[] = {{32, 127, true}, {32, 128, false}, {3, 100, true}, {104, 8, true}, {8, 104, true}, {1000, 4, true},
-            {256, 16, false}, {79, 45, false}, {106, 38, false}};
+    bool whole[2];  // complex float, complex double
+  } at[] = {{32, 39, {true, true}},    {32, 40, {true, false}}, {32, 79, {true, false}},  {32, 80, {false, false}},
+            {3, 100, {true, true}},    {104, 8, {true, true}},  {8, 104, {true, true}},   {600, 4, {true, true}},
+            {256, 16, {false, false}}, {79, 15, {false, false}}, {106, 38, {false, false}}};
   for (const auto &c : at)
     for (int t : {0, 1})
       for (int dbl : {0, 1}) {
@@ -178,7 +179,7 @@ static void few_lines() {
         dm::TableBuilder tb;
         dm::PendingPass pp;
         const int most = dm::fft_tile_capacity(dbl, t == 0) / c.n, held = (c.lines + most - 1) / most;
-        if (!dm::plan_pass(l.comm, s, s, t, dbl, false, nullptr, nullptr, tb, &pp) || (pp.L.tiles_u == held) != c.whole) {
+        if (!dm::plan_pass(l.comm, s, s, t, dbl, false, nullptr, nullptr, tb, &pp) || (pp.L.tiles_u == held) != c.whole[dbl]) {
           printf("%d lines of %d along axis %d, dbl %d: %lld tiles, %d hold them\n", c.lines, c.n, t, dbl,
                  (long long)pp.L.tiles_u, held);
           failures++;

@@ -112,9 +112,10 @@ def test_uneven_intermediates_of_long_lines(C, P, shape, grid, dbl):
 
 @pytest.mark.parametrize("dbl", [True, False])
 @pytest.mark.parametrize("shape,axis,gin,gout", [
-    ((32, 127), 0, (2, 1), (1, 3)),  # the most points that are not spread over workgroups
-    ((127, 32), 1, (3, 1), (1, 2)),
-    ((32, 128), 0, (2, 1), (1, 3)),  # one line more
+    ((32, 39), 0, (2, 1), (1, 3)),   # complex double: the most points that are not spread over workgroups
+    ((40, 32), 1, (3, 1), (1, 2)),   # and one line more
+    ((79, 32), 1, (3, 1), (1, 2)),   # the same for complex float
+    ((32, 80), 0, (2, 1), (1, 3)),
     ((104, 8), 0, (1, 1), (1, 1)),
     ((1, 2, 2), 1, (1, 1, 1), (1, 1, 1)),
     ((79, 45), 0, (2, 4), (2, 4)),   # a direct-sum prime: spread all the same

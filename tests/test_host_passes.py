@@ -55,5 +55,5 @@ def test_stages(driver):
 
 
 def test_workgroups_of_few_lines(driver):
-    """A pass over less than 4096 points is not spread over workgroups."""
+    """A pass over less than 20 KiB of points is not spread over workgroups."""
     run(driver, "few_lines")
